@@ -128,7 +128,7 @@ void run_gemv(mdma_ctx *ctx, int mode, const GemvJob *jobs, int n, const float *
   if (mode == MDMA_ACT_I8)
     launch_gemv_i8(ctx, jobs, n, x, T);
   else if (mode == MDMA_ACT_F32_CPU)
-    for (int i = 0; i < n; i++) launch_gemv_seq(ctx, jobs[i], x, T);
+    launch_gemv_seq(ctx, jobs, n, x, T);
   else
     launch_gemv_f32(ctx, jobs, n, x, T);
 }
@@ -919,8 +919,12 @@ int mdma_gfx950_ffn_gate_up(mdma_ctx *ctx, const mdma_qweight *gate, const mdma_
     uint64_t gse = f32_elems("ffn_gate_up", gate_scratch), use = f32_elems("ffn_gate_up", up_scratch);
     if (gse != T * gate->rows || use != gse || ctx->act_mode == MDMA_ACT_F32_CPU) {
       if (use != gse) shape_fail("silu_mul: input lengths differ");
-      run_gemv(ctx, ctx->act_mode, &gj, 1, xp, T);
-      run_gemv(ctx, ctx->act_mode, &uj, 1, xp, T);
+      if (ctx->act_mode == MDMA_ACT_F32_CPU) {
+        run_gemv(ctx, ctx->act_mode, gu_jobs, 2, xp, T);
+      } else {
+        run_gemv(ctx, ctx->act_mode, &gj, 1, xp, T);
+        run_gemv(ctx, ctx->act_mode, &uj, 1, xp, T);
+      }
       const float *gp = reinterpret_cast<const float *>(gate_scratch->ptr),
                   *up_p = reinterpret_cast<const float *>(up_scratch->ptr);
       if (ctx->act_mode == MDMA_ACT_F32_CPU)

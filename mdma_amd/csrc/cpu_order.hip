@@ -224,6 +224,267 @@ __global__ __launch_bounds__(64) void gemv_seq_kernel(const uint8_t *__restrict_
   }
 }
 
+// s plus n4 float4 of LDS (a multiple of 8), in order, one dependent
+// addition each: the next 8 reads are in flight while 8 are added. On gfx950
+// a dependent f32 addition takes 8.4 cycles (measured), so 4096 of them take
+// about 15 us whatever feeds them.
+typedef float v4f __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float chain8(float s, const v4f (&v)[8]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    s = s + v[k].x;
+    s = s + v[k].y;
+    s = s + v[k].z;
+    s = s + v[k].w;
+  }
+  return s;
+}
+template <class Read>
+__device__ __forceinline__ float chain_add(float s, uint32_t n4, Read &&rd) {
+  v4f v[8], w[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) v[k] = rd(k);
+  for (uint32_t g = 0; g < n4; g += 16) {
+    const uint32_t g1 = g + 8 < n4 ? g + 8 : g, g2 = g + 16 < n4 ? g + 16 : g;  // (past the end: read, not added)
+#pragma unroll
+    for (int k = 0; k < 8; k++) w[k] = rd(g1 + k);
+    s = chain8(s, v);
+    if (g + 8 >= n4) break;
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = rd(g2 + k);
+    s = chain8(s, w);
+  }
+  return s;
+}
+
+// ---- up to 4 tokens over prepared rows: dequantization and chains apart ----
+// With one lane doing everything for its row, the chain's next addition waits
+// for the column's whole dequantization (about 11 VALU instructions a
+// column), on one wave per SIMD. Here NP producer waves dequantize, multiply
+// by x and leave the f32-rounded products in LDS, and chain waves (one lane
+// per row and token) only add them, in column order: the same operations on
+// the same operands, so the same bits. What bounds it is the chain, one
+// dependent f32 addition per column, where the rows leave CUs free (one token,
+// 4096x4096 20.5 us of which 15 are additions, 4096x14336 57 of 52), and the
+// producers' VALU and LDS traffic where they do not.
+//
+// A stage is NP * 64 / R units of a row (UC columns each) for R rows; its
+// products sit in LDS as [column / 4][token][row] float4, double-buffered: the
+// producers fill stage s while the chains add stage s - 1. The next stage's
+// weights and x are in flight across the barrier (lds_barrier).
+struct SeqJob {
+  const uint8_t *w;
+  float *y;
+  uint32_t n_out, tiles;
+};
+struct SeqSet {
+  SeqJob j[3];
+};
+
+// One unit of a prepared row (layout.cpp): its bytes, and its weights
+// four columns at a time: quad i covers columns col(u, i) .. + 3 of the stage.
+template <int DT>
+struct SeqUnit;
+
+template <>
+struct SeqUnit<DT_Q4_K> {
+  static constexpr uint32_t UC = 64;
+  uint4 a, b, hd;
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t u, uint32_t U) {
+    a = ldx16(row + 16 * (size_t)u);
+    b = ldx16(row + 16 * (size_t)(U + u));
+    hd = ldx16(row + 32 * (size_t)U + 16 * (size_t)(u >> 2));
+  }
+  struct Scales {
+    float d[2], m[2];
+  };
+  __device__ __forceinline__ Scales scales(uint32_t u) const {
+    int sca, scb, ma, mb;
+    q4k_scales_i(hd, u & 3, sca, scb, ma, mb);
+    const float d = h2f(hd.x), dmin = h2f(hd.x >> 16);
+    return Scales{{d * (float)sca, d * (float)scb}, {dmin * (float)ma, dmin * (float)mb}};
+  }
+  __device__ static __forceinline__ uint32_t col(uint32_t u, int i) { return 64 * u + 4 * i; }
+  // fma: d1 * q is exact (17 + 4 bits), so it rounds once, as t - m1 does.
+  __device__ __forceinline__ void weights(const Scales &s, int i, float *o) const {
+    const uint32_t q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const uint32_t v = (i < 8 ? q[i & 7] : q[i & 7] >> 4) & 0x0F0F0F0Fu;
+    const float d = s.d[i >> 3], m = s.m[i >> 3];
+#pragma unroll
+    for (int k = 0; k < 4; k++) o[k] = __builtin_fmaf(d, (float)byte_of(v, k), -m);
+  }
+};
+
+template <>
+struct SeqUnit<DT_Q6_K> {
+  static constexpr uint32_t UC = 64;
+  uint4 a, b, q;
+  uint32_t sc, d;
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t u, uint32_t U) {
+    a = ldx16(row + 16 * (size_t)u);
+    b = ldx16(row + 16 * (size_t)(U + u));
+    q = ldx16(row + 16 * (size_t)(2 * U + u));
+    sc = *reinterpret_cast<const uint32_t *>(row + 48 * (size_t)U + 4 * (size_t)u);
+    d = ldu16(row + 52 * (size_t)U + 2 * (size_t)(u >> 2));
+  }
+  struct Scales {
+    float d[4];
+  };
+  __device__ __forceinline__ Scales scales(uint32_t) const {
+    Scales s;
+    const float df = h2f(d);
+#pragma unroll
+    for (int r = 0; r < 4; r++) s.d[r] = df * (float)(int)(int8_t)byte_of(sc, r);
+    return s;
+  }
+  // Quad i: quarter i / 4, columns 4 (i % 4) of the unit's 16.
+  __device__ static __forceinline__ uint32_t col(uint32_t u, int i) {
+    return 256 * (u >> 2) + 128 * ((u >> 1) & 1) + 32 * (i >> 2) + 16 * (u & 1) + 4 * (i & 3);
+  }
+  __device__ __forceinline__ void weights(const Scales &s, int i, float *o) const {
+    const uint32_t qa[4] = {a.x, a.y, a.z, a.w}, qb[4] = {b.x, b.y, b.z, b.w}, qh[4] = {q.x, q.y, q.z, q.w};
+    const int r = i >> 2, k4 = i & 3;
+    const uint32_t low = (r & 1 ? qb[k4] : qa[k4]) >> (r < 2 ? 0 : 4) & 0x0F0F0F0Fu;
+    const uint32_t h = r == 0 ? qh[k4] << 4 : r == 1 ? qh[k4] << 2 : r == 2 ? qh[k4] : qh[k4] >> 2;
+    const uint32_t v = low | (h & 0x30303030u);
+    // (q - 32) first, exact: a zero weight keeps the sign (d * sc) * 0 has.
+#pragma unroll
+    for (int k = 0; k < 4; k++) o[k] = s.d[r] * ((float)byte_of(v, k) - 32.0f);
+  }
+};
+
+template <>
+struct SeqUnit<DT_Q8_0> {
+  static constexpr uint32_t UC = 32;
+  uint4 a, b;
+  uint32_t d;
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t u, uint32_t U) {
+    a = ldx16(row + 16 * (size_t)u);
+    b = ldx16(row + 16 * (size_t)(U + u));
+    d = ldu16(row + 32 * (size_t)U + 2 * (size_t)u);
+  }
+  struct Scales {
+    float d;
+  };
+  __device__ __forceinline__ Scales scales(uint32_t) const { return Scales{h2f(d)}; }
+  __device__ static __forceinline__ uint32_t col(uint32_t u, int i) { return 32 * u + 4 * i; }
+  __device__ __forceinline__ void weights(const Scales &s, int i, float *o) const {
+    const uint32_t q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const uint32_t v = q[i] ^ 0x80808080u;
+#pragma unroll
+    for (int k = 0; k < 4; k++) o[k] = ((float)byte_of(v, k) - 128.0f) * s.d;
+  }
+};
+
+template <int DT, int R, int NP, int TT>
+__global__ __launch_bounds__(64 * (NP + (R * TT + 63) / 64)) void gemv_seq_pipe_kernel(
+    SeqSet js, uint32_t n_in, uint64_t row_bytes, const float *__restrict__ x, uint32_t T) {
+#pragma clang fp contract(off)
+  using Unit = SeqUnit<DT>;
+  constexpr int UC = Unit::UC, NC = (R * TT + 63) / 64, UPW = 64 / R, UPS = NP * UPW;
+  constexpr int SC = UPS * UC;          // columns of a stage
+  constexpr int LANES = R * TT;         // chains
+  constexpr int X4 = TT * SC / 4;       // float4 of x per stage
+  constexpr int XN = (X4 + 64 * NP - 1) / (64 * NP);
+  __shared__ __attribute__((aligned(16))) v4f prod[2][SC / 4][LANES];
+  __shared__ __attribute__((aligned(16))) v4f xs[2][TT][SC / 4];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t tile = blockIdx.x, ji = 0;
+  while (ji < 2 && tile >= js.j[ji].tiles) tile -= js.j[ji].tiles, ji++;
+  const uint8_t *w = ji == 0 ? js.j[0].w : ji == 1 ? js.j[1].w : js.j[2].w;
+  float *y = ji == 0 ? js.j[0].y : ji == 1 ? js.j[1].y : js.j[2].y;
+  const uint32_t n_out = ji == 0 ? js.j[0].n_out : ji == 1 ? js.j[1].n_out : js.j[2].n_out;
+  const uint32_t U = n_in / UC, S = (U + UPS - 1) / UPS, n4 = n_in / 4;
+  if (wave < NC) {  // chains
+    const uint32_t c = min(wave * 64 + lane, (uint32_t)LANES - 1);
+    float s = -0.0f;
+    lds_barrier();  // the first stage's x
+    for (uint32_t st = 0; st < S; st++) {
+      lds_barrier();  // stage st's products
+      const v4f(*pb)[LANES] = prod[st & 1];
+      const uint32_t q4 = min((uint32_t)SC / 4, n4 - st * (SC / 4));  // a multiple of 8
+      s = chain_add(s, q4, [&](uint32_t k) { return pb[k][c]; });
+    }
+    const uint32_t row = tile * R + c % R, t = c / R;
+    if (wave * 64 + lane < LANES && row < n_out && t < T) y[(size_t)t * n_out + row] = s;
+    return;
+  }
+  const uint32_t p = wave - NC, ptid = p * 64 + lane, r = lane % R, uu = p * UPW + lane / R;
+  const uint8_t *wr = w + (size_t)min(tile * R + r, n_out - 1) * row_bytes;
+  auto load_x = [&](uint32_t st, v4f (&o)[XN]) {
+#pragma unroll
+    for (int i = 0; i < XN; i++) {
+      const uint32_t e = ptid + 64 * NP * i, t = min(e / (SC / 4), T - 1), c4 = min(st * (SC / 4) + e % (SC / 4), n4 - 1);
+      o[i] = *reinterpret_cast<const v4f *>(x + (size_t)t * n_in + 4 * (size_t)c4);
+    }
+  };
+  auto store_x = [&](uint32_t st, const v4f (&v)[XN]) {
+#pragma unroll
+    for (int i = 0; i < XN; i++) {
+      const uint32_t e = ptid + 64 * NP * i;
+      if (X4 % (64 * NP) == 0 || e < X4) xs[st & 1][e / (SC / 4)][e % (SC / 4)] = v[i];
+    }
+  };
+  auto compute = [&](uint32_t st, const Unit &un) {
+    const uint32_t u = st * UPS + uu;
+    const typename Unit::Scales sc = un.scales(u);
+    const v4f(*xb)[SC / 4] = xs[st & 1];
+    v4f(*pb)[LANES] = prod[st & 1];
+#pragma unroll
+    for (int i = 0; i < UC / 4; i++) {
+      float wv[4];
+      un.weights(sc, i, wv);
+      const uint32_t c4 = Unit::col(uu, i) / 4;  // (a stage is whole blocks)
+#pragma unroll
+      for (int t = 0; t < TT; t++) {
+        const v4f xv = xb[t][c4];
+        pb[c4][t * R + r] = v4f{wv[0] * xv.x, wv[1] * xv.y, wv[2] * xv.z, wv[3] * xv.w};
+      }
+    }
+  };
+  auto unit_at = [&](uint32_t st) { return min(st * UPS + uu, U - 1); };
+  // D stages' weights and x in flight: a stage is 0.5 to 2 us of chain, a
+  // load from HBM about 1 us. S + 1 barriers in all, as in the chain waves.
+  constexpr int D = R == 64 ? 4 : 2;
+  Unit u0, u1, u2, u3;
+  v4f x0[XN], x1[XN], x2[XN], x3[XN];
+  load_x(0, x0);
+  u0.load(wr, unit_at(0), U);
+  store_x(0, x0);
+  load_x(1, x1);
+  u1.load(wr, unit_at(1), U);
+  if constexpr (D == 4) {
+    load_x(2, x2);
+    u2.load(wr, unit_at(2), U);
+    load_x(3, x3);
+    u3.load(wr, unit_at(3), U);
+    load_x(4, x0);
+  } else {
+    load_x(2, x0);
+  }
+  lds_barrier();
+  auto stage = [&](uint32_t st, Unit &un, v4f (&xn)[XN]) {
+    if (st >= S) return;
+    compute(st, un);
+    store_x(st + 1, xn);
+    load_x(st + 1 + D, xn);
+    un.load(wr, unit_at(st + D), U);
+    lds_barrier();
+  };
+  for (uint32_t st = 0; st < S; st += D) {
+    if constexpr (D == 4) {
+      stage(st, u0, x1);
+      stage(st + 1, u1, x2);
+      stage(st + 2, u2, x3);
+      stage(st + 3, u3, x0);
+    } else {
+      stage(st, u0, x1);
+      stage(st + 1, u1, x0);
+    }
+  }
+}
+
 // Float weights (F32, F16): the row read element by element, x from global
 // memory (uniform addresses).
 template <int DT, int TT>
@@ -255,29 +516,42 @@ __global__ __launch_bounds__(64) void gemv_seq_float_kernel(const uint8_t *__res
 
 // rmsnorm (cpu.rs:388-402) of one row per workgroup, optionally after the
 // residual add (Backend::add_rmsnorm default, src/backend.rs:502-513: sum =
-// a + b, then rmsnorm of the sum): lane 0 forms the sequential sum of
-// squares (dot(row, row), from -0.0), then every lane its outputs
-// (row[i] * scale) * w[i] with scale = 1 / sqrt(mean + eps).
-__global__ __launch_bounds__(256) void rmsnorm_seq_kernel(const float *__restrict__ w, uint32_t dim,
+// a + b, then rmsnorm of the sum): the rounded squares go to LDS in parallel
+// and wave 0 adds them in order (dot(row, row), from -0.0), then every lane
+// forms its outputs (row[i] * scale) * w[i] with scale = 1 / sqrt(mean + eps).
+__global__ __launch_bounds__(1024) void rmsnorm_seq_kernel(const float *__restrict__ w, uint32_t dim,
                                                           const float *__restrict__ a, const float *__restrict__ b,
                                                           float *__restrict__ sum, float *__restrict__ y, float eps) {
 #pragma clang fp contract(off)
+  constexpr uint32_t CHUNK = 8192;  // squares in LDS at a time
+  __shared__ __attribute__((aligned(16))) float sq[CHUNK];
   __shared__ float scale_sh;
   const size_t base = (size_t)blockIdx.x * dim;
   const float *ar = a + base, *br = b ? b + base : nullptr;
-  if (threadIdx.x == 0) {
-    float ss = -0.0f;
-    for (uint32_t i = 0; i < dim; i++) {
-      const float v = br ? ar[i] + br[i] : ar[i];
-      const float p = v * v;
-      ss = ss + p;
+  float ss = -0.0f;
+  for (uint32_t c0 = 0; c0 < dim; c0 += CHUNK) {
+    const uint32_t n = min(CHUNK, dim - c0);
+    if (c0) __syncthreads();  // the previous chunk is added
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
+      const float v = br ? ar[c0 + i] + br[c0 + i] : ar[c0 + i];
+      sq[i] = v * v;
     }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // the chain, the same in every lane of wave 0
+      uint32_t i = n / 32 * 32;
+      if (i) ss = chain_add(ss, i / 4, [&](uint32_t k) { return reinterpret_cast<const v4f *>(sq)[k]; });
+      for (; i < n; i++) ss = ss + sq[i];
+    }
+  }
+  if (threadIdx.x == 0) {
     const float mean = div_rn(ss, (float)dim);
     scale_sh = div_rn(1.0f, sqrt_rn(mean + eps));
   }
   __syncthreads();
   const float scale = scale_sh;
-  for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) {
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < dim; i += 1024) {
     const float v = br ? ar[i] + br[i] : ar[i];
     if (sum) sum[base + i] = v;
     const float t = v * scale;
@@ -367,6 +641,72 @@ __global__ __launch_bounds__(256) void attn_seq_kernel(const float *__restrict__
 
 }  // namespace
 
+namespace {
+// One token: rows past this take 64-row workgroups (a chain wave's lanes all
+// used), fewer take 16-row ones, which spread over every CU. The fused
+// 28672-row gate/up 45.9 us in 64-row workgroups; 4096 rows of 4096 columns
+// 20.5 us in 16-row ones (64-row ones would use 64 of the 256 CUs).
+constexpr uint64_t SEQ_WIDE_ROWS = 16384;
+// Tiles of 16 rows and 4 tokens up to which the split kernel is the faster
+// one: past them the launch is bound by its products' VALU work, which the
+// 8-token kernel spends less of per token. us, split / one-lane kernel:
+// 4096x4096 Q6_K T = 1: 20.5 / 96.2, 2: 30.8 / 391, 8 (512 tiles): 86.2 / 395;
+// 2x14336x4096 Q4_K T = 4 (1792 tiles): 262 / 520, 8 (3584): 518 / 542.
+constexpr uint64_t SEQ_PIPE_TILES = 3584;
+
+template <int DT, int R, int NP, int TT>
+void seq_pipe(mdma_ctx *ctx, const GemvJob *jobs, int n, uint64_t row_bytes, const float *x, uint64_t T) {
+  SeqSet js{};
+  uint64_t tiles = 0;
+  for (int i = 0; i < 3; i++) {
+    js.j[i] = i < n ? SeqJob{jobs[i].w, jobs[i].y, (uint32_t)jobs[i].n_out, (uint32_t)((jobs[i].n_out + R - 1) / R)}
+                    : SeqJob{nullptr, nullptr, 0, 0};
+    tiles += js.j[i].tiles;
+  }
+  gemv_seq_pipe_kernel<DT, R, NP, TT><<<dim3((uint32_t)tiles), dim3(64 * (NP + (R * TT + 63) / 64)), 0, ctx->stream>>>(
+      js, (uint32_t)jobs[0].n_in, row_bytes, x, (uint32_t)T);
+  hip_check(hipGetLastError(), "gemv_seq_pipe launch");
+}
+template <int DT>
+void seq_pipe_t(mdma_ctx *ctx, const GemvJob *jobs, int n, uint64_t row_bytes, const float *x, uint64_t T) {
+  uint64_t rows = 0;
+  for (int i = 0; i < n; i++) rows += jobs[i].n_out;
+  if (T == 1 && rows > SEQ_WIDE_ROWS)
+    // (Two producers need a stage of half a block, which Q6_K's interleaved
+    // columns do not have.)
+    seq_pipe<DT, 64, DT == DT_Q4_K ? 2 : 4, 1>(ctx, jobs, n, row_bytes, x, T);
+  else if (T == 1)
+    seq_pipe<DT, 16, 2, 1>(ctx, jobs, n, row_bytes, x, T);
+  else if (T == 2)
+    seq_pipe<DT, 16, 1, 2>(ctx, jobs, n, row_bytes, x, T);
+  else
+    for (uint64_t t0 = 0; t0 < T; t0 += 4) {
+      GemvJob js[3];
+      for (int i = 0; i < n; i++) js[i] = jobs[i], js[i].y += t0 * jobs[i].n_out;
+      seq_pipe<DT, 16, 1, 4>(ctx, js, n, row_bytes, x + t0 * jobs[0].n_in, T - t0 < 4 ? T - t0 : 4);
+    }
+}
+}  // namespace
+
+void launch_gemv_seq(mdma_ctx *ctx, const GemvJob *jobs, int n, const float *x, uint64_t T) {
+  const GemvJob &j = jobs[0];
+  bool one = T > 0 && n <= 3 && j.layout == MDMA_LAYOUT_GFX950 && j.n_in % block_size(j.dtype) == 0 &&
+             j.n_in > 0 && j.n_in <= 0xffffffffull;
+  uint64_t tiles = 0;
+  for (int i = 0; i < n; i++) {
+    one = one && jobs[i].layout == j.layout && jobs[i].dtype == j.dtype && jobs[i].n_in == j.n_in && jobs[i].n_out > 0;
+    tiles += (jobs[i].n_out + 15) / 16;
+  }
+  if (!one || (T + 3) / 4 * tiles > (T == 1 ? 0x7ffffffull : SEQ_PIPE_TILES)) {
+    for (int i = 0; i < n; i++) launch_gemv_seq(ctx, jobs[i], x, T);
+    return;
+  }
+  const uint64_t rb = gfx950_row_bytes(j.dtype, j.n_in);
+  if (j.dtype == DT_Q4_K) seq_pipe_t<DT_Q4_K>(ctx, jobs, n, rb, x, T);
+  else if (j.dtype == DT_Q6_K) seq_pipe_t<DT_Q6_K>(ctx, jobs, n, rb, x, T);
+  else seq_pipe_t<DT_Q8_0>(ctx, jobs, n, rb, x, T);
+}
+
 void launch_gemv_seq(mdma_ctx *ctx, const GemvJob &j, const float *x, uint64_t T) {
   if (!T || !j.n_out) return;
   if (j.n_out > 0xffffffffull || j.n_in > 0xffffffffull || T > 0xffffffffull)
@@ -407,7 +747,7 @@ void launch_gemv_seq(mdma_ctx *ctx, const GemvJob &j, const float *x, uint64_t T
 void launch_rmsnorm_seq(mdma_ctx *ctx, const float *w, uint64_t dim, const float *a, const float *b, float *sum,
                         float *y, uint64_t rows, float eps) {
   if (!rows) return;
-  rmsnorm_seq_kernel<<<dim3((uint32_t)rows), dim3(256), 0, ctx->stream>>>(w, (uint32_t)dim, a, b, sum, y, eps);
+  rmsnorm_seq_kernel<<<dim3((uint32_t)rows), dim3(1024), 0, ctx->stream>>>(w, (uint32_t)dim, a, b, sum, y, eps);
   hip_check(hipGetLastError(), "rmsnorm_seq launch");
 }
 

@@ -432,6 +432,9 @@ void launch_attn(mdma_ctx *ctx, const float *q, const uint16_t *k, const uint16_
 // silu_mul; causal GQA attention (seq_stride and pos_dev as launch_attn /
 // launch_attn_rope; kv_len is then the cache capacity).
 void launch_gemv_seq(mdma_ctx *ctx, const GemvJob &j, const float *x, uint64_t T);
+// Up to 3 jobs sharing x: one launch for a few tokens over prepared rows of
+// one type, else job by job; the same bits.
+void launch_gemv_seq(mdma_ctx *ctx, const GemvJob *jobs, int n, const float *x, uint64_t T);
 void launch_rmsnorm_seq(mdma_ctx *ctx, const float *w, uint64_t dim, const float *a, const float *b, float *sum,
                         float *y, uint64_t rows, float eps);
 void launch_silu_mul_seq(mdma_ctx *ctx, const float *g, const float *u, float *y, uint64_t n);

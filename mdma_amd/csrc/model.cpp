@@ -373,7 +373,7 @@ void gemv(mdma_ctx *ctx, const GemvJob *jobs, int n, const float *x, uint64_t T,
   if (ctx->act_mode == MDMA_ACT_I8)
     launch_gemv_i8(ctx, jobs, n, x, T);
   else if (ctx->act_mode == MDMA_ACT_F32_CPU)
-    for (int i = 0; i < n; i++) launch_gemv_seq(ctx, jobs[i], x, T);
+    launch_gemv_seq(ctx, jobs, n, x, T);
   else
     launch_gemv_f32(ctx, jobs, n, x, T);
 }
@@ -386,8 +386,8 @@ void gemv_gated(mdma_ctx *ctx, const GemvJob &g, const GemvJob &u, const float *
   if (ctx->act_mode == MDMA_ACT_I8) {
     launch_gemv_i8_gated(ctx, g, u, x, T, y);
   } else if (ctx->act_mode == MDMA_ACT_F32_CPU) {
-    launch_gemv_seq(ctx, g, x, T);
-    launch_gemv_seq(ctx, u, x, T);
+    const GemvJob gu[2] = {g, u};
+    launch_gemv_seq(ctx, gu, 2, x, T);
     launch_silu_mul_seq(ctx, g.y, u.y, y, T * g.n_out);
   } else {
     launch_gemv_f32_gated(ctx, g, u, x, T, y);

@@ -107,6 +107,33 @@ def test_ragged_tokens_and_raw_layout(cpu_mode, T):
             assert np.array_equal(bits(got), bits(want)), (dtype, layout)
 
 
+@pytest.mark.parametrize("dtype,k", [(Q4K, 256), (Q4K, 1280), (Q6K, 768), (Q6K, 2560), (Q8, 32), (Q8, 288), (Q8, 4096)])
+@pytest.mark.parametrize("T", [1, 2, 4, 5])
+def test_fused_projections_at_tile_edges(cpu_mode, dtype, k, T):
+    # The split kernel's 16-row tiles and whole stages (512 columns, 256 for
+    # Q8_0 or several tokens) with remainders of both, three jobs per launch.
+    be = cpu_mode
+    rows = (33, 1, 16)
+    raws = [synth.weight(dtype, r, k, 9 * r + k, True) for r in rows]
+    x = synth.normal_f32(T * k, T + k)
+    outs = [be.f32_buf(np.full(T * r + 8, CANARY, np.float32)) for r in rows]
+    be.qmatmul_qkv(*(be.upload_weight(raw, dtype, (r, k)) for raw, r in zip(raws, rows)), be.f32_buf(x), *outs)
+    for raw, r, o in zip(raws, rows, outs):
+        got = be.download_f32(o)
+        assert np.all(got[T * r:] == CANARY), "wrote past the output"
+        assert np.array_equal(bits(got[:T * r].reshape(T, r)), bits(ffi.qmatmul(dtype, raw, r, k, x))), r
+
+
+@pytest.mark.parametrize("dtype,k", [(Q4K, 256), (Q4K, 768), (Q6K, 512), (Q8, 160)])
+def test_wide_workgroups_at_tile_edges(cpu_mode, dtype, k):
+    # One token over more rows than the 16-row tiles take: 64-row workgroups.
+    rows = 16384 + 65
+    raw = synth.weight(dtype, rows, k, k, True)
+    x = synth.normal_f32(k, 5)
+    got = gpu_qmatmul(cpu_mode, weight(cpu_mode, dtype, raw, rows, k, "prepared"), rows, x, 1)
+    assert np.array_equal(bits(got), bits(ffi.qmatmul(dtype, raw, rows, k, x)))
+
+
 @pytest.mark.parametrize("dtype", [F32, F16])
 def test_float_weights_bit_equal_oracle(cpu_mode, dtype):
     rows, k, T = 33, 100, 3
@@ -139,6 +166,16 @@ def test_rmsnorm_and_add_rmsnorm_bit_equal(cpu_mode):
         ws, wy = ffi.add_rmsnorm(w, a, b, 1e-5)
         assert np.array_equal(bits(be.download_f32(s)), bits(ws))
         assert np.array_equal(bits(be.download_f32(y)), bits(wy))
+
+
+@pytest.mark.parametrize("dim,rows", [(1, 2), (35, 2), (8192, 1), (8193, 2), (8224, 1)])
+def test_rmsnorm_bit_equal_at_chunk_edges(cpu_mode, dim, rows):
+    # The squares go through LDS 8192 at a time, added 32 at a time and singly.
+    be = cpu_mode
+    w, a = synth.normal_f32(dim, dim), synth.normal_f32(rows * dim, 1) * 3
+    y = be.alloc(rows * dim * 4)
+    be.rmsnorm(be.f32_buf(w), be.f32_buf(a), y, 1e-5)
+    assert np.array_equal(bits(be.download_f32(y)), bits(ffi.rmsnorm(w, a, 1e-5)))
 
 
 def silu_inputs():
