@@ -1,0 +1,406 @@
+// f32-activation GEMM of several tokens on the f64 matrix cores, over the
+// prepared Q4_K / Q6_K / Q8_0 layouts (layout.cpp).
+//
+// y[t, r] = sum_i deq(W)[r, i] * x[t, i], the reference's Backend::qmatmul
+// (/root/reference/src/backend.rs:469) with the f32 mode's arithmetic: every
+// weight a double formed from its quant byte (byte_f64 and one FMA), every
+// product exact in the double it is added in, one f32 rounding at the end.
+//
+// What bounds it is v_mfma_f64_16x16x4 itself: 64 cycles for 2048
+// operations, 70 TFLOP/s on the whole chip (measured); the row teams it
+// replaces did the same sums in 8-token launches on the VALU, 6.5 TFLOP/s
+// (300 tokens: gate/up 2x14336x4096 Q4_K 9.88 -> 1.25 ms, 4096x14336 Q6_K
+// 5.13 -> 0.66 ms, 53 to 56 TFLOP/s of the operations asked for).
+// So the design keeps the rest out of the matrix core's way:
+//  - Weights go from HBM to registers to operands, no LDS: lane l supplies
+//    row l % 16 of a 16-row tile for the k group g = l / 16, and since a sum
+//    over k may be taken in any order, group g simply walks the 64 columns
+//    of unit g of the 256-column block: 16-byte plane loads, and per weight
+//    one v_perm_b32 and one f64 FMA, issued under the MFMAs.
+//  - x goes to LDS by DMA as f32, one token row of 256 columns per wave
+//    instruction, double-buffered by block, and is read 4 columns at a time
+//    and converted as it is read.
+//  - A block takes a wave 3.5 us per 16-token tile, so one wave per SIMD
+//    hides every load of the next block behind the current one.
+//  - The (tile, block) pairs of the whole launch are dealt out evenly in one
+//    contiguous run per workgroup, so every CU stays busy to the end whatever
+//    the rows and tokens; a tile cut by a run's end is left as f64 partials
+//    that a second kernel adds in run order (fixed order: the same bits every
+//    time). A tile is 64 us to 1 ms of work, its partials 64 KB.
+#include <algorithm>
+
+#include "kernels.h"
+
+namespace mdma {
+namespace {
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t BK = 256;           // columns of a block
+constexpr uint32_t XP = BK + 4;        // LDS pitch of a token's block (floats): 16 tokens on distinct banks
+constexpr int RW = 2;                  // 16-row tiles per wave
+constexpr uint32_t TR = 4 * RW * 16;   // rows of a workgroup's tile (gated: half gate, half up)
+
+struct F64Args {
+  const uint8_t *w[3];
+  float *y[3];
+  uint32_t n_out[3];
+  uint32_t tiles[3];  // row tiles of each job
+  const float *x;
+  uint64_t row_bytes;
+  uint32_t n_in, T, nb, nt;  // nb: blocks of a row; nt: token tiles
+  uint32_t per_q, per_r;     // run of workgroup w: [w per_q + min(w, per_r), ...)
+  uint32_t units;            // tiles * nb
+  double *part;              // [workgroup][2][RW * TW * 4][256], or null: runs are whole tiles
+};
+
+// A lane's 64 columns of a 256-column block: raw bytes, their quads (4
+// columns each) and the coefficients of w = c1 (2 + byte / 2048) + c0.
+template <int DT>
+struct Unit64;
+
+template <>
+struct Unit64<DT_Q4_K> {
+  uint4 a, b, hd;
+  double c1[2], c0[2];
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t b0, uint32_t g, uint32_t n_in) {
+    const uint32_t U = n_in / 64, u = 4 * b0 + g;
+    a = ld16(row + 16 * (size_t)u);
+    b = ld16(row + 16 * (size_t)(U + u));
+    hd = ldx16(row + 32 * (size_t)U + 16 * (size_t)b0);
+  }
+  __device__ __forceinline__ void coef(uint32_t, uint32_t g, uint32_t) {
+    int s[2], m[2];
+    q4k_scales_i(hd, g, s[0], s[1], m[0], m[1]);
+    const float d = h2f(hd.x), dmin = h2f(hd.x >> 16);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const double ds = (double)(d * (float)s[i]), dm = (double)(dmin * (float)m[i]);
+      c1[i] = 2048.0 * ds;
+      c0[i] = -fma(4096.0, ds, dm);
+    }
+  }
+  __device__ static __forceinline__ int part(int i) { return i >> 3; }
+  __device__ static __forceinline__ uint32_t col(uint32_t g, int i) { return 64 * g + 4 * i; }
+  __device__ __forceinline__ uint32_t quad(int i) const {
+    const uint32_t q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    return (i < 8 ? q[i & 7] : q[i & 7] >> 4) & 0x0F0F0F0Fu;
+  }
+};
+
+template <>
+struct Unit64<DT_Q6_K> {
+  uint4 a, b, q;
+  uint32_t sc, d;
+  double c1[4], c0[4];
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t b0, uint32_t g, uint32_t n_in) {
+    const uint32_t U = n_in / 64, u = 4 * b0 + g;
+    a = ld16(row + 16 * (size_t)u);
+    b = ld16(row + 16 * (size_t)(U + u));
+    q = ld16(row + 16 * (size_t)(2 * U + u));
+    sc = *reinterpret_cast<const uint32_t *>(row + 48 * (size_t)U + 4 * (size_t)u);
+    d = ldu16(row + 52 * (size_t)U + 2 * (size_t)b0);
+  }
+  __device__ __forceinline__ void coef(uint32_t, uint32_t, uint32_t) {
+    const double df = (double)h2f(d);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const double ds = df * (double)(int)(int8_t)((sc >> (8 * r)) & 0xff);
+      c1[r] = 2048.0 * ds;
+      c0[r] = -4128.0 * ds;
+    }
+  }
+  __device__ static __forceinline__ int part(int i) { return i >> 2; }
+  __device__ static __forceinline__ uint32_t col(uint32_t g, int i) {
+    return 128 * (g >> 1) + 16 * (g & 1) + 32 * (i >> 2) + 4 * (i & 3);
+  }
+  __device__ __forceinline__ uint32_t quad(int i) const {
+    const uint32_t qa[4] = {a.x, a.y, a.z, a.w}, qb[4] = {b.x, b.y, b.z, b.w}, qh[4] = {q.x, q.y, q.z, q.w};
+    const int r = i >> 2, k = i & 3;
+    const uint32_t low = ((r & 1 ? qb[k] : qa[k]) >> (r < 2 ? 0 : 4)) & 0x0F0F0F0Fu;
+    const uint32_t h = r == 0 ? qh[k] << 4 : r == 1 ? qh[k] << 2 : r == 2 ? qh[k] : qh[k] >> 2;
+    return low | (h & 0x30303030u);
+  }
+};
+
+// Q8_0: units (blocks) g and g + 4 of the 8 in a 256-column block; units
+// past the row's end count as zero weights.
+template <>
+struct Unit64<DT_Q8_0> {
+  uint4 a[2], b[2];
+  uint32_t d[2];
+  double c1[2], c0[2];
+  __device__ __forceinline__ void load(const uint8_t *row, uint32_t b0, uint32_t g, uint32_t n_in) {
+    const uint32_t U = n_in / 32;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const uint32_t u = min(8 * b0 + g + 4 * i, U - 1);
+      a[i] = ld16(row + 16 * (size_t)u);
+      b[i] = ld16(row + 16 * (size_t)(U + u));
+      d[i] = ldu16(row + 32 * (size_t)U + 2 * (size_t)u);
+    }
+  }
+  __device__ __forceinline__ void coef(uint32_t b0, uint32_t g, uint32_t n_in) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const double ds = 8 * b0 + g + 4 * i < n_in / 32 ? (double)h2f(d[i]) : 0.0;
+      c1[i] = 2048.0 * ds;
+      c0[i] = -4224.0 * ds;
+    }
+  }
+  __device__ static __forceinline__ int part(int i) { return i >> 3; }
+  __device__ static __forceinline__ uint32_t col(uint32_t g, int i) { return 32 * g + 128 * (i >> 3) + 4 * (i & 7); }
+  __device__ __forceinline__ uint32_t quad(int i) const {
+    const int h = i >> 3;
+    const uint32_t q[8] = {a[h].x, a[h].y, a[h].z, a[h].w, b[h].x, b[h].y, b[h].z, b[h].w};
+    return q[i & 7] ^ 0x80808080u;
+  }
+};
+
+// A tile's place: its job, first row and first token.
+template <int TW>
+struct Place {
+  const uint8_t *w;
+  float *y;
+  uint32_t n_out, row0, tok0;
+};
+template <int TW, bool GLU>
+__device__ __forceinline__ Place<TW> place(const F64Args &a, uint32_t tile) {
+  uint32_t rt = tile / a.nt;
+  const uint32_t tok0 = (tile - rt * a.nt) * (16 * TW);
+  const int j = GLU || rt < a.tiles[0] ? 0 : rt < a.tiles[0] + a.tiles[1] ? 1 : 2;
+  rt -= j > 0 ? a.tiles[0] : 0;
+  rt -= j > 1 ? a.tiles[1] : 0;
+  return Place<TW>{j == 0 ? a.w[0] : j == 1 ? a.w[1] : a.w[2], j == 0 ? a.y[0] : j == 1 ? a.y[1] : a.y[2],
+                   j == 0 ? a.n_out[0] : j == 1 ? a.n_out[1] : a.n_out[2], rt * (GLU ? TR / 2 : TR), tok0};
+}
+
+// The accumulators of v_mfma_f64_16x16x4 with x as A and w as B: element r
+// of lane l is token 4 r + l / 16, row l % 16 of the 16x16 tile.
+template <int TW, bool GLU>
+__device__ __forceinline__ void store_tile(const F64Args &a, const Place<TW> &p, const v4d (&acc)[RW][TW], float *yg,
+                                           uint32_t wave, uint32_t lane) {
+#pragma unroll
+  for (int t = 0; t < TW; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const uint32_t tok = p.tok0 + 16 * t + 4 * r + lane / 16;
+      if (tok >= a.T) continue;
+      if (GLU) {
+        const uint32_t row = p.row0 + 16 * wave + lane % 16;
+        if (row < p.n_out) yg[(size_t)tok * p.n_out + row] = silu_mul1((float)acc[0][t][r], (float)acc[1][t][r]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < RW; i++) {
+          const uint32_t row = p.row0 + 16 * (RW * wave + i) + lane % 16;
+          if (row < p.n_out) p.y[(size_t)tok * p.n_out + row] = (float)acc[i][t][r];
+        }
+      }
+    }
+}
+
+__device__ __forceinline__ uint32_t run_start(const F64Args &a, uint32_t w) { return w * a.per_q + min(w, a.per_r); }
+
+template <int DT, int TW, bool GLU>
+__global__ __launch_bounds__(256, TW <= 2 ? 2 : 1) void gemm_f64_kernel(F64Args a, float *yg) {
+  __shared__ __attribute__((aligned(16))) float xs[2][16 * TW][XP];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t g = lane / 16, l16 = lane % 16;
+  // Contiguous runs on one XCD (workgroups go to the 8 XCDs round-robin), so
+  // neighbouring tiles share their weights and x in its L2.
+  const uint32_t G = gridDim.x, wg = G % 8 ? blockIdx.x : (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
+  uint32_t u = run_start(a, wg);
+  const uint32_t u_end = min(run_start(a, wg + 1), a.units);
+  bool first = true;
+  while (u < u_end) {
+    const uint32_t tile = u / a.nb, b0 = u - tile * a.nb, b1 = min(a.nb, b0 + (u_end - u));
+    const Place<TW> p = place<TW, GLU>(a, tile);
+    const uint8_t *wr[RW];
+#pragma unroll
+    for (int i = 0; i < RW; i++) {
+      const uint32_t row = GLU ? p.row0 + 16 * wave + l16 : p.row0 + 16 * (RW * wave + i) + l16;
+      wr[i] = (GLU && i ? a.w[1] : p.w) + (size_t)min(row, p.n_out - 1) * a.row_bytes;
+    }
+    // x of a block: one DMA per token row, the wave's rows wave * 4 TW ..
+    auto load_x = [&](uint32_t b, uint32_t buf) {
+      const uint32_t col = min(b * BK + 4 * lane, a.n_in - 4);
+#pragma unroll
+      for (int i = 0; i < 4 * TW; i++) {
+        const uint32_t r = wave * (4 * TW) + i, tok = min(p.tok0 + r, a.T - 1);
+        lds_dma16(a.x + (size_t)tok * a.n_in, 4 * col, &xs[buf][r][0]);
+      }
+    };
+    v4d acc[RW][TW];
+#pragma unroll
+    for (int i = 0; i < RW; i++)
+#pragma unroll
+      for (int t = 0; t < TW; t++) acc[i][t] = v4d{0, 0, 0, 0};
+    Unit64<DT> cur[RW], nxt[RW];
+    lds_barrier();  // the previous tile's reads of xs are done
+    load_x(b0, b0 & 1);
+#pragma unroll
+    for (int i = 0; i < RW; i++) nxt[i].load(wr[i], b0, g, a.n_in);
+    for (uint32_t b = b0; b < b1; b++) {
+#pragma unroll
+      for (int i = 0; i < RW; i++) {
+        cur[i] = nxt[i];
+        cur[i].coef(b, g, a.n_in);
+      }
+      lds_wait_dma();
+      lds_barrier();  // every wave's x of block b is in LDS; block b - 1's reads are done
+      if (b + 1 < b1) {
+        load_x(b + 1, (b + 1) & 1);
+#pragma unroll
+        for (int i = 0; i < RW; i++) nxt[i].load(wr[i], b + 1, g, a.n_in);
+      }
+      const float(*xb)[XP] = xs[b & 1];
+#pragma unroll
+      for (int s = 0; s < 16; s++) {
+        v4f xv[TW];
+#pragma unroll
+        for (int t = 0; t < TW; t++)
+          xv[t] = *reinterpret_cast<const v4f *>(&xb[16 * t + l16][Unit64<DT>::col(g, s)]);
+        uint32_t q[RW];
+#pragma unroll
+        for (int i = 0; i < RW; i++) q[i] = cur[i].quad(s);
+        const int c = Unit64<DT>::part(s);
+#define MDMA_F64_STEP(K)                                                                        \
+  {                                                                                             \
+    double wv[RW];                                                                              \
+    _Pragma("unroll") for (int i = 0; i < RW; i++)                                              \
+        wv[i] = fma(cur[i].c1[c], byte_f64<K>(q[i]), cur[i].c0[c]);                             \
+    _Pragma("unroll") for (int t = 0; t < TW; t++) {                                            \
+      const double xd = (double)xv[t][K];                                                       \
+      _Pragma("unroll") for (int i = 0; i < RW; i++)                                            \
+          acc[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(xd, wv[i], acc[i][t], 0, 0, 0);      \
+    }                                                                                           \
+  }
+        MDMA_F64_STEP(0)
+        MDMA_F64_STEP(1)
+        MDMA_F64_STEP(2)
+        MDMA_F64_STEP(3)
+#undef MDMA_F64_STEP
+      }
+    }
+    if (b0 == 0 && b1 == a.nb) {
+      store_tile<TW, GLU>(a, p, acc, yg, wave, lane);
+    } else {  // (only with a.part: a run's first or last tile)
+      double *o = a.part + (size_t)(2 * wg + (first ? 0 : 1)) * (RW * TW * 4) * 256 + threadIdx.x;
+#pragma unroll
+      for (int i = 0; i < RW; i++)
+#pragma unroll
+        for (int t = 0; t < TW; t++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) o[((i * TW + t) * 4 + r) * 256] = acc[i][t][r];
+    }
+    first = false;
+    u += b1 - b0;
+  }
+}
+
+// One workgroup per tile: the tiles that two or more runs share, their
+// partials added in run order.
+template <int TW, bool GLU>
+__global__ __launch_bounds__(256) void gemm_f64_merge_kernel(F64Args a, uint32_t G, float *yg) {
+  const uint32_t tile = blockIdx.x, ub = tile * a.nb, ue = ub + a.nb;
+  // The run holding unit u.
+  auto run_of = [&](uint32_t u) {
+    const uint32_t big = a.per_r * (a.per_q + 1);
+    return u < big ? u / (a.per_q + 1) : a.per_r + (u - big) / a.per_q;
+  };
+  const uint32_t w0 = run_of(ub), w1 = run_of(ue - 1);
+  if (w0 == w1) return;
+  const Place<TW> p = place<TW, GLU>(a, tile);
+  v4d acc[RW][TW];
+  for (uint32_t w = w0; w <= w1; w++) {
+    // The run's first piece is its slot 0, a later one (its last) slot 1.
+    const double *o = a.part + (size_t)(2 * w + (run_start(a, w) >= ub ? 0 : 1)) * (RW * TW * 4) * 256 + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < RW; i++)
+#pragma unroll
+      for (int t = 0; t < TW; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const double v = o[((i * TW + t) * 4 + r) * 256];
+          acc[i][t][r] = w == w0 ? v : acc[i][t][r] + v;
+        }
+  }
+  store_tile<TW, GLU>(a, p, acc, yg, threadIdx.x >> 6, threadIdx.x & 63);
+}
+
+template <int DT, int TW, bool GLU>
+void launch(mdma_ctx *ctx, F64Args &a, uint32_t tiles, float *yg) {
+  const uint32_t units = tiles * a.nb;  // (checked to fit by the caller)
+  uint32_t G = (uint32_t)ctx->cu_count * (TW <= 2 ? 2 : 1);
+  if (G > units) G = units;
+  a.units = units;
+  a.part = tiles % G ? static_cast<double *>(f64_parts(ctx, (uint64_t)G * 2 * RW * TW * 4 * 256 * 8)) : nullptr;
+  if (a.part) {
+    a.per_q = units / G, a.per_r = units % G;
+  } else {  // runs of whole tiles
+    const uint32_t n = (tiles + G - 1) / G;
+    G = (tiles + n - 1) / n;
+    a.per_q = n * a.nb, a.per_r = 0;
+  }
+  gemm_f64_kernel<DT, TW, GLU><<<dim3(G), dim3(256), 0, ctx->stream>>>(a, yg);
+  hip_check(hipGetLastError(), "gemm_f64 launch");
+  if (a.part) {
+    gemm_f64_merge_kernel<TW, GLU><<<dim3(tiles), dim3(256), 0, ctx->stream>>>(a, G, yg);
+    hip_check(hipGetLastError(), "gemm_f64 merge launch");
+  }
+}
+
+template <int DT, bool GLU>
+void launch_tw(mdma_ctx *ctx, F64Args &a, int tw, uint32_t tiles, float *yg) {
+  switch (tw) {
+    case 1: launch<DT, 1, GLU>(ctx, a, tiles, yg); break;
+    case 2: launch<DT, 2, GLU>(ctx, a, tiles, yg); break;
+    case 3: launch<DT, 3, GLU>(ctx, a, tiles, yg); break;
+    default: launch<DT, 4, GLU>(ctx, a, tiles, yg); break;
+  }
+}
+
+}  // namespace
+
+bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T, float *glu_y) {
+  const GemvJob &j0 = jobs[0];
+  const bool glu = glu_y != nullptr;
+  if (T < F64_MIN_TOKENS || T > 1u << 20 || n_jobs < 1 || n_jobs > 3 || !j0.n_in || j0.n_in > 1u << 20 ||
+      j0.layout != MDMA_LAYOUT_GFX950 || j0.n_in % block_size(j0.dtype))
+    return false;
+  F64Args a{};
+  uint64_t row_tiles = 0;
+  for (int i = 0; i < n_jobs; i++) {
+    if (jobs[i].layout != j0.layout || jobs[i].dtype != j0.dtype || jobs[i].n_in != j0.n_in || !jobs[i].n_out ||
+        jobs[i].n_out > 1u << 24 || (glu && jobs[i].n_out != j0.n_out))
+      return false;
+    a.w[i] = jobs[i].w;
+    a.y[i] = jobs[i].y;
+    a.n_out[i] = (uint32_t)jobs[i].n_out;
+    a.tiles[i] = (uint32_t)((jobs[i].n_out + (glu ? TR / 2 : TR) - 1) / (glu ? TR / 2 : TR));
+    if (!glu || i == 0) row_tiles += a.tiles[i];
+  }
+  // Token tiles of 16 tw tokens, tw <= 4: as few as cover T, then as narrow
+  // as still do (the 16-token tiles past T are the only padding).
+  const uint64_t t16 = (T + 15) / 16;
+  a.nt = (uint32_t)((t16 + 3) / 4);
+  const int tw = (int)((t16 + a.nt - 1) / a.nt);
+  a.nb = (uint32_t)((j0.n_in + BK - 1) / BK);
+  if (row_tiles * a.nt * a.nb > 0x7fffffffull) return false;
+  a.x = x;
+  a.row_bytes = gfx950_row_bytes(j0.dtype, j0.n_in);
+  a.n_in = (uint32_t)j0.n_in;
+  a.T = (uint32_t)T;
+  const uint32_t tiles = (uint32_t)row_tiles * a.nt;
+#define MDMA_F64_GO(DT)                                 \
+  if (glu) launch_tw<DT, true>(ctx, a, tw, tiles, glu_y); \
+  else launch_tw<DT, false>(ctx, a, tw, tiles, nullptr)
+  if (j0.dtype == DT_Q4_K) { MDMA_F64_GO(DT_Q4_K); }
+  else if (j0.dtype == DT_Q6_K) { MDMA_F64_GO(DT_Q6_K); }
+  else { MDMA_F64_GO(DT_Q8_0); }
+#undef MDMA_F64_GO
+  return true;
+}
+
+}  // namespace mdma

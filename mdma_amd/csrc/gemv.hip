@@ -853,6 +853,7 @@ static bool any_prepared(const GemvJob *jobs, int n) {
 }
 
 void launch_gemv_f32(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T) {
+  if (launch_gemm_f64(ctx, jobs, n_jobs, x, T)) return;
   if (team_layout_ok(jobs, n_jobs)) {
     launch_gemv_team(ctx, MDMA_ACT_F32, jobs, n_jobs, false, x, T, nullptr);
     return;
@@ -871,6 +872,7 @@ void launch_gemv_f32(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
 void launch_gemv_f32_gated(mdma_ctx *ctx, const GemvJob &gate, const GemvJob &up, const float *x, uint64_t T,
                            float *y) {
   const GemvJob gu[2] = {gate, up};
+  if (launch_gemm_f64(ctx, gu, 2, x, T, y)) return;
   if (team_layout_ok(gu, 2)) {
     launch_gemv_team(ctx, MDMA_ACT_F32, gu, 2, true, x, T, y);
     return;

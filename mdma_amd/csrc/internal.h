@@ -142,6 +142,9 @@ struct mdma_ctx {
   uint64_t attn_cnt_cap = 0;
   uint32_t *gemm_cnt = nullptr;  // split-K GEMM arrival counters (zero between launches)
   uint64_t gemm_cnt_cap = 0;
+  char *f64_part = nullptr;  // partial tiles of the f64 GEMM
+  uint64_t f64_part_cap = 0;
+  bool f64_part_captured = false;  // a captured launch points into it
   double *ssq = nullptr;  // per-workgroup sums of squares of a residual-stream GEMV (norm fusion)
   uint64_t ssq_cap = 0;
   uint32_t team_grid = 0;  // workgroups of the last row-team launch
@@ -378,6 +381,19 @@ bool gemm_f16_glu_ok(const GemvJob &gate, const GemvJob &up);
 void launch_gemm_f16(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t M, char *scratch,
                      float *part, uint64_t part_bytes, uint32_t *cnt, uint64_t counters, float *glu_y = nullptr,
                      bool have_input = false);
+// f32-mode GEMM on the f64 matrix cores (gemm_f64.hip) for F64_MIN_TOKENS
+// tokens and up: up to 3 prepared jobs of one type sharing x, or (glu_y) gate
+// and up with silu(gate) * up written there. False, launching nothing, where
+// it does not cover the call (another layout, mixed types).
+// At 4 tokens and fewer the row teams are as fast (4096x14336 Q6_K at 3
+// tokens 52 us against 67; from 5 they take an 8-token launch: 130 us).
+constexpr uint64_t F64_MIN_TOKENS = 5;
+bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T,
+                     float *glu_y = nullptr);
+// Device space for its partial tiles, or null where it may not grow now (a
+// capture, an allocation-free call, a full budget or device): the launch then
+// runs unsplit.
+void *f64_parts(mdma_ctx *ctx, uint64_t bytes);
 void launch_quantize_act(mdma_ctx *ctx, const float *x, uint64_t n, uint64_t group, int8_t *q,
                          float *d, int32_t *sum16);
 void launch_block_dot(mdma_ctx *ctx, const GemvJob &w, const int8_t *qx, uint64_t T, int32_t *out);

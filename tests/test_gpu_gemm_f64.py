@@ -1,0 +1,115 @@
+"""The f32 mode's several-token kernels (f64 matrix cores) at the sizes where
+their tiles, blocks and work split have remainders, against the f64 dot
+product of the dequantized weights: every output must be as close to it as the
+CPU's sequential f32 sum is (assert_parity, correctly_rounded), which a sum in
+f64 rounded once meets."""
+import numpy as np
+import pytest
+
+import npq
+from conftest import assert_parity, f32_exact
+from mdma_amd import synth
+from mdma_amd.backend import DOMAIN_DEVICE, Gfx950Backend
+from oracle import ffi
+
+pytestmark = pytest.mark.gpu
+Q8, Q4K, Q6K = 8, 12, 14
+CANARY = np.float32(123456.25)
+
+
+def out_buf(be, n):
+    return be.f32_buf(np.full(n + 8, CANARY, np.float32))
+
+
+def check(be, buf, T, dtype, raw, rows, k, x, what):
+    got = be.download_f32(buf)
+    assert np.all(got[T * rows:] == CANARY), f"{what}: wrote past the output"
+    exact = f32_exact(npq.dequantize(dtype, raw, rows, k), x)
+    assert_parity(got[:T * rows], ffi.qmatmul(dtype, raw, rows, k, x), exact, 1e-5, what=what, correctly_rounded=True)
+
+
+@pytest.mark.parametrize("dtype,k", [(Q4K, 256), (Q4K, 2304), (Q6K, 256), (Q6K, 2560), (Q8, 32), (Q8, 288), (Q8, 2048)])
+@pytest.mark.parametrize("T", [2, 4, 5, 8, 9, 16, 17, 33, 49, 64, 65, 130])
+def test_projections_at_tile_edges(backend, dtype, k, T):
+    # Three jobs per launch: one row, one tile of rows and one more, several.
+    rows = (129, 1, 300)
+    raws = [synth.weight(dtype, r, k, 3 * r + k, True) for r in rows]
+    x = synth.normal_f32(T * k, T + k)
+    outs = [out_buf(backend, T * r) for r in rows]
+    backend.qmatmul_qkv(*(backend.upload_weight(raw, dtype, (r, k)) for raw, r in zip(raws, rows)),
+                        backend.f32_buf(x), *outs)
+    for raw, r, o in zip(raws, rows, outs):
+        check(backend, o, T, dtype, raw, r, k, x, f"dtype={dtype} k={k} T={T} rows={r}")
+
+
+@pytest.mark.parametrize("dtype,k", [(Q4K, 1280), (Q6K, 512), (Q8, 288)])
+@pytest.mark.parametrize("T", [2, 4, 7, 16, 40, 100])
+def test_gate_up_at_tile_edges(backend, dtype, k, T):
+    # silu(gate) * up of outputs rounded once: equal to the separate calls' up
+    # to the few ulps of silu_mul's own roundings.
+    rows = 97
+    raws = [synth.weight(dtype, rows, k, s, True) for s in (5, 6)]
+    w = [backend.upload_weight(r, dtype, (rows, k)) for r in raws]
+    x = backend.f32_buf(synth.normal_f32(T * k, T) * 0.1)
+    g, u, gs, us = (backend.alloc(T * rows * 4) for _ in range(4))
+    y, want = out_buf(backend, T * rows), backend.alloc(T * rows * 4)
+    backend.ffn_gate_up(w[0], w[1], x, gs, us, y)
+    backend.qmatmul(w[0], x, g)
+    backend.qmatmul(w[1], x, u)
+    backend.silu_mul(g, u, want)
+    got, ref = backend.download_f32(y), backend.download_f32(want)
+    assert np.all(got[T * rows:] == CANARY)
+    assert np.allclose(got[:T * rows], ref, rtol=6 * 2.0**-24, atol=0)
+
+
+def test_captured_launch_without_partials_space(backend):
+    # Under capture the partial tiles' space cannot be made: the launch runs
+    # unsplit, and its replays give the eager results.
+    be = Gfx950Backend(0)
+    rows, k, T = 200, 1024, 70
+    raw = synth.weight(Q6K, rows, k, 1, True)
+    w, x_h = be.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
+    x, y = be.f32_buf(x_h), out_buf(be, T * rows)
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        be.qmatmul(w, x, be.alloc(T * rows * 4))  # eager: makes the space; the graph does not hold it
+        graph.launch()
+        check(be, y, T, Q6K, raw, rows, k, x_h, "captured")
+    graph.close()
+    be.close()
+
+
+def test_partials_space_gives_way_to_the_budget():
+    be = Gfx950Backend(0)
+    rows, k, T = 200, 1024, 70
+    raw = synth.weight(Q4K, rows, k, 1, True)
+    be.set_buffer_budget(device=80 << 20)
+    w, x_h = be.upload_weight(raw, Q4K, (rows, k)), synth.normal_f32(T * k, 2)
+    x, y = be.f32_buf(x_h), out_buf(be, T * rows)
+    before, limit = be.buffer_usage(DOMAIN_DEVICE)
+    be.qmatmul(w, x, y)
+    assert be.buffer_usage(DOMAIN_DEVICE)[0] > before  # charged as it grew
+    rest = be.alloc(limit - before)  # all that the caller had left
+    assert be.buffer_usage(DOMAIN_DEVICE)[0] == limit
+    be.upload(y, 0, np.zeros(T * rows, np.float32))
+    be.qmatmul(w, x, y)  # no space: unsplit
+    check(be, y, T, Q4K, raw, rows, k, x_h, "over budget")
+    rest.close()
+    be.close()
+
+
+def test_nan_and_infinity_stay_in_their_token(backend):
+    rows, k, T = 64, 512, 20
+    raw = synth.weight(Q6K, rows, k, 1, True)
+    w, x_h = backend.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
+    clean, y = backend.alloc(T * rows * 4), backend.alloc(T * rows * 4)
+    backend.qmatmul(w, backend.f32_buf(x_h), clean)
+    bad = x_h.reshape(T, k).copy()
+    bad[3, 17], bad[18, 300] = np.nan, np.inf
+    backend.qmatmul(w, backend.f32_buf(bad), y)
+    got, ref = backend.download_f32(y).reshape(T, rows), backend.download_f32(clean).reshape(T, rows)
+    keep = [t for t in range(T) if t not in (3, 18)]
+    assert np.array_equal(got[keep], ref[keep])
+    assert np.isnan(got[3]).all() and not np.isfinite(got[18]).any()
+
