@@ -361,6 +361,147 @@ void launch_tw(mdma_ctx *ctx, F64Args &a, int tw, uint32_t tiles, float *yg) {
   }
 }
 
+// ---- 2 to 8 tokens ----
+// v_mfma_f64_4x4x4 does four 4x4x4 products in 18 cycles (measured, 62
+// TFLOP/s): its four blocks take the same 4 tokens and 4 rows each of a
+// 16-row tile, so up to 4 tokens cost about a third of the 16-token tile. It
+// does not overlap with the VALU (also measured: an MFMA and a v_perm_b32
+// take the sum of their times), so the products and the weights' two VALU
+// operations bound the kernel together, about 33 cycles per 64 weights and 4
+// tokens. us, row teams / here: gate/up 2x14336x4096 Q4_K T = 2: 73 / 38.7,
+// 4: 135 / 45, 8: 267 / 62 (the 16-token tile: 83); 4096x14336 Q6_K 40 / 24.4,
+// 66 / 26.6, 134 / 41.5. Lane l supplies
+// row l % 16 of the tile and token l % 4, both for k group l / 16, as above,
+// and holds the sum of token l / 16, row l % 16.
+//
+// The NW waves of a workgroup take the blocks of a 16-row tile (gated: 16
+// rows of gate and the same of up) in turn, so that neighbouring waves read
+// neighbouring 64 bytes of a row, and add their sums in wave order through
+// LDS. x comes by DMA into the wave's own double buffer: no barrier but the
+// one per tile. The next block's loads are in flight behind the current one's
+// products, across tiles too.
+template <int DT, int TT, bool GLU, int NW>
+__global__ __launch_bounds__(64 * NW, TT <= 4 ? 4 : 2) void gemv_f64_kernel(F64Args a, float *yg) {
+  constexpr int R = GLU ? 2 : 1, NT = (TT + 3) / 4, RB = TT <= 4 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) float xs[NW][2][TT][XP];
+  __shared__ __attribute__((aligned(16))) double red[RB][NW][R * NT][64];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t g = lane / 16, l16 = lane % 16;
+  const uint32_t tiles = a.units;
+  struct At {
+    const uint8_t *w;
+    float *y;
+    uint32_t n_out, row0;
+  };
+  auto at = [&](uint32_t rt) {
+    const int j = GLU || rt < a.tiles[0] ? 0 : rt < a.tiles[0] + a.tiles[1] ? 1 : 2;
+    rt -= j > 0 ? a.tiles[0] : 0;
+    rt -= j > 1 ? a.tiles[1] : 0;
+    return At{j == 0 ? a.w[0] : j == 1 ? a.w[1] : a.w[2], j == 0 ? a.y[0] : j == 1 ? a.y[1] : a.y[2],
+              j == 0 ? a.n_out[0] : j == 1 ? a.n_out[1] : a.n_out[2], 16 * rt};
+  };
+  Unit64<DT> cur[R], nxt[R];
+  auto issue = [&](uint32_t tile, uint32_t b, uint32_t buf) {
+    const At p = at(tile);
+    const size_t off = (size_t)min(p.row0 + l16, p.n_out - 1) * a.row_bytes;
+#pragma unroll
+    for (int i = 0; i < R; i++) nxt[i].load((i ? a.w[1] : p.w) + off, b, g, a.n_in);
+    const uint32_t col = min(b * BK + 4 * lane, a.n_in - 4);
+#pragma unroll
+    for (int t = 0; t < TT; t++) lds_dma16(a.x + (size_t)min((uint32_t)t, a.T - 1) * a.n_in, 4 * col, &xs[wave][buf][t][0]);
+  };
+  uint32_t tile = blockIdx.x, buf = 0, par = 0;
+  if (wave < a.nb) issue(tile, wave, 0);
+  for (; tile < tiles; tile += gridDim.x) {
+    double acc[R][NT];
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) acc[i][t] = 0.0;
+    for (uint32_t b = wave; b < a.nb; b += NW) {
+      lds_wait_dma();
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        cur[i] = nxt[i];
+        cur[i].coef(b, g, a.n_in);
+      }
+      const bool more = b + NW < a.nb;
+      const uint32_t tn = more ? tile : tile + gridDim.x;
+      if (tn < tiles) issue(tn, more ? b + NW : wave, buf ^ 1);
+      const float(*xb)[XP] = xs[wave][buf];
+#pragma unroll
+      for (int s = 0; s < 16; s++) {
+        v4f xv[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          xv[t] = *reinterpret_cast<const v4f *>(&xb[TT == 2 ? lane & 1 : 4 * t + (lane & 3)]
+                                                   [Unit64<DT>::col(g, s)]);
+        uint32_t q[R];
+#pragma unroll
+        for (int i = 0; i < R; i++) q[i] = cur[i].quad(s);
+        const int c = Unit64<DT>::part(s);
+#define MDMA_F64_STEP(K)                                                                   \
+  {                                                                                        \
+    double wv[R];                                                                          \
+    _Pragma("unroll") for (int i = 0; i < R; i++)                                          \
+        wv[i] = fma(cur[i].c1[c], byte_f64<K>(q[i]), cur[i].c0[c]);                        \
+    _Pragma("unroll") for (int t = 0; t < NT; t++) {                                       \
+      const double xd = (double)xv[t][K];                                                  \
+      _Pragma("unroll") for (int i = 0; i < R; i++)                                        \
+          acc[i][t] = __builtin_amdgcn_mfma_f64_4x4x4f64(xd, wv[i], acc[i][t], 0, 0, 0);   \
+    }                                                                                      \
+  }
+        MDMA_F64_STEP(0)
+        MDMA_F64_STEP(1)
+        MDMA_F64_STEP(2)
+        MDMA_F64_STEP(3)
+#undef MDMA_F64_STEP
+      }
+      buf ^= 1;
+    }
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) red[par][wave][i * NT + t][lane] = acc[i][t];
+    lds_barrier();
+    if (wave < NT) {
+      double s[R];
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        s[i] = red[par][0][i * NT + wave][lane];
+#pragma unroll
+        for (int w = 1; w < NW; w++) s[i] += red[par][w][i * NT + wave][lane];
+      }
+      const At p = at(tile);
+      const uint32_t tok = 4 * wave + g, row = p.row0 + l16;
+      if (tok < a.T && row < p.n_out) {
+        if (GLU) yg[(size_t)tok * p.n_out + row] = silu_mul1((float)s[0], (float)s[R - 1]);
+        else p.y[(size_t)tok * p.n_out + row] = (float)s[0];
+      }
+    }
+    if (RB == 2) par ^= 1;
+    else lds_barrier();
+  }
+}
+
+template <int DT, int TT, bool GLU, int NW>
+void launch_small(mdma_ctx *ctx, F64Args &a, float *yg) {
+  const uint32_t G = std::min(a.units, (uint32_t)ctx->cu_count * (TT <= 4 ? 16 : 8) / NW);
+  gemv_f64_kernel<DT, TT, GLU, NW><<<dim3(G), dim3(64 * NW), 0, ctx->stream>>>(a, yg);
+  hip_check(hipGetLastError(), "gemv_f64 launch");
+}
+template <int DT, bool GLU>
+void launch_small_t(mdma_ctx *ctx, F64Args &a, float *yg) {
+  const bool wide = a.nb >= 8;
+#define MDMA_F64_T(TT)                                                    \
+  if (wide) launch_small<DT, TT, GLU, TT <= 4 ? 8 : 4>(ctx, a, yg);       \
+  else launch_small<DT, TT, GLU, 4>(ctx, a, yg)
+  if (a.T <= 2) { MDMA_F64_T(2); }
+  else if (a.T <= 4) { MDMA_F64_T(4); }
+  else { MDMA_F64_T(8); }
+#undef MDMA_F64_T
+}
+
 }  // namespace
 
 bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T, float *glu_y) {
@@ -381,25 +522,38 @@ bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
     a.tiles[i] = (uint32_t)((jobs[i].n_out + (glu ? TR / 2 : TR) - 1) / (glu ? TR / 2 : TR));
     if (!glu || i == 0) row_tiles += a.tiles[i];
   }
+  a.nb = (uint32_t)((j0.n_in + BK - 1) / BK);
+  a.x = x;
+  a.row_bytes = gfx950_row_bytes(j0.dtype, j0.n_in);
+  a.n_in = (uint32_t)j0.n_in;
+  a.T = (uint32_t)T;
+#define MDMA_F64_DT(GO)                            \
+  if (j0.dtype == DT_Q4_K) { GO(DT_Q4_K); }        \
+  else if (j0.dtype == DT_Q6_K) { GO(DT_Q6_K); }   \
+  else { GO(DT_Q8_0); }
+  if (T <= 8) {
+    a.units = 0;
+    for (int i = 0; i < (glu ? 1 : n_jobs); i++) a.units += a.tiles[i] = (a.n_out[i] + 15) / 16;
+#define MDMA_F64_GO(DT)                                  \
+  if (glu) launch_small_t<DT, true>(ctx, a, glu_y);      \
+  else launch_small_t<DT, false>(ctx, a, nullptr)
+    MDMA_F64_DT(MDMA_F64_GO)
+#undef MDMA_F64_GO
+    return true;
+  }
   // Token tiles of 16 tw tokens, tw <= 4: as few as cover T, then as narrow
   // as still do (the 16-token tiles past T are the only padding).
   const uint64_t t16 = (T + 15) / 16;
   a.nt = (uint32_t)((t16 + 3) / 4);
   const int tw = (int)((t16 + a.nt - 1) / a.nt);
-  a.nb = (uint32_t)((j0.n_in + BK - 1) / BK);
   if (row_tiles * a.nt * a.nb > 0x7fffffffull) return false;
-  a.x = x;
-  a.row_bytes = gfx950_row_bytes(j0.dtype, j0.n_in);
-  a.n_in = (uint32_t)j0.n_in;
-  a.T = (uint32_t)T;
   const uint32_t tiles = (uint32_t)row_tiles * a.nt;
 #define MDMA_F64_GO(DT)                                 \
   if (glu) launch_tw<DT, true>(ctx, a, tw, tiles, glu_y); \
   else launch_tw<DT, false>(ctx, a, tw, tiles, nullptr)
-  if (j0.dtype == DT_Q4_K) { MDMA_F64_GO(DT_Q4_K); }
-  else if (j0.dtype == DT_Q6_K) { MDMA_F64_GO(DT_Q6_K); }
-  else { MDMA_F64_GO(DT_Q8_0); }
+  MDMA_F64_DT(MDMA_F64_GO)
 #undef MDMA_F64_GO
+#undef MDMA_F64_DT
   return true;
 }
 

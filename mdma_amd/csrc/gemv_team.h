@@ -1,6 +1,6 @@
 // Decode GEMV on gfx950 over the prepared weight layouts (layout.cpp): the
-// streaming "row team" kernels, in the int8-activation and the
-// f32-activation mode, for 1..8 tokens. Instantiated per format and mode by
+// streaming "row team" kernels, for 1..8 tokens in the int8-activation mode
+// and one in the f32-activation mode (more: gemm_f64.hip). Instantiated per format and mode by
 // gemv_team_{q4,q6,q8}_{i8,f32}.hip; host entry points in gemv_team.hip.
 //
 // y[t, r] = sum_i deq(W)[r, i] * x[t, i]   (reference Backend::qmatmul,
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(team_wg(PRO, TW)) void gemv_team(TeamSet ts, const 
     uid[p] = uok[p] ? u : U - 1;
   }
   typename F::XI xi[F32 ? 1 : PL][F32 ? 1 : TT];
-  typename F::XF xr[F32 && TT == 1 ? PL : 1];
+  typename F::XF xr[F32 ? PL : 1];
   // Rows past the weight's end (last team of a job) re-read its last row;
   // their sums are not stored.
   typename F::W buf[NBUF][PL][NR];  // rotating row-group buffers
@@ -606,22 +606,12 @@ __global__ __launch_bounds__(team_wg(PRO, TW)) void gemv_team(TeamSet ts, const 
             }
           }
         }
-      } else if constexpr (TT == 1) {
+      } else {
+        static_assert(TT == 1, "f32 mode: one token (more: gemm_f64.hip)");
 #pragma unroll
         for (int r = 0; r < NR; r++) {
           const double v = F::dot_f32(w[p][r], xr[p], uid[p]);
           s[r][0] += uok[p] ? v : 0.0;
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-          if (t >= (int)T) break;
-          const typename F::XF xt = F::loadxf(xf + (size_t)t * n_in, uid[p]);
-#pragma unroll
-          for (int r = 0; r < NR; r++) {
-            const double v = F::dot_f32(w[p][r], xt, uid[p]);
-            s[r][t] += uok[p] ? v : 0.0;
-          }
         }
       }
     }
@@ -795,12 +785,10 @@ __global__ __launch_bounds__(team_wg(PRO, TW)) void gemv_team(TeamSet ts, const 
         xi[p][t] = F::loadxi(qx + (size_t)tc * n_in, dx + (size_t)tc * (n_in / 256),
                              s16 + (size_t)tc * (n_in / 16), uid[p]);
       }
-  } else if constexpr (TT == 1) {
+  } else {
     first_loads();
 #pragma unroll
     for (int p = 0; p < PL; p++) xr[p] = F::loadxf(xf, uid[p]);
-  } else {
-    first_loads();
   }
 
   // The team's run is ITERS row groups, fully unrolled: straight-line code
@@ -991,7 +979,7 @@ void launch_fmt(mdma_ctx *ctx, TeamSet ts, const float *xf, const int8_t *qx, co
   }
 }
 
-// One format and activation mode: the launch for 1..8 tokens.
+// One format and activation mode: the launch for 1..8 tokens (f32: one).
 template <class F, bool F32>
 void launch_mode(mdma_ctx *ctx, bool gated, const TeamSet &ts, const float *xf, const int8_t *qx, const float *dx,
                  const int32_t *s16, uint32_t T, float *yg) {
@@ -1003,10 +991,14 @@ void launch_mode(mdma_ctx *ctx, bool gated, const TeamSet &ts, const float *xf, 
     else                                                                      \
       launch_fmt<F, F32, RP, TT_, false>(ctx, ts, xf, qx, dx, s16, T, yg);   \
   } while (0)
-  if (T <= 1) MDMA_TEAM_T(1);
-  else if (T <= 2) MDMA_TEAM_T(2);
-  else if (T <= 4) MDMA_TEAM_T(4);
-  else MDMA_TEAM_T(8);
+  if constexpr (F32) {
+    MDMA_TEAM_T(1);
+  } else {
+    if (T <= 1) MDMA_TEAM_T(1);
+    else if (T <= 2) MDMA_TEAM_T(2);
+    else if (T <= 4) MDMA_TEAM_T(4);
+    else MDMA_TEAM_T(8);
+  }
 #undef MDMA_TEAM_T
 }
 

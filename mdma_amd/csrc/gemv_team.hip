@@ -123,8 +123,10 @@ void launch_gemv_team(mdma_ctx *ctx, int mode, const GemvJob *jobs, int n_jobs, 
   const bool f32 = mode != MDMA_ACT_I8;
   const int32_t dt = jobs[0].dtype;
   if (!f32 && !pro && !(nm && nm->nsum)) quantize_into_scratch(ctx, x, T, n_in, &qx, &dx, &s16);
-  for (uint64_t t0 = 0; t0 < T; t0 += 8) {
-    const uint32_t tn = (uint32_t)(T - t0 < 8 ? T - t0 : 8);
+  // (More than one f32 token only where gemm_f64.hip does not cover the call.)
+  const uint64_t step = f32 ? 1 : 8;
+  for (uint64_t t0 = 0; t0 < T; t0 += step) {
+    const uint32_t tn = (uint32_t)(T - t0 < step ? T - t0 : step);
     TeamSet ts{};
     ts.pro = pro;
     if (nm) {  // one token only (the callers check)

@@ -385,9 +385,10 @@ void launch_gemm_f16(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
 // tokens and up: up to 3 prepared jobs of one type sharing x, or (glu_y) gate
 // and up with silu(gate) * up written there. False, launching nothing, where
 // it does not cover the call (another layout, mixed types).
-// At 4 tokens and fewer the row teams are as fast (4096x14336 Q6_K at 3
-// tokens 52 us against 67; from 5 they take an 8-token launch: 130 us).
-constexpr uint64_t F64_MIN_TOKENS = 5;
+// One token: the row teams (us, teams / this kernel: gate/up 2x14336x4096
+// Q4_K 24.3 / 37.9, 4096x4096 Q6_K 6.5 / 9.5; at two tokens 73 / 38.7 and
+// 20.2 / 9.7).
+constexpr uint64_t F64_MIN_TOKENS = 2;
 bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T,
                      float *glu_y = nullptr);
 // Device space for its partial tiles, or null where it may not grow now (a
