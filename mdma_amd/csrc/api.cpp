@@ -315,24 +315,24 @@ void no_capture(mdma_ctx *ctx, const char *what) {
   if (ctx->fixed_scratch) fail(MDMA_ERR_BACKEND, std::string(what) + " would allocate inside an allocation-free call");
 }
 
-// Gives the f64 GEMM's partial tiles back (they only spread its work): a
+// Gives the split launches' partials back (they only spread work over the CUs): a
 // caller's allocation that the budget or the device has no room for comes
 // first. False when there is nothing to give or the stream cannot be drained
 // now.
-static bool drop_f64_parts(mdma_ctx *ctx) {
-  if (!ctx->f64_part || ctx->capturing || ctx->fixed_scratch) return false;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->f64_part) != hipSuccess) return false;
-  budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->f64_part_cap);
-  if (ctx->f64_part_captured) ctx->buf_epoch++;
-  ctx->f64_part = nullptr;
-  ctx->f64_part_cap = 0;
-  ctx->f64_part_captured = false;
+static bool drop_split_parts(mdma_ctx *ctx) {
+  if (!ctx->split_part || ctx->capturing || ctx->fixed_scratch) return false;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->split_part) != hipSuccess) return false;
+  budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_cap);
+  if (ctx->split_part_captured) ctx->buf_epoch++;
+  ctx->split_part = nullptr;
+  ctx->split_part_cap = 0;
+  ctx->split_part_captured = false;
   return true;
 }
 
 void budget_charge(mdma_ctx *ctx, int domain, uint64_t bytes, const char *what) {
   Ledger &l = ctx->budget[domain];
-  if (domain == MDMA_DOMAIN_DEVICE && l.used + bytes > l.limit) drop_f64_parts(ctx);
+  if (domain == MDMA_DOMAIN_DEVICE && l.used + bytes > l.limit) drop_split_parts(ctx);
   if (l.used + bytes < l.used || l.used + bytes > l.limit)
     fail(MDMA_ERR_BUFFER_BUDGET,
          fmt("%s: %s buffer budget exhausted: requested %llu bytes, used %llu, limit %llu", what,
@@ -400,24 +400,24 @@ char *argmax_parts(mdma_ctx *ctx, uint64_t chunks) {
   return regrow(ctx, ctx->argmax_part, ctx->argmax_part_cap, cap, 12, "argmax buffer growth");
 }
 
-void *f64_parts(mdma_ctx *ctx, uint64_t bytes) {
-  if (bytes > ctx->f64_part_cap) {
+void *split_parts(mdma_ctx *ctx, uint64_t bytes) {
+  if (bytes > ctx->split_part_cap) {
     if (ctx->capturing || ctx->fixed_scratch) return nullptr;
     // Graphs that do not hold it stay valid: the epoch moves only for those
     // that do.
     const uint64_t epoch = ctx->buf_epoch;
     try {
-      regrow(ctx, ctx->f64_part, ctx->f64_part_cap, bytes, 1, "f64 GEMM partials growth");
+      regrow(ctx, ctx->split_part, ctx->split_part_cap, bytes, 1, "split partials growth");
     } catch (const Error &) {
       (void)hipGetLastError();
-      if (!ctx->f64_part_captured) ctx->buf_epoch = epoch;
-      if (bytes > ctx->f64_part_cap) return nullptr;
+      if (!ctx->split_part_captured) ctx->buf_epoch = epoch;
+      if (bytes > ctx->split_part_cap) return nullptr;
     }
-    if (!ctx->f64_part_captured) ctx->buf_epoch = epoch;
-    ctx->f64_part_captured = false;
+    if (!ctx->split_part_captured) ctx->buf_epoch = epoch;
+    ctx->split_part_captured = false;
   }
-  if (ctx->capturing) ctx->f64_part_captured = true;
-  return ctx->f64_part;
+  if (ctx->capturing) ctx->split_part_captured = true;
+  return ctx->split_part;
 }
 
 double *ssq_parts(mdma_ctx *ctx, uint64_t n) {
@@ -542,7 +542,7 @@ void mdma_gfx950_destroy(mdma_ctx *ctx) {
   if (ctx->attn_cnt) (void)hipFree(ctx->attn_cnt);
   if (ctx->gemm_cnt) (void)hipFree(ctx->gemm_cnt);
   if (ctx->ssq) (void)hipFree(ctx->ssq);
-  if (ctx->f64_part) (void)hipFree(ctx->f64_part);
+  if (ctx->split_part) (void)hipFree(ctx->split_part);
   if (ctx->rope_tab) (void)hipFree(ctx->rope_tab);
   if (ctx->host_ids) (void)hipHostFree(ctx->host_ids);
   (void)hipStreamDestroy(ctx->stream);
@@ -693,7 +693,7 @@ int mdma_gfx950_alloc(mdma_ctx *ctx, uint64_t bytes, int pool, mdma_buf **out) {
     void *d = nullptr;
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = hipMalloc(&d, rounded);
-    if (e == hipErrorOutOfMemory && drop_f64_parts(ctx)) e = hipMalloc(&d, rounded);
+    if (e == hipErrorOutOfMemory && drop_split_parts(ctx)) e = hipMalloc(&d, rounded);
     if (e != hipSuccess) {
       budget_refund(ctx, MDMA_DOMAIN_DEVICE, charged);
       hip_check(e, "hipMalloc");

@@ -335,7 +335,7 @@ void launch(mdma_ctx *ctx, F64Args &a, uint32_t tiles, float *yg) {
   uint32_t G = (uint32_t)ctx->cu_count * (TW <= 2 ? 2 : 1);
   if (G > units) G = units;
   a.units = units;
-  a.part = tiles % G ? static_cast<double *>(f64_parts(ctx, (uint64_t)G * 2 * RW * TW * 4 * 256 * 8)) : nullptr;
+  a.part = tiles % G ? static_cast<double *>(split_parts(ctx, (uint64_t)G * 2 * RW * TW * 4 * 256 * 8)) : nullptr;
   if (a.part) {
     a.per_q = units / G, a.per_r = units % G;
   } else {  // runs of whole tiles

@@ -987,6 +987,7 @@ void launch_gemv_i8(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float 
     // One token: quantized in the GEMV's own prologue (one launch).
     if (launch_gemv_i8_x(ctx, jobs, n_jobs, false, x, nullptr)) return;
   }
+  if (launch_gemv_wide(ctx, jobs, n_jobs, false, x, T, nullptr)) return;
   if (T >= BATCH_MIN_TOKENS && gemv_batch_ok(jobs, n_jobs, 16)) {
     // Up to 16 tokens per matrix-core launch (a short remainder: row teams).
     for (uint64_t t0 = 0; t0 < T; t0 += 16) {
@@ -1033,6 +1034,7 @@ void launch_gemv_i8_gated(mdma_ctx *ctx, const GemvJob &gate, const GemvJob &up,
   if (T == 1 && !q8_holds(ctx, x, gate.n_in)) {
     if (launch_gemv_i8_x(ctx, gu, 2, true, x, y)) return;
   }
+  if (launch_gemv_wide(ctx, gu, 2, true, x, T, y)) return;
   if (T >= BATCH_MIN_TOKENS && gemv_batch_ok(gu, 2, 16)) {
     for (uint64_t t0 = 0; t0 < T; t0 += 16) {
       const uint64_t tn = T - t0 < 16 ? T - t0 : 16;

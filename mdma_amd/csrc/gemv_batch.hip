@@ -36,6 +36,8 @@
 //    continue the same 128-byte lines.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace mdma {
@@ -1219,6 +1221,490 @@ __global__ __launch_bounds__(256) void tile_repack_q6_kernel(const uint8_t *__re
   *reinterpret_cast<uint4 *>(out + 16 * idx) = v;
 }
 
+// ---------------------------------------------------------------------------
+// 17 to 63 tokens: one launch instead of one ring launch per 16 tokens, so
+// the weights are read and unpacked once. The same products, scalings and
+// summation order as above (the results are the same bits as 16-token
+// launches).
+//
+// A workgroup is 4 waves of 16 rows each (gated: two of gate, two of the
+// same rows of up) over NT tiles of 16 tokens. The weights go from HBM to
+// registers, four lanes per row reading 64 contiguous bytes of a plane, and
+// through the wave's own LDS into the MFMA operand layout (loaded in that
+// layout, 8 bytes per lane and a row per neighbouring lane, every lane is a
+// request of its own: gate/up at 43 tokens 43 us against 38.5). x and its
+// scales come by DMA into LDS once per workgroup and block, the 16-byte
+// chunk k of token t at position k ^ (t % 16) of its 256 bytes (16 tokens
+// reading one 32-column group hit distinct banks).
+//
+// Launches of no more tiles than CUs split the fixed column chunks over
+// workgroups: each leaves its chunks' sums, and a second kernel adds them in
+// chunk order. What bounds it is instruction issue at two waves per SIMD (one
+// integer multiply-add per result and scale group, and the unpacking). us at
+// 43 tokens, 16-token launches / here: gate/up 2x14336x4096 Q4_K 56.9 / 35.6,
+// 4096x14336 Q6_K 55.1 / 32.2, 4096x4096 Q6_K 28.0 / 17.6; at 17: 34.4 / 27.9,
+// 32.6 / 27.3, 17.3 / 15.4.
+
+// A lane's operands of one block of its row, and the block's contributions
+// c[t][j] (before the activation scale) for token tiles t.
+// c + a * b (24-bit, full rate), formed here: left to itself the compiler
+// regroups the integer sums so that every group's products live to the end
+// (256 VGPRs and spills at 48 tokens) and takes three instructions for two.
+__device__ __forceinline__ int mad24(int a, int b, int c) {
+  int r = __mul24(a, b) + c;
+  asm("" : "+v"(r));
+  return r;
+}
+struct WQ4 {
+  using F = BQ4;
+  uint64_t q[4];
+  uint4 h;
+  struct Raw {
+    uint4 a, b;
+    uint32_t h;
+    __device__ void load(const uint8_t *row, uint32_t n_in, uint32_t blk, uint32_t l) {
+      const uint32_t U = n_in / 64;
+      const size_t o = 64 * (size_t)blk + 16 * (l & 3);
+      a = ldx16(row + o);
+      b = ldx16(row + 16 * (size_t)U + o);
+      h = ldw4(row + 32 * (size_t)U + 16 * (size_t)blk + 4 * (l & 3));
+    }
+    __device__ void store(uint8_t *lds, uint32_t l) const {
+      uint8_t *p = lds + (l >> 2) * F::RS + 32 * (l & 3);
+      *reinterpret_cast<uint4 *>(p) = a;
+      *reinterpret_cast<uint4 *>(p + 16) = b;
+      *reinterpret_cast<uint32_t *>(lds + 16 * F::RS + 4 * l) = h;
+    }
+  };
+  __device__ void read(const uint8_t *lds, uint32_t n, uint32_t g, uint32_t) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = *reinterpret_cast<const uint64_t *>(lds + n * F::RS + 32 * i + 8 * g);
+    h = *reinterpret_cast<const uint4 *>(lds + 16 * F::RS + 16 * n);
+  }
+  template <int NT, class X>
+  __device__ void compute(const X &xg, float (&c)[NT][4], const Dots &dc, uint32_t g) const {
+    constexpr uint64_t M4 = 0x0F0F0F0F0F0F0F0Full;
+    int ai[NT][4] = {};
+    v4i dm[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) dm[t] = v4i{};
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+      int sca, scb, ma, mb;
+      q4k_scales_i(h, p, sca, scb, ma, mb);
+      const uint64_t wa = q[p] & M4, wb = (q[p] >> 4) & M4, ba = bytes8(ma), bb = bytes8(mb);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const uint64_t xlo = xg(t, 2 * p), xhi = xg(t, 2 * p + 1);
+        const v4i z = {};
+        const v4i da = mma(xlo, wa, z), db = mma(xhi, wb, z);
+        if (dc.p)
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+            dc.put(16 * t + 4 * g + j, 2 * p, da[j]), dc.put(16 * t + 4 * g + j, 2 * p + 1, db[j]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          ai[t][j] = mad24(sca, da[j], ai[t][j]);
+          ai[t][j] = mad24(scb, db[j], ai[t][j]);
+        }
+        dm[t] = mma(xlo, ba, dm[t]);
+        dm[t] = mma(xhi, bb, dm[t]);
+      }
+    }
+    const float d = h2f(h.x), dmin = h2f(h.x >> 16);
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) c[t][j] = d * (float)ai[t][j] - dmin * (float)dm[t][j];
+  }
+};
+
+// The other k-group pair's weights are zeroed (once for all token tiles)
+// where compute() zeroes its activations.
+struct WQ6 {
+  using F = BQ6;
+  uint64_t q[2][3];
+  uint4 s;
+  uint32_t dw, dsh;
+  struct Raw {
+    uint4 p[3];
+    uint32_t s, d;
+    __device__ void load(const uint8_t *row, uint32_t n_in, uint32_t blk, uint32_t l) {
+      const uint32_t U = n_in / 64;
+#pragma unroll
+      for (int k = 0; k < 3; k++) p[k] = ldx16(row + 16 * (size_t)U * k + 64 * (size_t)blk + 16 * (l & 3));
+      s = ldw4(row + 48 * (size_t)U + 16 * (size_t)blk + 4 * (l & 3));
+      // (A whole word, its half taken at use; the row's padding covers it.)
+      d = ldw4(row + 52 * (size_t)U + 4 * (size_t)(blk >> 1));
+    }
+    __device__ void store(uint8_t *lds, uint32_t l) const {
+#pragma unroll
+      for (int k = 0; k < 3; k++) *reinterpret_cast<uint4 *>(lds + (l >> 2) * F::RS + 48 * (l & 3) + 16 * k) = p[k];
+      *reinterpret_cast<uint32_t *>(lds + 16 * F::RS + 4 * l) = s;
+      *reinterpret_cast<uint32_t *>(lds + 16 * F::RS + 256 + 4 * (l >> 2)) = d;  // (a row's four lanes: the same word)
+    }
+  };
+  __device__ void read(const uint8_t *lds, uint32_t n, uint32_t g, uint32_t blk) {
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+        q[v][k] = *reinterpret_cast<const uint64_t *>(lds + n * F::RS + 48 * (2 * v + (g >> 1)) + 8 * (g & 1) + 16 * k);
+    s = *reinterpret_cast<const uint4 *>(lds + 16 * F::RS + 16 * n);
+    dw = *reinterpret_cast<const uint32_t *>(lds + 16 * F::RS + 256 + 4 * n);
+    dsh = 16 * (blk & 1);
+  }
+  template <int NT, class X>
+  __device__ void compute(const X &xg, float (&c)[NT][4], const Dots &dc, uint32_t g) const {
+    const uint32_t scw[4] = {s.x, s.y, s.z, s.w};
+    const uint64_t m0 = g < 2 ? ~0ull : 0ull;
+    int ai[NT][4] = {};
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const uint32_t lo = q6_centre4(F::u6((uint32_t)q[v][0], (uint32_t)q[v][1], (uint32_t)q[v][2], r));
+        const uint32_t hi = q6_centre4(
+            F::u6((uint32_t)(q[v][0] >> 32), (uint32_t)(q[v][1] >> 32), (uint32_t)(q[v][2] >> 32), r));
+        const uint64_t wv = (uint64_t)lo | ((uint64_t)hi << 32), w0 = wv & m0, w1 = wv & ~m0;
+        const int s0 = (int)(int8_t)((scw[2 * v] >> (8 * r)) & 0xff);
+        const int s1 = (int)(int8_t)((scw[2 * v + 1] >> (8 * r)) & 0xff);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          const uint64_t xq = xg(t, 4 * v + r);
+          const v4i z = {};
+          const v4i d0 = mma(xq, w0, z), d1 = mma(xq, w1, z);
+          if (dc.p)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              dc.put(16 * t + 4 * g + j, 8 * v + 2 * r, d0[j]), dc.put(16 * t + 4 * g + j, 8 * v + 2 * r + 1, d1[j]);
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            ai[t][j] = mad24(s0, d0[j], ai[t][j]);
+            ai[t][j] = mad24(s1, d1[j], ai[t][j]);
+          }
+        }
+      }
+    const float d = h2f(dw >> dsh);
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) c[t][j] = d * (float)ai[t][j];
+  }
+};
+
+struct WQ8 {
+  using F = BQ8;
+  uint64_t q[8];
+  uint4 s;
+  struct Raw {
+    uint4 a[2], b[2];
+    uint32_t d;
+    __device__ void load(const uint8_t *row, uint32_t n_in, uint32_t blk, uint32_t l) {
+      const uint32_t U = n_in / 32;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const size_t o = 128 * (size_t)blk + 16 * (l & 3) + 64 * i;
+        a[i] = ldx16(row + o);
+        b[i] = ldx16(row + 16 * (size_t)U + o);
+      }
+      d = ldw4(row + 32 * (size_t)U + 16 * (size_t)blk + 4 * (l & 3));
+    }
+    __device__ void store(uint8_t *lds, uint32_t l) const {
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        uint8_t *p = lds + (l >> 2) * F::RS + 32 * ((l & 3) + 4 * i);
+        *reinterpret_cast<uint4 *>(p) = a[i];
+        *reinterpret_cast<uint4 *>(p + 16) = b[i];
+      }
+      *reinterpret_cast<uint32_t *>(lds + 16 * F::RS + 4 * l) = d;
+    }
+  };
+  __device__ void read(const uint8_t *lds, uint32_t n, uint32_t g, uint32_t) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) q[i] = *reinterpret_cast<const uint64_t *>(lds + n * F::RS + 32 * i + 8 * g);
+    s = *reinterpret_cast<const uint4 *>(lds + 16 * F::RS + 16 * n);
+  }
+  template <int NT, class X>
+  __device__ void compute(const X &xg, float (&c)[NT][4], const Dots &dc, uint32_t g) const {
+    const uint32_t dw[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) c[t][j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float d = h2f(dw[i >> 1] >> (16 * (i & 1)));
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const v4i z = {};
+        const v4i dq = mma(xg(t, i), q[i], z);
+        if (dc.p)
+#pragma unroll
+          for (int j = 0; j < 4; j++) dc.put(16 * t + 4 * g + j, i, dq[j]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[t][j] = fmaf(d, (float)dq[j], c[t][j]);
+      }
+    }
+  }
+};
+
+struct WideSet {
+  BatchSet s;           // tiles: a job's tiles of 64 rows (gated: 32)
+  uint32_t T, nch;
+  uint32_t per_q, per_r, items;  // run of workgroup w: chunk items [w per_q + min(w, per_r), ...)
+  float *part;          // [tile][chunk][NT * 4][256] chunk sums of the tiles that runs share
+  float *yg;
+};
+__device__ __forceinline__ uint32_t wide_start(const WideSet &ws, uint32_t w) {
+  return min(w * ws.per_q + min(w, ws.per_r), ws.items);
+}
+// The tile's job, and its first row.
+template <bool GLU>
+__device__ __forceinline__ uint32_t wide_place(const WideSet &ws, uint32_t tile, int &ji) {
+  ji = 0;
+  if (!GLU && ws.s.n > 1 && tile >= ws.s.j[0].tiles) {
+    tile -= ws.s.j[0].tiles;
+    ji = 1;
+    if (ws.s.n > 2 && tile >= ws.s.j[1].tiles) {
+      tile -= ws.s.j[1].tiles;
+      ji = 2;
+    }
+  }
+  return tile * (GLU ? 32 : 64);
+}
+
+template <class W, int NT, bool GLU, bool CAP>
+__global__ __launch_bounds__(256, 2) void gemv_wide(WideSet ws, const int8_t *__restrict__ qx,
+                                                    const float *__restrict__ dx) {
+  using F = typename W::F;
+  constexpr uint32_t XB = NT * 16 * 256;
+  __shared__ __attribute__((aligned(1024))) uint8_t xs[3][XB + 256];
+  __shared__ __attribute__((aligned(16))) uint8_t wl[4][F::LDS];  // a wave's weights of one block
+  __shared__ float xch[GLU ? 2 : 1][GLU ? NT * 4 : 1][64];  // up's sums for gate's waves
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n = lane & 15, g = lane >> 4;
+  const uint32_t n_in = ws.s.n_in, nb = n_in / 256, nch = ws.nch, T = ws.T;
+  const size_t rb = F::row_bytes(n_in);
+  const uint32_t i0 = wide_start(ws, blockIdx.x), i1 = wide_start(ws, blockIdx.x + 1);
+  if (i0 >= i1) return;
+  auto chunk_start = [&](uint32_t c) { return c * nb / nch; };
+  auto block_of = [&](uint32_t i) { return i / nch * nb + chunk_start(i % nch); };
+  uint32_t u = block_of(i0);
+  const uint32_t u_end = block_of(i1);
+  // x by DMA: 4 tokens' 256 bytes per instruction, the wave's share of them,
+  // and (wave 0) the tokens' scales.
+  uint32_t xsrc[NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) {
+    const uint32_t t = 4 * (NT * wave + k) + lane / 16;
+    xsrc[k] = min(t, T - 1) * n_in + 16 * ((lane & 15) ^ (t & 15));
+  }
+  const uint32_t ssrc = min(lane, T - 1) * nb * 4;
+  // Two blocks' loads are in flight behind the current block's products. A
+  // block's x DMAs go out before its weights' loads, and loads complete in
+  // order: once the wave holds the block's weights, its part of x is in LDS.
+  typename W::Raw raw[2];
+  uint32_t iu = u, it = u / nb;  // the next block to load, and its tile
+  const uint8_t *wr = nullptr;   // the row of the lane's loads there: l / 4 of the wave's 16
+  auto row_of = [&](uint32_t t, uint32_t r, const uint8_t *&w, uint32_t &n_out) {
+    int j;
+    const uint32_t row0 = wide_place<GLU>(ws, t, j);
+    if (GLU) j = (int)(wave >> 1);
+    n_out = j == 0 ? ws.s.j[0].n_out : j == 1 ? ws.s.j[1].n_out : ws.s.j[2].n_out;
+    w = j == 0 ? ws.s.j[0].w : j == 1 ? ws.s.j[1].w : ws.s.j[2].w;
+    return row0 + 16 * (GLU ? wave & 1 : wave) + r;
+  };
+  auto enter = [&]() {
+    const uint8_t *w;
+    uint32_t no;
+    const uint32_t r = row_of(it, lane / 4, w, no);
+    wr = w + (size_t)min(r, no - 1) * rb;
+  };
+  auto issue = [&](typename W::Raw &r, uint32_t buf) {
+    if (iu >= u_end) return;
+    const uint32_t b = iu - it * nb;
+#pragma unroll
+    for (int k = 0; k < NT; k++) lds_dma16(qx, xsrc[k] + 256 * b, &xs[buf][1024 * (NT * wave + k)]);
+    if (wave == 0) lds_dma4(dx, ssrc + 4 * b, &xs[buf][XB]);
+    r.load(wr, n_in, b, lane);
+    if (++iu == (it + 1) * nb && iu < u_end) it++, enter();
+  };
+  const uint32_t xo = 256 * n + 16 * ((g >> 1) ^ n) + 8 * (g & 1);
+  enter();
+  issue(raw[0], 0);
+  issue(raw[1], 1);
+  uint32_t tile = i0 / nch, b = u - tile * nb, ch = i0 % nch, buf = 0;
+  const uint8_t *w_;
+  uint32_t n_out, r_lane = row_of(tile, n, w_, n_out);
+  float acc[NT][4], tot[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[t][j] = tot[t][j] = 0.f;
+  uint32_t ch_end = chunk_start(ch + 1);
+  // The tile's chunks are all this run's: no partials.
+  bool whole = ch == 0 && u + nb <= u_end;
+  auto block = [&](typename W::Raw &r) {
+    W cur;
+    r.store(wl[wave], lane);  // (the wave's own LDS, in order)
+    cur.read(wl[wave], n, g, b);
+    lds_barrier();  // every wave's part of the block's x is in LDS; the buffer refilled now is read
+    issue(r, buf == 0 ? 2 : buf - 1);
+    const uint8_t *xb = xs[buf];
+    buf = buf == 2 ? 0 : buf + 1;
+    float c[NT][4];
+    Dots dc{nullptr, 0, T};
+    if constexpr (CAP) {
+      int jw;
+      wide_place<GLU>(ws, tile, jw);
+      if (GLU) jw = (int)(wave >> 1);
+      const uint32_t nsub = n_in / (256 / F::SUBS);
+      int32_t *dp = jw == 0 ? ws.s.j[0].dots : jw == 1 ? ws.s.j[1].dots : ws.s.j[2].dots;
+      dc.stride = (size_t)n_out * nsub;
+      if (r_lane < n_out) dc.p = dp + (size_t)r_lane * nsub + F::SUBS * b;
+    }
+    cur.template compute<NT>(
+        [&](int t, int j) { return *reinterpret_cast<const uint64_t *>(xb + 4096 * t + (xo ^ (32 * j))); }, c, dc, g);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const float4 sv = *reinterpret_cast<const float4 *>(xb + XB + 64 * t + 16 * g);
+      const float sj[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[t][j] = fmaf(sj[j], c[t][j], acc[t][j]);
+    }
+    if (++b != ch_end) return;
+    // Chunk ch is done.
+    if (whole) {
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) tot[t][j] += acc[t][j];
+    } else {
+      float *o = ws.part + ((size_t)tile * nch + ch) * (NT * 4 * 256) + threadIdx.x;
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[(4 * t + j) * 256] = acc[t][j];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[t][j] = 0.f;
+    if (++ch < nch) {
+      ch_end = chunk_start(ch + 1);
+      return;
+    }
+    // The tile is done.
+    if (whole) {
+      if constexpr (GLU) {
+        lds_barrier();  // the previous tile's exchange is read
+        if (wave >= 2)
+#pragma unroll
+          for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) xch[wave & 1][4 * t + j][lane] = tot[t][j];
+        lds_barrier();
+      }
+      int ji;
+      wide_place<GLU>(ws, tile, ji);
+      float *y = GLU ? ws.yg : ji == 0 ? ws.s.j[0].y : ji == 1 ? ws.s.j[1].y : ws.s.j[2].y;
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const uint32_t tok = 16 * t + 4 * g + j;
+          if (tok < T && r_lane < n_out && (!GLU || wave < 2)) {
+            float v = tot[t][j];
+            if constexpr (GLU) {
+              const float uv = xch[wave & 1][4 * t + j][lane];
+              v = v / (1.0f + expf(-v)) * uv;
+            }
+            y[(size_t)tok * n_out + r_lane] = v;
+          }
+          tot[t][j] = 0.f;
+        }
+    }
+    ch = b = 0;
+    ch_end = chunk_start(1);
+    tile++;
+    if (tile * nb < u_end) {
+      r_lane = row_of(tile, n, w_, n_out);
+      whole = (tile + 1) * nb <= u_end;
+    }
+  };
+  for (; u < u_end; u += 2) {
+    block(raw[0]);
+    if (u + 1 < u_end) block(raw[1]);
+  }
+}
+
+// The tiles that several runs share: their chunk sums added in chunk order.
+template <int NT, bool GLU>
+__global__ __launch_bounds__(256) void gemv_wide_merge(WideSet ws) {
+  const uint32_t tile = blockIdx.x, nch = ws.nch;
+  // The tile is one run's own if no run starts inside it.
+  const uint32_t a = tile * nch, e = a + nch, big = ws.per_r * (ws.per_q + 1);
+  auto run_of = [&](uint32_t i) { return i < big ? i / (ws.per_q + 1) : ws.per_r + (i - big) / ws.per_q; };
+  if (run_of(a) == run_of(e - 1)) return;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+  if (GLU && wave >= 2) return;
+  int ji;
+  const uint32_t row0 = wide_place<GLU>(ws, tile, ji);
+  const uint32_t r = row0 + 16 * wave + n;
+  const uint32_t n_out = ji == 0 ? ws.s.j[0].n_out : ji == 1 ? ws.s.j[1].n_out : ws.s.j[2].n_out;
+  float *y = GLU ? ws.yg : ji == 0 ? ws.s.j[0].y : ji == 1 ? ws.s.j[1].y : ws.s.j[2].y;
+  const uint32_t q = blockIdx.y, tok = 16 * (q >> 2) + 4 * g + (q & 3);  // one result of every thread
+  const float *p = ws.part + ((size_t)tile * nch * (NT * 4) + q) * 256 + threadIdx.x;
+  float cv[NCHMAX], cu[NCHMAX];
+#pragma unroll
+  for (uint32_t k = 0; k < NCHMAX; k++) {  // (past the last chunk: read again, not added)
+    cv[k] = p[(size_t)min(k, nch - 1) * (NT * 4 * 256)];
+    cu[k] = GLU ? p[(size_t)min(k, nch - 1) * (NT * 4 * 256) + 128] : 0.f;
+  }
+  float v = 0.f, uv = 0.f;
+#pragma unroll
+  for (uint32_t k = 0; k < NCHMAX; k++) {
+    if (k >= nch) break;
+    v += cv[k];
+    if (GLU) uv += cu[k];
+  }
+  if (tok >= ws.T || r >= n_out) return;
+  if constexpr (GLU) v = v / (1.0f + expf(-v)) * uv;
+  y[(size_t)tok * n_out + r] = v;
+}
+
+template <class W, int NT, bool GLU>
+void wide_launch(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, const float *dx) {
+  // Enough tiles for every CU: whole tiles, handed out as workgroups end.
+  // Fewer: two workgroups per CU share the chunks.
+  uint32_t G = tiles;
+  ws.items = tiles * ws.nch;
+  ws.per_q = ws.nch, ws.per_r = 0;
+  if (tiles <= (uint32_t)ctx->cu_count) {
+    const uint32_t g2 = std::min(ws.items, 2 * (uint32_t)ctx->cu_count);
+    ws.part = static_cast<float *>(split_parts(ctx, (uint64_t)ws.items * NT * 4 * 256 * 4));
+    if (ws.part && g2 > tiles) G = g2, ws.per_q = ws.items / G, ws.per_r = ws.items % G;
+  }
+  if (ws.s.j[0].dots)
+    gemv_wide<W, NT, GLU, true><<<dim3(G), dim3(256), 0, ctx->stream>>>(ws, qx, dx);
+  else
+    gemv_wide<W, NT, GLU, false><<<dim3(G), dim3(256), 0, ctx->stream>>>(ws, qx, dx);
+  hip_check(hipGetLastError(), "gemv wide launch");
+  if (G > tiles) {
+    gemv_wide_merge<NT, GLU><<<dim3(tiles, NT * 4), dim3(256), 0, ctx->stream>>>(ws);
+    hip_check(hipGetLastError(), "gemv wide merge launch");
+  }
+}
+
+template <class W, bool GLU>
+void wide_fmt(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, const float *dx) {
+  if (ws.T <= 16) wide_launch<W, 1, GLU>(ctx, ws, tiles, qx, dx);
+  else if (ws.T <= 32) wide_launch<W, 2, GLU>(ctx, ws, tiles, qx, dx);
+  else if (ws.T <= 48) wide_launch<W, 3, GLU>(ctx, ws, tiles, qx, dx);
+  else wide_launch<W, 4, GLU>(ctx, ws, tiles, qx, dx);
+}
+
 }  // namespace
 
 uint64_t batch_tile_bytes(int32_t dtype, uint64_t n_out, uint64_t n_in) {
@@ -1250,6 +1736,44 @@ bool gemv_batch_ok(const GemvJob *jobs, int n_jobs, uint64_t T) {
     if (j.dtype != DT_Q4_K && j.dtype != DT_Q6_K && j.dtype != DT_Q8_0) return false;
   }
   return jobs[0].n_in % 256 == 0 && jobs[0].n_in > 0;
+}
+
+bool launch_gemv_wide(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated, const float *x, uint64_t T,
+                      float *ygated) {
+  if (ctx->batch_kernel != MDMA_BATCH_AUTO || T < WIDE_MIN_TOKENS || T > 64 || !gemv_batch_ok(jobs, n_jobs, 16)) return false;
+  const uint64_t n_in = jobs[0].n_in;
+  if (n_in > 1u << 20) return false;
+  WideSet ws{};
+  ws.s.n = gated ? 1 : n_jobs;
+  ws.s.n_in = (uint32_t)n_in;
+  const uint32_t nb = ws.s.n_in / 256;
+  ws.nch = nb < NCHMAX ? nb : NCHMAX;
+  ws.T = (uint32_t)T;
+  ws.yg = ygated;
+  uint64_t tiles = 0;
+  for (int i = 0; i < (gated ? 2 : n_jobs); i++) {
+    if (!jobs[i].n_out || jobs[i].n_out > 1u << 24 || (gated && jobs[i].n_out != jobs[0].n_out)) return false;
+    BatchJob &j = ws.s.j[i];
+    j.w = jobs[i].w;
+    j.y = jobs[i].y;
+    j.dots = jobs[i].dots;
+    j.n_out = (uint32_t)jobs[i].n_out;
+    j.tiles = (j.n_out + (gated ? 31 : 63)) / (gated ? 32 : 64);
+    if (i < ws.s.n) tiles += j.tiles;
+  }
+  int8_t *qx;
+  float *dx;
+  int32_t *s16;
+  quantize_into_scratch(ctx, x, T, n_in, &qx, &dx, &s16);
+  const uint32_t nt = (uint32_t)tiles;
+#define MDMA_WIDE_GO(W)                                  \
+  if (gated) wide_fmt<W, true>(ctx, ws, nt, qx, dx);     \
+  else wide_fmt<W, false>(ctx, ws, nt, qx, dx)
+  if (jobs[0].dtype == DT_Q4_K) { MDMA_WIDE_GO(WQ4); }
+  else if (jobs[0].dtype == DT_Q6_K) { MDMA_WIDE_GO(WQ6); }
+  else { MDMA_WIDE_GO(WQ8); }
+#undef MDMA_WIDE_GO
+  return true;
 }
 
 void launch_gemv_batch(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated, const float *x, uint64_t T,

@@ -142,9 +142,9 @@ struct mdma_ctx {
   uint64_t attn_cnt_cap = 0;
   uint32_t *gemm_cnt = nullptr;  // split-K GEMM arrival counters (zero between launches)
   uint64_t gemm_cnt_cap = 0;
-  char *f64_part = nullptr;  // partial tiles of the f64 GEMM
-  uint64_t f64_part_cap = 0;
-  bool f64_part_captured = false;  // a captured launch points into it
+  char *split_part = nullptr;  // partial sums of launches that split K (gemm_f64.hip, gemv_wide)
+  uint64_t split_part_cap = 0;
+  bool split_part_captured = false;  // a captured launch points into it
   double *ssq = nullptr;  // per-workgroup sums of squares of a residual-stream GEMV (norm fusion)
   uint64_t ssq_cap = 0;
   uint32_t team_grid = 0;  // workgroups of the last row-team launch
@@ -280,6 +280,11 @@ void launch_gemv_batch(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gate
                        float *ygated);
 // Tokens from which int8-mode GEMVs of prepared rows go to the batch kernel.
 constexpr uint64_t BATCH_MIN_TOKENS = 3;
+// 17 to 63 tokens in one launch (gemv_batch.hip), the same bits as 16-token
+// launches; false, launching nothing, where it does not cover the call.
+constexpr uint64_t WIDE_MIN_TOKENS = 17;
+bool launch_gemv_wide(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated, const float *x, uint64_t T,
+                      float *ygated);
 // The batch kernel's tile images of a prepared weight (Q6_K, rows of whole
 // 512-column pairs; 0 bytes otherwise), the kernel that writes them, and
 // the job's images (made now when the context's batch layout is on and the
@@ -391,10 +396,10 @@ void launch_gemm_f16(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
 constexpr uint64_t F64_MIN_TOKENS = 2;
 bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T,
                      float *glu_y = nullptr);
-// Device space for its partial tiles, or null where it may not grow now (a
+// Device space for the partial sums of a launch that splits K, or null where it may not grow now (a
 // capture, an allocation-free call, a full budget or device): the launch then
 // runs unsplit.
-void *f64_parts(mdma_ctx *ctx, uint64_t bytes);
+void *split_parts(mdma_ctx *ctx, uint64_t bytes);
 void launch_quantize_act(mdma_ctx *ctx, const float *x, uint64_t n, uint64_t group, int8_t *q,
                          float *d, int32_t *sum16);
 void launch_block_dot(mdma_ctx *ctx, const GemvJob &w, const int8_t *qx, uint64_t T, int32_t *out);
