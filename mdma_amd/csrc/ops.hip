@@ -5,6 +5,7 @@
 // (/root/reference/src/backend/cpu.rs) op for op; these are simple, correct
 // kernels, not the hot path.
 #include <algorithm>
+#include <cmath>
 
 #include "internal.h"
 #include "kernels.h"
@@ -455,12 +456,20 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 //     q is split exactly into three f16 parts (hi = f16(q), mid = f16(q -
 //     hi), lo = q - hi - mid: 11 + 11 + 2 of its 24 bits), three MFMAs of
 //     exact products added in f32, as the f32 kernels' dot products are;
-//   an online softmax per row: the row's 64 scores sit on the 16 lanes of
-//     one DPP row (4 per lane, one per 16-key block), max and sum by DPP;
-//   O += P V on the same MFMA, P (f32, through a per-wave LDS tile of rows x
-//     keys) split into f16 hi and lo as it is read; V goes to LDS
-//     transposed (dims x keys), so an operand's 8 keys are one 16-byte read.
-// s = (q.k) * scale and p = expf(s - m) in f32, the output O / l.
+//   the MFMAs form S^T (keys x queries), so a lane holds 16 scores of one
+//     query: the online softmax is in registers, its maximum two lane
+//     swaps, and the exponentials are already the B operand of
+//   O^T += V^T P^T on the same MFMA (the k order is any order of the keys,
+//     taken as S^T left them), P split into f16 hi and lo in place; V goes
+//     to LDS transposed (dims x keys).
+// p = exp2((s - m) * scale * log2 e), the constant in two parts so that the
+// product is rounded once; m is the largest score seen to within 2^8 (the
+// sums are rescaled only when a tile passes it by more: p <= 256), l the
+// sum, the output O / l. Only tiles past a wave's first query mask.
+// What bounds it is issue: 80 MFMAs a tile and wave (16 cycles each) beside
+// about 250 VALU instructions, two waves per SIMD. 1500 queries over 2500
+// keys, 32 heads of 128: 142 us; with P through LDS, expf and a mask per score
+// (600 VALU instructions) it was 252.
 // Key chunks (ct > 0): a query block's tiles are split into chunks of ct
 // tiles, one workgroup each (blockIdx.z), so the long blocks at the end of
 // a causal prompt no longer set the launch's length alone and more
@@ -478,36 +487,32 @@ constexpr uint32_t ATT_PREFILL_MIN = 64;
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_row_op_max(float v) {
-  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, -INFINITY),
-                                                                         __builtin_bit_cast(int, v), CTRL, 0xF, 0xF,
-                                                                         false)));
+typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Max / sum over the lanes l, l ^ 16, l ^ 32, l ^ 48, in every one of them.
+__device__ __forceinline__ float quarter_max(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float w = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+  const uint32_t x = __builtin_bit_cast(uint32_t, w);
+  const auto c = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)c[0]), __builtin_bit_cast(float, (uint32_t)c[1]));
 }
-template <int CTRL>
-__device__ __forceinline__ float dpp_row_op_sum(float v) {
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF,
-                                                                    false));
-}
-// Max / sum over the 16 lanes of this lane's DPP row, in every lane of it.
-__device__ __forceinline__ float row16_max(float v) {
-  v = dpp_row_op_max<0xB1>(v);
-  v = dpp_row_op_max<0x4E>(v);
-  v = dpp_row_op_max<0x141>(v);
-  return dpp_row_op_max<0x140>(v);
-}
-__device__ __forceinline__ float row16_sum(float v) {
-  v = dpp_row_op_sum<0xB1>(v);
-  v = dpp_row_op_sum<0x4E>(v);
-  v = dpp_row_op_sum<0x141>(v);
-  return dpp_row_op_sum<0x140>(v);
+__device__ __forceinline__ float quarter_sum(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const float w = __builtin_bit_cast(float, (uint32_t)a[0]) + __builtin_bit_cast(float, (uint32_t)a[1]);
+  const uint32_t x = __builtin_bit_cast(uint32_t, w);
+  const auto c = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return __builtin_bit_cast(float, (uint32_t)c[0]) + __builtin_bit_cast(float, (uint32_t)c[1]);
 }
 
 template <int G, int HD>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restrict__ q, const uint16_t *__restrict__ K,
                                                            const uint16_t *__restrict__ V, float *__restrict__ o,
                                                            uint32_t n_q, uint32_t prefix, uint32_t n_q_heads,
-                                                           uint32_t n_kv_heads, float scale, uint32_t ct,
+                                                           uint32_t n_kv_heads, float c_hi, float c_lo, uint32_t ct,
                                                            float *__restrict__ part, uint32_t *__restrict__ cnt,
                                                            F16In in) {
   constexpr int QT = 64 / G;             // queries per workgroup
@@ -516,11 +521,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   constexpr int KCH = HD / 8;            // 16-byte chunks of a key row
   constexpr int LPT = 64 * KCH / 256;    // chunks of K (and of V) per thread per tile
   constexpr int VP = 64 + 8;             // padded row of the transposed V tile (f16)
-  constexpr int PP = 64 + 4;             // padded row of the P tiles (f32)
   __shared__ __attribute__((aligned(16))) uint16_t ks[64 * HD];        // keys x dims, chunks swizzled
   __shared__ __attribute__((aligned(16))) uint16_t vt[HD * VP];        // dims x keys
-  __shared__ __attribute__((aligned(16))) float pw[4][16 * PP];         // per wave: P, rows x keys
-  sgpr_ready(q, K, V, o, n_q, prefix, n_q_heads, n_kv_heads, scale);
+  sgpr_ready(q, K, V, o, n_q, prefix, n_q_heads, n_kv_heads, c_hi, c_lo);
   const uint32_t kvh = blockIdx.x, q0 = blockIdx.y * QT;
   const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -533,7 +536,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   // words of the transposed tile, and a wave's 32-bit writes for one dim
   // fall on 64 different banks (lanes 32..63 write the rows 8 dims on).
   constexpr int IT = LPT / 2;  // items per thread
-  uint4 kr[IT][2], vr[IT][2];
+  u32x4 kr[IT][2], vr[IT][2];
   auto item_ch = [&](int i) { return (lane >> 5) + 2 * (wave + 4 * i); };
   const uint32_t kp = lane & 31;
   auto gload = [&](uint32_t t) {
@@ -543,8 +546,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 #pragma unroll
       for (int e = 0; e < 2; e++) {
         const size_t row = (size_t)min(64 * t + 2 * kp + e, kv_last) * kv_row + 8 * ch;
-        kr[i][e] = *reinterpret_cast<const uint4 *>(Kh + row);
-        vr[i][e] = *reinterpret_cast<const uint4 *>(Vh + row);
+        kr[i][e] = *reinterpret_cast<const u32x4 *>(Kh + row);
+        vr[i][e] = *reinterpret_cast<const u32x4 *>(Vh + row);
       }
     }
   };
@@ -558,9 +561,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   // This lane's Q operand row (16 wave + l16) as f16 hi + mid + lo, dims
   // 32c + 8lq (each remainder is exact in f32).
   v8h_t qhi[NC], qmid[NC], qlo[NC];
+  const uint32_t row = 16 * wave + l16, qi = q0 + row / G, head = kvh * G + row % G;
   {
-    const uint32_t r = 16 * wave + l16, qi = min(q0 + r / G, n_q - 1), h = kvh * G + r % G;
-    const float *qr = q + ((size_t)qi * n_q_heads + h) * HD + 8 * lq;
+    const float *qr = q + ((size_t)min(qi, n_q - 1) * n_q_heads + head) * HD + 8 * lq;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       const float4 a = *reinterpret_cast<const float4 *>(qr + 32 * c);
@@ -577,17 +580,13 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
       }
     }
   }
-  // Output rows of this lane: 16 wave + 4 lq + j; the last key each sees.
-  uint32_t vis[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) vis[j] = prefix + q0 + (16 * wave + 4 * lq + j) / G;
-  float m[4], l[4];
+  // The last key this lane's query sees, and the wave's first query.
+  const uint32_t vis = prefix + qi, vis0 = prefix + q0 + 16 * wave / G;
+  const float slack = 8.0f / c_hi;  // in scores: a factor 2^8 of p
+  float m = -INFINITY, l = 0.f;     // l: this lane's keys only
   v4f_t O[ND];
 #pragma unroll
-  for (int j = 0; j < 4; j++) m[j] = -INFINITY, l[j] = 0.f;
-#pragma unroll
   for (int n = 0; n < ND; n++) O[n] = v4f_t{0.f, 0.f, 0.f, 0.f};
-  float *pwf = pw[wave];
 
   for (uint32_t t = t_begin; t < t_end; t++) {
     lds_barrier();  // the previous tile's reads of ks and vt are done
@@ -597,7 +596,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 #pragma unroll
       for (int e = 0; e < 2; e++) {
         const uint32_t key = 2 * kp + e;
-        *reinterpret_cast<uint4 *>(&ks[key * HD + 8 * (ch ^ (key & (KCH - 1)))]) = kr[i][e];
+        *reinterpret_cast<u32x4 *>(&ks[key * HD + 8 * (ch ^ (key & (KCH - 1)))]) = kr[i][e];
       }
       const uint32_t a[4] = {vr[i][0].x, vr[i][0].y, vr[i][0].z, vr[i][0].w};
       const uint32_t b[4] = {vr[i][1].x, vr[i][1].y, vr[i][1].z, vr[i][1].w};
@@ -611,91 +610,90 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     lds_barrier();
     if (t + 1 < t_end) gload(t + 1);  // in flight over this tile's arithmetic
 
-    // ---- S = Q K^T: 16 rows x 64 keys per wave ----
+    // ---- S^T = K Q^T: 64 keys x 16 queries per wave ----
     v4f_t S[4];
 #pragma unroll
     for (int kb = 0; kb < 4; kb++) S[kb] = v4f_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      v8h_t B[4];
+      v8h_t A[4];
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) {
         const uint32_t key = 16 * kb + l16;
-        B[kb] = *reinterpret_cast<const v8h_t *>(&ks[key * HD + 8 * ((4 * c + lq) ^ (key & (KCH - 1)))]);
+        A[kb] = *reinterpret_cast<const v8h_t *>(&ks[key * HD + 8 * ((4 * c + lq) ^ (key & (KCH - 1)))]);
       }
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qlo[c], B[kb], S[kb], 0, 0, 0);
+      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qlo[c], S[kb], 0, 0, 0);
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qmid[c], B[kb], S[kb], 0, 0, 0);
+      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qmid[c], S[kb], 0, 0, 0);
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qhi[c], B[kb], S[kb], 0, 0, 0);
+      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qhi[c], S[kb], 0, 0, 0);
     }
-    // ---- online softmax; P to this wave's LDS tile ----
+    // ---- online softmax: S[kb][r] is key 64 t + 16 kb + 4 lq + r ----
+    if (64 * t + 63 > vis0) {  // (uniform) a key some query of the wave does not see
+      const uint32_t k0 = 64 * t + 4 * lq;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      float s[4], mx = -INFINITY;
+      for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) {
-        const uint32_t key = 64 * t + 16 * kb + l16;
-        s[kb] = key <= vis[j] ? S[kb][j] * scale : -INFINITY;
-        mx = fmaxf(mx, s[kb]);
-      }
-      // mn is finite once a visible key has been seen (the first tile of
-      // chunk 0 holds key 0); a later chunk's row may see none yet.
-      const float mn = fmaxf(m[j], row16_max(mx));
-      const float alpha = mn == -INFINITY ? 1.f : expf(m[j] - mn);  // 0 on the first visible tile (m = -inf)
-      float ps = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 4; kb++) {
-        const float p = s[kb] == -INFINITY ? 0.f : expf(s[kb] - mn);  // 0 for masked keys
-        ps += p;
-        pwf[(4 * lq + j) * PP + 16 * kb + l16] = p;
-      }
-      l[j] = l[j] * alpha + row16_sum(ps);
-      m[j] = mn;
-#pragma unroll
-      for (int n = 0; n < ND; n++) O[n][j] *= alpha;
+        for (int r = 0; r < 4; r++)
+          if (k0 + 16 * kb + r > vis) S[kb][r] = -INFINITY;
     }
-    // ---- O += P V (the wave reads back only its own P tile) ----
+    float mx = S[0][0];
+#pragma unroll
+    for (int i = 1; i < 16; i++) mx = fmaxf(mx, S[i >> 2][i & 3]);
+    mx = quarter_max(mx);
+    if (__any(mx > m + slack)) {  // (also the first visible tile, m = -inf)
+      const float mn = fmaxf(m, mx);
+      const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * c_hi);
+      l *= al;
+#pragma unroll
+      for (int n = 0; n < ND; n++) O[n] *= al;
+      m = mn;
+    }
+    const float mr = m == -INFINITY ? 0.f : m;  // a later chunk's query may see no key yet
+    v8h_t Ph[2], Pl[2];
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float d = S[kb][r] - mr;
+        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(d, c_hi, d * c_lo));  // 0 for masked keys
+        l += pv;
+        const _Float16 hi = (_Float16)pv;
+        Ph[kb >> 1][4 * (kb & 1) + r] = hi;
+        Pl[kb >> 1][4 * (kb & 1) + r] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, pv);
+      }
+    // ---- O^T += V^T P^T: element e of lane lq is key 32 c + 16 (e / 4) + 4 lq + e % 4 ----
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-      const float4 p0 = *reinterpret_cast<const float4 *>(&pwf[l16 * PP + 32 * c + 8 * lq]);
-      const float4 p1 = *reinterpret_cast<const float4 *>(&pwf[l16 * PP + 32 * c + 8 * lq + 4]);
-      const float pv[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-      v8h_t Ah, Al;
+      v8h_t A[ND];
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const _Float16 hi = (_Float16)pv[e];
-        Ah[e] = hi;
-        Al[e] = (_Float16)(pv[e] - (float)hi);
+      for (int n = 0; n < ND; n++) {
+        const uint16_t *vp = &vt[(16 * n + l16) * VP + 32 * c + 4 * lq];
+        const v4h_t a = *reinterpret_cast<const v4h_t *>(vp), b = *reinterpret_cast<const v4h_t *>(vp + 16);
+        A[n] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
       }
-      v8h_t B[ND];
 #pragma unroll
-      for (int n = 0; n < ND; n++) B[n] = *reinterpret_cast<const v8h_t *>(&vt[(16 * n + l16) * VP + 32 * c + 8 * lq]);
+      for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[n], Ph[c], O[n], 0, 0, 0);
 #pragma unroll
-      for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, B[n], O[n], 0, 0, 0);
-#pragma unroll
-      for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, B[n], O[n], 0, 0, 0);
+      for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[n], Pl[c], O[n], 0, 0, 0);
     }
   }
   if (n_ch > 1) {
     // Leave this chunk's (m, l, O), then the last chunk to arrive merges.
-    constexpr int NV = 8 + 4 * ND;
+    constexpr int NV = 2 + 4 * ND;
     __shared__ uint32_t last;
     const size_t blk = (size_t)kvh * gridDim.y + blockIdx.y;
     float *pb = part + blk * gridDim.z * (NV * 256) + tid;
     {
       float *pc = pb + (size_t)ch * (NV * 256);
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        __hip_atomic_store(pc + 256 * j, m[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(pc + 256 * (4 + j), l[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+      __hip_atomic_store(pc, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(pc + 256, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
       for (int n = 0; n < ND; n++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
-          __hip_atomic_store(pc + 256 * (8 + 4 * n + j), O[n][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(pc + 256 * (2 + 4 * n + j), O[n][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -707,79 +705,68 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     }
     __syncthreads();
     if (!last) return;
-    float M[4], L[4];
+    float M = 0.f, L = 0.f;
     v4f_t OA[ND];
     for (uint32_t c = 0; c < n_ch; c++) {
       const float *pc = pb + (size_t)c * (NV * 256);
-      float mc[4], lc[4];
+      const float mc = c == ch ? m : __hip_atomic_load(pc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const float lc = c == ch ? l : __hip_atomic_load(pc + 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       v4f_t Oc[ND];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        mc[j] = c == ch ? m[j] : __hip_atomic_load(pc + 256 * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        lc[j] = c == ch ? l[j] : __hip_atomic_load(pc + 256 * (4 + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
 #pragma unroll
       for (int n = 0; n < ND; n++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
           Oc[n][j] = c == ch ? O[n][j]
-                             : __hip_atomic_load(pc + 256 * (8 + 4 * n + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                             : __hip_atomic_load(pc + 256 * (2 + 4 * n + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (c == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) M[j] = mc[j], L[j] = lc[j];
+        M = mc, L = lc;
 #pragma unroll
         for (int n = 0; n < ND; n++) OA[n] = Oc[n];
       } else {
+        const float mn = fmaxf(M, mc);  // finite: chunk 0's M is
+        const float da = M - mn, db = mc - mn;
+        const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(da, c_hi, da * c_lo));
+        const float b = mc == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(db, c_hi, db * c_lo));
+        L = L * a + lc * b;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const float mn = fmaxf(M[j], mc[j]);  // finite: chunk 0's M is
-          const float a = expf(M[j] - mn), b = mc[j] == -INFINITY ? 0.f : expf(mc[j] - mn);
-          L[j] = L[j] * a + lc[j] * b;
-#pragma unroll
-          for (int n = 0; n < ND; n++) OA[n][j] = OA[n][j] * a + Oc[n][j] * b;
-          M[j] = mn;
-        }
+        for (int n = 0; n < ND; n++) OA[n] = OA[n] * a + Oc[n] * b;
+        M = mn;
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) l[j] = L[j];
+    l = L;
 #pragma unroll
     for (int n = 0; n < ND; n++) O[n] = OA[n];
   }
+  l = quarter_sum(l);
   const bool qo = in.xh != nullptr;  // uniform
   const uint32_t KO = n_q_heads * HD;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint32_t r = 16 * wave + 4 * lq + j, qi = q0 + r / G, h = kvh * G + r % G;
-    float val[ND];
+  for (int n = 0; n < ND; n++) O[n] = O[n] / l;
+  if (qo) {
+    // The output projection's f16-path input (gemm_act_kernel's arithmetic):
+    // dims 32 b + [0, 32) of row (qi, head) are one quantization block, dims
+    // 16 n + 4 lq + j of the four lanes that hold the row.
 #pragma unroll
-    for (int n = 0; n < ND; n++) val[n] = O[n][j] / l[j];
-    if (qo) {
-      // The output projection's f16-path input (gemm_act_kernel's arithmetic):
-      // dims 32 b + [0, 32) of row (qi, h) are one quantization block, dims
-      // 2 b and 2 b + 1 of the 16 lanes that hold the row. Lane pairs swap
-      // halves so that each lane stores one pair of adjacent dims: an even
-      // lane dims l16, l16 + 1, an odd lane dims 15 + l16, 16 + l16.
+    for (int b = 0; b < ND / 2; b++) {
+      float am = 0.f;
 #pragma unroll
-      for (int b = 0; b < ND / 2; b++) {
-        const float am = row16_max(fmaxf(fabsf(val[2 * b]), fabsf(val[2 * b + 1])));
-        const float iv = am == 0.f ? 0.f : 127.0f / am;
-        const uint32_t ha = __builtin_bit_cast(uint16_t, (_Float16)(float)q8_quant(val[2 * b], iv));
-        const uint32_t hb = __builtin_bit_cast(uint16_t, (_Float16)(float)q8_quant(val[2 * b + 1], iv));
-        const uint32_t na = dpp_u32<0xB1, 0xF>(ha), nb = dpp_u32<0xB1, 0xF>(hb);  // lane l16 ^ 1's
-        if (qi < n_q) {
-          const bool ev = (l16 & 1) == 0;
-          _Float16 *xr = in.xh + (size_t)qi * KO + h * HD + 32 * b + (ev ? l16 : 15 + l16);
-          *reinterpret_cast<uint32_t *>(xr) = ev ? ha | na << 16 : nb | hb << 16;
-          if (l16 == 0) in.sx[(size_t)qi * (KO / 32) + h * (HD / 32) + b] = am / 127.0f;
-        }
+      for (int i = 0; i < 8; i++) am = fmaxf(am, fabsf(O[2 * b + (i >> 2)][i & 3]));
+      am = quarter_max(am);
+      const float iv = am == 0.f ? 0.f : 127.0f / am;
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        v4h_t hv;
+#pragma unroll
+        for (int j = 0; j < 4; j++) hv[j] = (_Float16)(float)q8_quant(O[2 * b + e][j], iv);
+        if (qi < n_q) *reinterpret_cast<v4h_t *>(in.xh + (size_t)qi * KO + head * HD + 32 * b + 16 * e + 4 * lq) = hv;
       }
+      if (qi < n_q && lq == 0) in.sx[(size_t)qi * (KO / 32) + head * (HD / 32) + b] = am / 127.0f;
     }
-    if (qi >= n_q) continue;
-    float *orow = o + ((size_t)qi * n_q_heads + h) * HD + l16;
-#pragma unroll
-    for (int n = 0; n < ND; n++) orow[16 * n] = val[n];
   }
+  if (qi >= n_q) return;
+  float *orow = o + ((size_t)qi * n_q_heads + head) * HD + 4 * lq;
+#pragma unroll
+  for (int n = 0; n < ND; n++) *reinterpret_cast<v4f_u *>(orow + 16 * n) = O[n];
 }
 
 // Split-key attention (flash-decoding). A workgroup takes one query, one KV
@@ -1473,7 +1460,10 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
       kv_len * n_kv_heads * hd < (1ull << 32) && n_kv_heads < 65536) {
     // A prompt's causal attention on the matrix cores (attn_prefill_kernel).
     const uint64_t QT = 64 / GP, nqb = (n_q + QT - 1) / QT;
-    const float sc = 1.0f / sqrtf((float)hd);
+    // scale * log2 e in two floats, both positive (a masked score's -inf
+    // times each of them is then -inf).
+    const double c = 1.4426950408889634 / std::sqrt((double)hd);
+    const float c_hi = std::nextafter((float)c, 0.f), c_lo = (float)(c - (double)c_hi);
     const uint32_t pre = (uint32_t)(kv_len - n_q);
     // Key chunks of ct tiles: about two workgroups per CU (what stays
     // resident) over the prompt's tile work, at least two tiles each; none
@@ -1488,7 +1478,7 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     units *= n_kv_heads;
     const uint64_t cus = ctx->cu_count ? ctx->cu_count : 256;
     uint64_t ct = std::max<uint64_t>(2, (units + 2 * cus - 1) / (2 * cus)), n_ch = (max_t + ct - 1) / ct;
-    const uint64_t NV = 8 + 4 * (hd / 16), pbytes = n_kv_heads * nqb * n_ch * NV * 256 * 4;
+    const uint64_t NV = 2 + 4 * (hd / 16), pbytes = n_kv_heads * nqb * n_ch * NV * 256 * 4;
     if (n_ch < 2 || ctx->capturing || ctx->fixed_scratch || pbytes > (256ull << 20)) ct = 0, n_ch = 1;
     float *part = ct ? reinterpret_cast<float *>(scratch(ctx, pbytes)) : nullptr;
     uint32_t *cnt = ct ? attn_counters(ctx, n_kv_heads * nqb) : nullptr;
@@ -1500,7 +1490,7 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     const dim3 grid((uint32_t)n_kv_heads, (uint32_t)nqb, (uint32_t)n_ch);
 #define MDMA_ATTP(GG, HH)                                                                                          \
   attn_prefill_kernel<GG, HH><<<grid, dim3(256), 0, ctx->stream>>>(q, k, v, o, (uint32_t)n_q, pre, (uint32_t)n_q_heads, \
-                                                                   (uint32_t)n_kv_heads, sc, (uint32_t)ct, part, cnt, \
+                                                                   (uint32_t)n_kv_heads, c_hi, c_lo, (uint32_t)ct, part, cnt, \
                                                                    fin)
     if (hd == 128) {
       if (GP == 1) MDMA_ATTP(1, 128);

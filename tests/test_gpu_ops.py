@@ -205,3 +205,25 @@ def test_greedy(backend):
     bad[9999] = np.nan
     with pytest.raises(BackendError):
         backend.greedy(backend.f32_buf(bad))
+
+
+@pytest.mark.parametrize("hd,nq,nkv,n_q,kv_len", [(128, 8, 2, 70, 400), (64, 4, 4, 130, 131)])
+@pytest.mark.parametrize("rising", [True, False])
+def test_prompt_attention_with_growing_scores(backend, hd, nq, nkv, n_q, kv_len, rising):
+    # Scores that grow (fall) along the keys to +-40: each tile passes the
+    # running maximum by more than its slack (never does after the first).
+    # A score's own f32 sum is off by up to hd u |s| / 2 = 1.5e-4 at 40; the
+    # weights, and so the outputs (|v| < 5), by that factor.
+    ramp = np.linspace(0.0, 40.0, kv_len, dtype=np.float32)[::1 if rising else -1]
+    q = synth.normal_f32(n_q * nq * hd, 1).reshape(-1, hd) * 0.1
+    q[:, 0] = np.sqrt(hd)
+    k = synth.normal_f32(kv_len * nkv * hd, 2).reshape(kv_len, nkv, hd)
+    k[:, :, 0] = ramp[:, None]
+    k, v = f16r(k.reshape(-1)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
+    kb, vb = backend.alloc(k.size * 2), backend.alloc(v.size * 2)
+    backend.upload(kb, 0, k.astype(np.float16))
+    backend.upload(vb, 0, v.astype(np.float16))
+    o = backend.alloc(q.size * 4)
+    backend.attn(backend.f32_buf(q), KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
+    want = ffi.attention(q.reshape(-1), k, v, kv_len, hd, nq, nkv)
+    np.testing.assert_allclose(backend.download_f32(o), want, rtol=0, atol=5 * 1.5e-4)
