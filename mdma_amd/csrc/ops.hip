@@ -482,7 +482,17 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // in.xh set: the writer of O / l also writes the output projection's
 // f16-path input (per 32 dims of a row the int8 values as f16 and
 // amax / 127, the gemm_f16 quantization pass's arithmetic), no P halves.
-constexpr uint32_t ATT_PREFILL_MIN = 64;
+// Chunks of at least sqrt(ATT_MERGE_TILES * tiles) tiles: a chunk's place in
+// the serial merge costs about a quarter of a tile's time (16 queries over
+// 3900 keys, G = 4: 31 chunks of 2 tiles 26.3 us, 16 of 4 tiles 21.2, 10 of
+// 7 tiles 23.3).
+constexpr double ATT_MERGE_TILES = 0.25;
+// Queries from which it is the faster kernel: any prompt of 64, and from 8
+// where the per-query kernel's K/V reads add up (us, per query / here, 32
+// heads: 48 queries over 3900 keys 98 / 27.5, 16 over 1500 20.4 / 15.1, 8 over
+// 3900 25.6 / 20.9, 16 over 500 11.4 / 11.3, 16 over 100 6.9 / 8.1; 20 heads of
+// G = 1: 8 over 1000 11.9 / 14.9).
+constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_PREFILL_PAIRS = 16384;
 
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
@@ -652,17 +662,19 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     }
     const float mr = m == -INFINITY ? 0.f : m;  // a later chunk's query may see no key yet
     v8h_t Ph[2], Pl[2];
+    float ps[4] = {};  // (summed apart: l takes one rounding a tile at its own size)
 #pragma unroll
     for (int kb = 0; kb < 4; kb++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const float d = S[kb][r] - mr;
         const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(d, c_hi, d * c_lo));  // 0 for masked keys
-        l += pv;
+        ps[r] += pv;
         const _Float16 hi = (_Float16)pv;
         Ph[kb >> 1][4 * (kb & 1) + r] = hi;
         Pl[kb >> 1][4 * (kb & 1) + r] = (_Float16)__builtin_fmaf(-1.0f, (float)hi, pv);
       }
+    l += (ps[0] + ps[1]) + (ps[2] + ps[3]);
     // ---- O^T += V^T P^T: element e of lane lq is key 32 c + 16 (e / 4) + 4 lq + e % 4 ----
 #pragma unroll
     for (int c = 0; c < 2; c++) {
@@ -705,31 +717,40 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     }
     __syncthreads();
     if (!last) return;
+    // Four chunks' loads at a time (past the last: read again, not added).
+    constexpr int MC = 4;
     float M = 0.f, L = 0.f;
     v4f_t OA[ND];
-    for (uint32_t c = 0; c < n_ch; c++) {
-      const float *pc = pb + (size_t)c * (NV * 256);
-      const float mc = c == ch ? m : __hip_atomic_load(pc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float lc = c == ch ? l : __hip_atomic_load(pc + 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      v4f_t Oc[ND];
+    for (uint32_t c0 = 0; c0 < n_ch; c0 += MC) {
+      float mc[MC], lc[MC];
+      v4f_t Oc[MC][ND];
 #pragma unroll
-      for (int n = 0; n < ND; n++)
+      for (int i = 0; i < MC; i++) {
+        const float *pc = pb + (size_t)min(c0 + i, n_ch - 1) * (NV * 256);
+        mc[i] = __hip_atomic_load(pc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lc[i] = __hip_atomic_load(pc + 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-          Oc[n][j] = c == ch ? O[n][j]
-                             : __hip_atomic_load(pc + 256 * (2 + 4 * n + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (c == 0) {
-        M = mc, L = lc;
+        for (int n = 0; n < ND; n++)
 #pragma unroll
-        for (int n = 0; n < ND; n++) OA[n] = Oc[n];
-      } else {
-        const float mn = fmaxf(M, mc);  // finite: chunk 0's M is
-        const float da = M - mn, db = mc - mn;
+          for (int j = 0; j < 4; j++)
+            Oc[i][n][j] = __hip_atomic_load(pc + 256 * (2 + 4 * n + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int i = 0; i < MC; i++) {
+        if (c0 + i >= n_ch) break;
+        if (c0 + i == 0) {
+          M = mc[0], L = lc[0];
+#pragma unroll
+          for (int n = 0; n < ND; n++) OA[n] = Oc[0][n];
+          continue;
+        }
+        const float mn = fmaxf(M, mc[i]);  // finite: chunk 0's M is
+        const float da = M - mn, db = mc[i] - mn;
         const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(da, c_hi, da * c_lo));
-        const float b = mc == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(db, c_hi, db * c_lo));
-        L = L * a + lc * b;
+        const float b = mc[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(db, c_hi, db * c_lo));
+        L = L * a + lc[i] * b;
 #pragma unroll
-        for (int n = 0; n < ND; n++) OA[n] = OA[n] * a + Oc[n] * b;
+        for (int n = 0; n < ND; n++) OA[n] = OA[n] * a + Oc[i][n] * b;
         M = mn;
       }
     }
@@ -1455,7 +1476,8 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
   uint16_t *k = const_cast<uint16_t *>(kc), *v = const_cast<uint16_t *>(vc);
   const uint32_t *pos_dev = rope_in ? rope_in->pos_dev : nullptr;
   const uint64_t GP = n_kv_heads ? n_q_heads / n_kv_heads : 0;
-  if (!rope_in && !q8 && !seq_stride && n_q >= ATT_PREFILL_MIN && kv_len >= n_q && (hd == 64 || hd == 128) &&
+  if (!rope_in && !q8 && !seq_stride && kv_len >= n_q &&
+      (n_q >= ATT_PREFILL_MIN || (n_q >= ATT_PREFILL_FEW && n_q * kv_len >= ATT_PREFILL_PAIRS)) && (hd == 64 || hd == 128) &&
       n_kv_heads && GP * n_kv_heads == n_q_heads && (GP == 1 || GP == 2 || GP == 4 || GP == 8) &&
       kv_len * n_kv_heads * hd < (1ull << 32) && n_kv_heads < 65536) {
     // A prompt's causal attention on the matrix cores (attn_prefill_kernel).
@@ -1466,7 +1488,8 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     const float c_hi = std::nextafter((float)c, 0.f), c_lo = (float)(c - (double)c_hi);
     const uint32_t pre = (uint32_t)(kv_len - n_q);
     // Key chunks of ct tiles: about two workgroups per CU (what stays
-    // resident) over the prompt's tile work, at least two tiles each; none
+    // resident) over the prompt's tile work, at least two tiles each and long
+    // enough for the merge; none
     // when no block has more than ct tiles, under stream capture or in a
     // fixed scratch.
     uint64_t units = 0, max_t = 0;
@@ -1477,7 +1500,8 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     }
     units *= n_kv_heads;
     const uint64_t cus = ctx->cu_count ? ctx->cu_count : 256;
-    uint64_t ct = std::max<uint64_t>(2, (units + 2 * cus - 1) / (2 * cus)), n_ch = (max_t + ct - 1) / ct;
+    const uint64_t mrg = (uint64_t)std::ceil(std::sqrt(ATT_MERGE_TILES * (double)max_t));  // cheap enough to merge
+    uint64_t ct = std::max({(uint64_t)2, (units + 2 * cus - 1) / (2 * cus), mrg}), n_ch = (max_t + ct - 1) / ct;
     const uint64_t NV = 2 + 4 * (hd / 16), pbytes = n_kv_heads * nqb * n_ch * NV * 256 * 4;
     if (n_ch < 2 || ctx->capturing || ctx->fixed_scratch || pbytes > (256ull << 20)) ct = 0, n_ch = 1;
     float *part = ct ? reinterpret_cast<float *>(scratch(ctx, pbytes)) : nullptr;

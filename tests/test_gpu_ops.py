@@ -227,3 +227,22 @@ def test_prompt_attention_with_growing_scores(backend, hd, nq, nkv, n_q, kv_len,
     backend.attn(backend.f32_buf(q), KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
     want = ffi.attention(q.reshape(-1), k, v, kv_len, hd, nq, nkv)
     np.testing.assert_allclose(backend.download_f32(o), want, rtol=0, atol=5 * 1.5e-4)
+
+
+@pytest.mark.parametrize("hd,nq,nkv,n_q,kv_len", [(128, 32, 8, 8, 2048), (128, 8, 2, 9, 1821), (64, 4, 4, 17, 1000),
+                                                  (128, 4, 4, 63, 300), (64, 16, 2, 20, 2500), (128, 8, 4, 12, 4000)])
+def test_few_queries_over_long_prefixes(backend, hd, nq, nkv, n_q, kv_len):
+    # 8 to 63 queries on the matrix-core kernel: part-filled query blocks,
+    # many key chunks and their merge (four at a time, remainders of four).
+    q = synth.normal_f32(n_q * nq * hd, 1)
+    k, v = f16r(synth.normal_f32(kv_len * nkv * hd, 2)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
+    kb, vb = backend.alloc(k.size * 2), backend.alloc(v.size * 2)
+    backend.upload(kb, 0, k.astype(np.float16))
+    backend.upload(vb, 0, v.astype(np.float16))
+    o = backend.f32_buf(np.full(q.size + 2, -3.0, np.float32))
+    for _ in range(2):  # the second call finds the chunk counters as the first left them
+        backend.attn(backend.f32_buf(q), KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
+    got = backend.download_f32(o)
+    assert np.all(got[q.size:] == -3.0)
+    want = ffi.attention(q, k, v, kv_len, hd, nq, nkv)
+    np.testing.assert_allclose(got[:q.size], want, rtol=2e-5, atol=2e-6)
