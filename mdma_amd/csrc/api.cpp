@@ -320,8 +320,14 @@ void no_capture(mdma_ctx *ctx, const char *what) {
 // first. False when there is nothing to give or the stream cannot be drained
 // now.
 static bool drop_split_parts(mdma_ctx *ctx) {
-  if (!ctx->split_part || ctx->capturing || ctx->fixed_scratch) return false;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->split_part) != hipSuccess) return false;
+  if ((!ctx->split_part && ctx->split_part_old.empty()) || ctx->capturing || ctx->fixed_scratch) return false;
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+  for (; !ctx->split_part_old.empty(); ctx->split_part_old.pop_back()) {
+    if (hipFree(ctx->split_part_old.back().first) != hipSuccess) return false;
+    budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_old.back().second);
+    ctx->buf_epoch++;  // a captured launch points into it
+  }
+  if (ctx->split_part && hipFree(ctx->split_part) != hipSuccess) return false;
   budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_cap);
   if (ctx->split_part_captured) ctx->buf_epoch++;
   ctx->split_part = nullptr;
@@ -403,17 +409,32 @@ char *argmax_parts(mdma_ctx *ctx, uint64_t chunks) {
 void *split_parts(mdma_ctx *ctx, uint64_t bytes) {
   if (bytes > ctx->split_part_cap) {
     if (ctx->capturing || ctx->fixed_scratch) return nullptr;
-    // Graphs that do not hold it stay valid: the epoch moves only for those
-    // that do.
-    const uint64_t epoch = ctx->buf_epoch;
-    try {
-      regrow(ctx, ctx->split_part, ctx->split_part_cap, bytes, 1, "split partials growth");
-    } catch (const Error &) {
-      (void)hipGetLastError();
-      if (!ctx->split_part_captured) ctx->buf_epoch = epoch;
-      if (bytes > ctx->split_part_cap) return nullptr;
+    // A captured launch keeps the space it points into (its graph stays
+    // valid); the next one is at least twice as large, so what is kept is
+    // less than what is in use.
+    const bool keep = ctx->split_part_captured;
+    const uint64_t cap = keep ? std::max(bytes, 2 * ctx->split_part_cap) : bytes;
+    const Ledger &l = ctx->budget[MDMA_DOMAIN_DEVICE];
+    const uint64_t used = l.used - (keep ? 0 : ctx->split_part_cap);
+    if (used + cap < used || used + cap > l.limit) return nullptr;
+    if (keep) {
+      ctx->split_part_old.reserve(ctx->split_part_old.size() + 1);
+    } else if (ctx->split_part) {
+      // (What older graphs hold stays: only the space in use is replaced.)
+      if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->split_part) != hipSuccess) return nullptr;
+      budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_cap);
+      ctx->split_part = nullptr;
+      ctx->split_part_cap = 0;
     }
-    if (!ctx->split_part_captured) ctx->buf_epoch = epoch;
+    void *p = nullptr;
+    if (hipMalloc(&p, cap) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    budget_charge(ctx, MDMA_DOMAIN_DEVICE, cap, "split partials growth");
+    if (keep) ctx->split_part_old.emplace_back(ctx->split_part, ctx->split_part_cap);
+    ctx->split_part = static_cast<char *>(p);
+    ctx->split_part_cap = cap;
     ctx->split_part_captured = false;
   }
   if (ctx->capturing) ctx->split_part_captured = true;
@@ -543,6 +564,7 @@ void mdma_gfx950_destroy(mdma_ctx *ctx) {
   if (ctx->gemm_cnt) (void)hipFree(ctx->gemm_cnt);
   if (ctx->ssq) (void)hipFree(ctx->ssq);
   if (ctx->split_part) (void)hipFree(ctx->split_part);
+  for (auto &o : ctx->split_part_old) (void)hipFree(o.first);
   if (ctx->rope_tab) (void)hipFree(ctx->rope_tab);
   if (ctx->host_ids) (void)hipHostFree(ctx->host_ids);
   (void)hipStreamDestroy(ctx->stream);

@@ -145,6 +145,7 @@ struct mdma_ctx {
   char *split_part = nullptr;  // partial sums of launches that split K (gemm_f64.hip, gemv_wide)
   uint64_t split_part_cap = 0;
   bool split_part_captured = false;  // a captured launch points into it
+  std::vector<std::pair<char *, uint64_t>> split_part_old;  // outgrown, held for the graphs that point into them
   double *ssq = nullptr;  // per-workgroup sums of squares of a residual-stream GEMV (norm fusion)
   uint64_t ssq_cap = 0;
   uint32_t team_grid = 0;  // workgroups of the last row-team launch

@@ -491,7 +491,9 @@ constexpr double ATT_MERGE_TILES = 0.25;
 // where the per-query kernel's K/V reads add up (us, per query / here, 32
 // heads: 48 queries over 3900 keys 98 / 27.5, 16 over 1500 20.4 / 15.1, 8 over
 // 3900 25.6 / 20.9, 16 over 500 11.4 / 11.3, 16 over 100 6.9 / 8.1; 20 heads of
-// G = 1: 8 over 1000 11.9 / 14.9).
+// G = 1: 8 over 1000 11.9 / 14.9). Under a capture or in a fixed scratch, where
+// the key chunks are not made, few queries stay with the per-query kernel: one
+// workgroup a KV head would walk all the tiles in turn.
 constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_PREFILL_PAIRS = 16384;
 
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
@@ -1477,7 +1479,8 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
   const uint32_t *pos_dev = rope_in ? rope_in->pos_dev : nullptr;
   const uint64_t GP = n_kv_heads ? n_q_heads / n_kv_heads : 0;
   if (!rope_in && !q8 && !seq_stride && kv_len >= n_q &&
-      (n_q >= ATT_PREFILL_MIN || (n_q >= ATT_PREFILL_FEW && n_q * kv_len >= ATT_PREFILL_PAIRS)) && (hd == 64 || hd == 128) &&
+      (n_q >= ATT_PREFILL_MIN || (n_q >= ATT_PREFILL_FEW && n_q * kv_len >= ATT_PREFILL_PAIRS && !ctx->capturing &&
+                                  !ctx->fixed_scratch)) && (hd == 64 || hd == 128) &&
       n_kv_heads && GP * n_kv_heads == n_q_heads && (GP == 1 || GP == 2 || GP == 4 || GP == 8) &&
       kv_len * n_kv_heads * hd < (1ull << 32) && n_kv_heads < 65536) {
     // A prompt's causal attention on the matrix cores (attn_prefill_kernel).

@@ -9,7 +9,7 @@ import pytest
 import npq
 from conftest import assert_parity, f32_exact
 from mdma_amd import synth
-from mdma_amd.backend import DOMAIN_DEVICE, Gfx950Backend
+from mdma_amd.backend import DOMAIN_DEVICE, BackendError, Gfx950Backend
 from oracle import ffi
 
 pytestmark = pytest.mark.gpu
@@ -96,6 +96,42 @@ def test_partials_space_gives_way_to_the_budget():
     be.qmatmul(w, x, y)  # no space: unsplit
     check(be, y, T, Q4K, raw, rows, k, x_h, "over budget")
     rest.close()
+    be.close()
+
+
+@pytest.mark.parametrize("full", [False, True])
+def test_captured_partials_space_outlives_its_growth(full):
+    # A graph that holds the partial tiles' space replays after a larger call
+    # wanted more of it: the space was replaced but kept for the graph, or the
+    # budget had no room and that call ran unsplit. Once a caller's allocation
+    # takes it back, the graph refuses.
+    be = Gfx950Backend(0)
+    be.set_buffer_budget(device=512 << 20)
+    rows, k, T, big_rows, big_T = 200, 1024, 20, 2100, 100
+    raw, big_raw = synth.weight(Q6K, rows, k, 1, True), synth.weight(Q6K, big_rows, k, 3, True)
+    w, bw = be.upload_weight(raw, Q6K, (rows, k)), be.upload_weight(big_raw, Q6K, (big_rows, k))
+    x_h, bx_h = synth.normal_f32(T * k, 2), synth.normal_f32(big_T * k, 4)
+    x, bx, y, by = be.f32_buf(x_h), be.f32_buf(bx_h), out_buf(be, T * rows), out_buf(be, big_T * big_rows)
+    be.qmatmul(w, x, y)  # makes the space
+    used = be.buffer_usage(DOMAIN_DEVICE)[0]
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+    filler = be.alloc(((512 << 20) - used) // 4096 * 4096 - 4096) if full else None
+    used = be.buffer_usage(DOMAIN_DEVICE)[0]
+    for _ in range(3):
+        be.qmatmul(bw, bx, by)
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        graph.launch()
+        check(be, y, T, Q6K, raw, rows, k, x_h, "replayed")
+        check(be, by, big_T, Q6K, big_raw, big_rows, k, bx_h, "grown")
+    now, limit = be.buffer_usage(DOMAIN_DEVICE)
+    assert (now == used) if full else (now > used)
+    rest = be.alloc((limit - now) // 4096 * 4096 + 8192)
+    with pytest.raises(BackendError):
+        graph.launch()
+    rest.close()
+    if filler:
+        filler.close()
+    graph.close()
     be.close()
 
 

@@ -246,3 +246,30 @@ def test_few_queries_over_long_prefixes(backend, hd, nq, nkv, n_q, kv_len):
     assert np.all(got[q.size:] == -3.0)
     want = ffi.attention(q, k, v, kv_len, hd, nq, nkv)
     np.testing.assert_allclose(got[:q.size], want, rtol=2e-5, atol=2e-6)
+
+
+def test_captured_few_queries_take_the_per_query_kernel(backend):
+    # Under a capture the matrix-core kernel has no key chunks: 8 queries stay
+    # with the per-query kernel, whose first 7 rows are a 7-query call's bits
+    # (the same runs of tiles per query).
+    hd, nq, nkv, n_q, kv_len = 128, 32, 8, 8, 2048
+    q = synth.normal_f32(n_q * nq * hd, 1)
+    k, v = f16r(synth.normal_f32(kv_len * nkv * hd, 2)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
+    kb, vb = backend.alloc(k.size * 2), backend.alloc(v.size * 2)
+    backend.upload(kb, 0, k.astype(np.float16))
+    backend.upload(vb, 0, v.astype(np.float16))
+    spec, qb, o = AttnSpec(hd, nq, nkv), backend.f32_buf(q), backend.alloc(q.size * 4)
+    few = q.size // n_q * 7
+    o7 = backend.alloc(few * 4)
+    backend.attn(backend.f32_buf(q[:few]), KvView(kb, vb, kv_len - 1), spec, o7)
+    backend.reserve_scratch(16 << 20)
+    backend.attn(qb, KvView(kb, vb, 600), spec, o)  # (the arrival counters' space)
+    graph = backend.capture(lambda: backend.attn(qb, KvView(kb, vb, kv_len), spec, o))
+    want = ffi.attention(q, k, v, kv_len, hd, nq, nkv)
+    for _ in range(3):
+        backend.upload(o, 0, np.zeros(q.size, np.float32))
+        graph.launch()
+        got = backend.download_f32(o)
+        np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-6)
+        assert np.array_equal(got[:few], backend.download_f32(o7))
+    graph.close()
