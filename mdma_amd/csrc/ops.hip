@@ -448,8 +448,8 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 }
 
 // Causal GQA attention for a prompt (one sequence, seq_stride 0: query i
-// sees keys [0, prefix + i]; at least ATT_PREFILL_MIN queries) on the matrix
-// cores, flash-attention style. A workgroup takes 64 rows, 64/G queries
+// sees keys [0, prefix + i]; ATT_PREFILL_MIN queries or more, or a few over a
+// long prefix) on the matrix cores, flash-attention style. A workgroup takes 64 rows, 64/G queries
 // times the G query heads of one KV head; wave w owns rows 16w..16w+15.
 // Per tile of 64 keys:
 //   S = Q K^T on v_mfma_f32_16x16x32_f16. The f16 keys are exact operands;
@@ -1492,9 +1492,8 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     const uint32_t pre = (uint32_t)(kv_len - n_q);
     // Key chunks of ct tiles: about two workgroups per CU (what stays
     // resident) over the prompt's tile work, at least two tiles each and long
-    // enough for the merge; none
-    // when no block has more than ct tiles, under stream capture or in a
-    // fixed scratch.
+    // enough for the merge; none when no block has more than ct tiles, under
+    // stream capture or in a fixed scratch.
     uint64_t units = 0, max_t = 0;
     for (uint64_t b = 0; b < nqb; b++) {
       const uint64_t t = (pre + std::min((b + 1) * QT, n_q) - 1) / 64 + 1;

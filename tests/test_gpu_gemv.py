@@ -1000,3 +1000,22 @@ def test_prefill_gemm_fused_calls(backend, dtype):
         np.testing.assert_allclose(backend.download_f32(y), want, rtol=2e-3, atol=1e-3)
     finally:
         backend.set_act_mode(0)
+
+
+@pytest.mark.parametrize("T,rows", [(64, 128), (65, 33)])
+def test_prefill_q8_block_dots_at_their_largest(backend, T, rows):
+    # Every block dot at +-32 * 127 * 128 and the values next to it: the GEMM
+    # reads them from a float's bits. One 128-column stage, d = 1, x = +-127:
+    # whole numbers below 2^24, so the result is exact.
+    k = 128
+    w = np.full((rows, k // 32, 34), 0x80, np.uint8)  # q = -128
+    w[:, :, 0:2] = np.array([1.0], np.float16).view(np.uint8)
+    w[np.arange(rows), np.arange(rows) % 4, 2 + np.arange(rows) % 32] = 127
+    w[::5, :, 2:] = 127
+    x = np.where(np.arange(T)[:, None] % 2, -127.0, 127.0).astype(np.float32) * np.ones((1, k), np.float32)
+    wb, y = backend.upload_weight(w.reshape(-1), Q8, (rows, k)), backend.alloc(T * rows * 4)
+    backend.set_act_mode(backend_mod.ACT_I8)
+    backend.qmatmul(wb, backend.f32_buf(x), y)
+    backend.set_act_mode(backend_mod.ACT_F32)
+    want = x.astype(np.float64) @ w[:, :, 2:].reshape(rows, k).view(np.int8).astype(np.float64).T
+    assert np.array_equal(backend.download_f32(y).reshape(T, rows).astype(np.float64), want)
