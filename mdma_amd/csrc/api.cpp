@@ -315,12 +315,20 @@ void no_capture(mdma_ctx *ctx, const char *what) {
   if (ctx->fixed_scratch) fail(MDMA_ERR_BACKEND, std::string(what) + " would allocate inside an allocation-free call");
 }
 
-// Gives the split launches' partials back (they only spread work over the CUs): a
-// caller's allocation that the budget or the device has no room for comes
-// first. False when there is nothing to give or the stream cannot be drained
-// now.
+// What giving the split launches' partials back would free now: nothing under
+// a capture or in an allocation-free call.
+static uint64_t split_parts_held(const mdma_ctx *ctx) {
+  if (ctx->capturing || ctx->fixed_scratch) return 0;
+  uint64_t n = ctx->split_part_cap;
+  for (const auto &o : ctx->split_part_old) n += o.second;
+  return n;
+}
+
+// Gives them back (they only spread work over the CUs): a caller's allocation
+// that fits in their place comes first. False when there is nothing to give
+// or the stream cannot be drained now.
 static bool drop_split_parts(mdma_ctx *ctx) {
-  if ((!ctx->split_part && ctx->split_part_old.empty()) || ctx->capturing || ctx->fixed_scratch) return false;
+  if (!split_parts_held(ctx)) return false;
   if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
   for (; !ctx->split_part_old.empty(); ctx->split_part_old.pop_back()) {
     if (hipFree(ctx->split_part_old.back().first) != hipSuccess) return false;
@@ -338,8 +346,10 @@ static bool drop_split_parts(mdma_ctx *ctx) {
 
 void budget_charge(mdma_ctx *ctx, int domain, uint64_t bytes, const char *what) {
   Ledger &l = ctx->budget[domain];
-  if (domain == MDMA_DOMAIN_DEVICE && l.used + bytes > l.limit) drop_split_parts(ctx);
-  if (l.used + bytes < l.used || l.used + bytes > l.limit)
+  const auto fits = [&](uint64_t used) { return used + bytes >= used && used + bytes <= l.limit; };
+  // (A request that does not fit without the partials either changes nothing.)
+  if (domain == MDMA_DOMAIN_DEVICE && !fits(l.used) && fits(l.used - split_parts_held(ctx))) drop_split_parts(ctx);
+  if (!fits(l.used))
     fail(MDMA_ERR_BUFFER_BUDGET,
          fmt("%s: %s buffer budget exhausted: requested %llu bytes, used %llu, limit %llu", what,
              domain == MDMA_DOMAIN_DEVICE ? "device" : "host", (unsigned long long)bytes,

@@ -149,3 +149,26 @@ def test_nan_and_infinity_stay_in_their_token(backend):
     assert np.array_equal(got[keep], ref[keep])
     assert np.isnan(got[3]).all() and not np.isfinite(got[18]).any()
 
+
+
+def test_refused_allocation_leaves_partials_and_graphs():
+    # A request that the budget has no room for even without the partials'
+    # space is refused and changes nothing.
+    be = Gfx950Backend(0)
+    be.set_buffer_budget(device=256 << 20)
+    rows, k, T = 200, 1024, 20
+    raw = synth.weight(Q6K, rows, k, 1, True)
+    w, x_h = be.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
+    x, y = be.f32_buf(x_h), out_buf(be, T * rows)
+    be.qmatmul(w, x, y)  # makes the space
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+    used, limit = be.buffer_usage(DOMAIN_DEVICE)
+    for n in (limit, limit + 1, 2**64 - 1 - limit, 2**64 - 300):
+        with pytest.raises(BackendError):
+            be.alloc(n)
+        assert be.buffer_usage(DOMAIN_DEVICE)[0] == used
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        graph.launch()
+        check(be, y, T, Q6K, raw, rows, k, x_h, "replayed")
+    graph.close()
+    be.close()
