@@ -359,6 +359,24 @@ void budget_charge(mdma_ctx *ctx, int domain, uint64_t bytes, const char *what) 
 
 void budget_refund(mdma_ctx *ctx, int domain, uint64_t bytes) { ctx->budget[domain].used -= bytes; }
 
+// hipMalloc, for a caller's buffer or one the context cannot do without: where
+// the device has no room, the split partials' space comes second, given back if
+// the request then fits. A failed attempt's error is taken out of the
+// runtime's last-error slot, where it would meet the next launch's check.
+static hipError_t device_malloc(mdma_ctx *ctx, void **p, uint64_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  size_t fr = 0, tot = 0;
+  const uint64_t held = split_parts_held(ctx);
+  if (e != hipErrorOutOfMemory || !held || hipMemGetInfo(&fr, &tot) != hipSuccess || bytes > fr + held ||
+      !drop_split_parts(ctx))
+    return e;
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 // Replace a context-owned device buffer (buf, cap units of `unit` bytes)
 // by one of new_cap units: charged to the device budget first
 // (BufferBudget::allocate; a refusal leaves the old buffer as it was), the
@@ -387,7 +405,7 @@ static T *regrow(mdma_ctx *ctx, T *&buf, uint64_t &cap, uint64_t new_cap, uint64
     }
   }
   void *p = nullptr;
-  e = hipMalloc(&p, new_bytes);
+  e = device_malloc(ctx, &p, new_bytes);
   if (e != hipSuccess) {
     budget_refund(ctx, MDMA_DOMAIN_DEVICE, new_bytes);
     hip_check(e, what);
@@ -724,8 +742,7 @@ int mdma_gfx950_alloc(mdma_ctx *ctx, uint64_t bytes, int pool, mdma_buf **out) {
     budget_charge(ctx, MDMA_DOMAIN_DEVICE, charged, "alloc");
     void *d = nullptr;
     hipError_t e = hipSetDevice(ctx->device);
-    if (e == hipSuccess) e = hipMalloc(&d, rounded);
-    if (e == hipErrorOutOfMemory && drop_split_parts(ctx)) e = hipMalloc(&d, rounded);
+    if (e == hipSuccess) e = device_malloc(ctx, &d, rounded);
     if (e != hipSuccess) {
       budget_refund(ctx, MDMA_DOMAIN_DEVICE, charged);
       hip_check(e, "hipMalloc");

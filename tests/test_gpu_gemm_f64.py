@@ -172,3 +172,25 @@ def test_refused_allocation_leaves_partials_and_graphs():
         check(be, y, T, Q6K, raw, rows, k, x_h, "replayed")
     graph.close()
     be.close()
+
+
+@pytest.mark.parametrize("partials", [False, True])
+def test_launches_after_an_allocation_the_device_refused(partials):
+    # The refused hipMalloc's error does not meet the next launch, and the
+    # partials' space, which could not have made the room, stays.
+    be = Gfx950Backend(0)
+    rows, k, T = 200, 1024, 20
+    raw = synth.weight(Q6K, rows, k, 1, True)
+    w, x_h = be.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
+    x, y = be.f32_buf(x_h), out_buf(be, T * rows)
+    if partials:
+        be.qmatmul(w, x, y)
+    used = be.buffer_usage(DOMAIN_DEVICE)[0]
+    with pytest.raises(BackendError, match="hipMalloc"):
+        be.alloc(1 << 50)
+    assert be.buffer_usage(DOMAIN_DEVICE)[0] == used
+    be.silu_mul(x, x, x)  # a launch whose check reads the last error
+    be.upload(x, 0, x_h)
+    be.qmatmul(w, x, y)
+    check(be, y, T, Q6K, raw, rows, k, x_h, "after the refusal")
+    be.close()
