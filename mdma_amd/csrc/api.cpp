@@ -318,29 +318,21 @@ void no_capture(mdma_ctx *ctx, const char *what) {
 // What giving the split launches' partials back would free now: nothing under
 // a capture or in an allocation-free call.
 static uint64_t split_parts_held(const mdma_ctx *ctx) {
-  if (ctx->capturing || ctx->fixed_scratch) return 0;
-  uint64_t n = ctx->split_part_cap;
-  for (const auto &o : ctx->split_part_old) n += o.second;
-  return n;
+  return ctx->capturing || ctx->fixed_scratch ? 0 : ctx->split_part_cap;
 }
 
-// Gives them back (they only spread work over the CUs): a caller's allocation
-// that fits in their place comes first. False when there is nothing to give
-// or the stream cannot be drained now.
+// Gives them back (they only spread work over the CUs, and no graph points
+// into them): a caller's allocation that fits in their place comes first.
+// False when there is nothing to give or the stream cannot be drained now.
 static bool drop_split_parts(mdma_ctx *ctx) {
   if (!split_parts_held(ctx)) return false;
-  if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
-  for (; !ctx->split_part_old.empty(); ctx->split_part_old.pop_back()) {
-    if (hipFree(ctx->split_part_old.back().first) != hipSuccess) return false;
-    budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_old.back().second);
-    ctx->buf_epoch++;  // a captured launch points into it
+  if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->split_part) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
-  if (ctx->split_part && hipFree(ctx->split_part) != hipSuccess) return false;
   budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_cap);
-  if (ctx->split_part_captured) ctx->buf_epoch++;
   ctx->split_part = nullptr;
   ctx->split_part_cap = 0;
-  ctx->split_part_captured = false;
   return true;
 }
 
@@ -435,38 +427,23 @@ char *argmax_parts(mdma_ctx *ctx, uint64_t chunks) {
 }
 
 void *split_parts(mdma_ctx *ctx, uint64_t bytes) {
-  if (bytes > ctx->split_part_cap) {
-    if (ctx->capturing || ctx->fixed_scratch) return nullptr;
-    // A captured launch keeps the space it points into (its graph stays
-    // valid); the next one is at least twice as large, so what is kept is
-    // less than what is in use.
-    const bool keep = ctx->split_part_captured;
-    const uint64_t cap = keep ? std::max(bytes, 2 * ctx->split_part_cap) : bytes;
-    const Ledger &l = ctx->budget[MDMA_DOMAIN_DEVICE];
-    const uint64_t used = l.used - (keep ? 0 : ctx->split_part_cap);
-    if (used + cap < used || used + cap > l.limit) return nullptr;
-    if (keep) {
-      ctx->split_part_old.reserve(ctx->split_part_old.size() + 1);
-    } else if (ctx->split_part) {
-      // (What older graphs hold stays: only the space in use is replaced.)
-      if (hipStreamSynchronize(ctx->stream) != hipSuccess || hipFree(ctx->split_part) != hipSuccess) return nullptr;
-      budget_refund(ctx, MDMA_DOMAIN_DEVICE, ctx->split_part_cap);
-      ctx->split_part = nullptr;
-      ctx->split_part_cap = 0;
-    }
-    void *p = nullptr;
-    if (hipMalloc(&p, cap) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    budget_charge(ctx, MDMA_DOMAIN_DEVICE, cap, "split partials growth");
-    if (keep) ctx->split_part_old.emplace_back(ctx->split_part, ctx->split_part_cap);
-    ctx->split_part = static_cast<char *>(p);
-    ctx->split_part_cap = cap;
-    ctx->split_part_captured = false;
+  if (bytes <= ctx->scratch_cap) return ctx->scratch;
+  if (ctx->capturing) return nullptr;
+  if (bytes <= ctx->split_part_cap) return ctx->split_part;
+  if (ctx->fixed_scratch) return nullptr;
+  const Ledger &l = ctx->budget[MDMA_DOMAIN_DEVICE];
+  const uint64_t used = l.used - ctx->split_part_cap;
+  if (used + bytes < used || used + bytes > l.limit) return nullptr;
+  if (ctx->split_part && !drop_split_parts(ctx)) return nullptr;
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
   }
-  if (ctx->capturing) ctx->split_part_captured = true;
-  return ctx->split_part;
+  budget_charge(ctx, MDMA_DOMAIN_DEVICE, bytes, "split partials growth");
+  ctx->split_part = static_cast<char *>(p);
+  ctx->split_part_cap = bytes;
+  return p;
 }
 
 double *ssq_parts(mdma_ctx *ctx, uint64_t n) {
@@ -592,7 +569,6 @@ void mdma_gfx950_destroy(mdma_ctx *ctx) {
   if (ctx->gemm_cnt) (void)hipFree(ctx->gemm_cnt);
   if (ctx->ssq) (void)hipFree(ctx->ssq);
   if (ctx->split_part) (void)hipFree(ctx->split_part);
-  for (auto &o : ctx->split_part_old) (void)hipFree(o.first);
   if (ctx->rope_tab) (void)hipFree(ctx->rope_tab);
   if (ctx->host_ids) (void)hipHostFree(ctx->host_ids);
   (void)hipStreamDestroy(ctx->stream);

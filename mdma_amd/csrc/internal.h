@@ -142,10 +142,8 @@ struct mdma_ctx {
   uint64_t attn_cnt_cap = 0;
   uint32_t *gemm_cnt = nullptr;  // split-K GEMM arrival counters (zero between launches)
   uint64_t gemm_cnt_cap = 0;
-  char *split_part = nullptr;  // partial sums of launches that split K (gemm_f64.hip, gemv_wide)
+  char *split_part = nullptr;  // partial sums of launches that split K (split_parts); never in a graph
   uint64_t split_part_cap = 0;
-  bool split_part_captured = false;  // a captured launch points into it
-  std::vector<std::pair<char *, uint64_t>> split_part_old;  // outgrown, held for the graphs that point into them
   double *ssq = nullptr;  // per-workgroup sums of squares of a residual-stream GEMV (norm fusion)
   uint64_t ssq_cap = 0;
   uint32_t team_grid = 0;  // workgroups of the last row-team launch
@@ -397,9 +395,12 @@ void launch_gemm_f16(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
 constexpr uint64_t F64_MIN_TOKENS = 2;
 bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T,
                      float *glu_y = nullptr);
-// Device space for the partial sums of a launch that splits K, or null where it may not grow now (a
-// capture, an allocation-free call, a full budget or device): the launch then
-// runs unsplit.
+// Device space for the partial sums of a launch that splits K (until the next
+// launch that asks): the context's scratch where it is large enough, else
+// space of its own, which a caller's allocation may take back; null where
+// that may not grow now (an allocation-free call, a full budget or device).
+// A captured launch gets the scratch or nothing: the growth of the scratch
+// ends a graph in any case (buf_epoch), giving the other space back must not.
 void *split_parts(mdma_ctx *ctx, uint64_t bytes);
 void launch_quantize_act(mdma_ctx *ctx, const float *x, uint64_t n, uint64_t group, int8_t *q,
                          float *d, int32_t *sum16);

@@ -101,10 +101,10 @@ def test_partials_space_gives_way_to_the_budget():
 
 @pytest.mark.parametrize("full", [False, True])
 def test_captured_partials_space_outlives_its_growth(full):
-    # A graph that holds the partial tiles' space replays after a larger call
-    # wanted more of it: the space was replaced but kept for the graph, or the
-    # budget had no room and that call ran unsplit. Once a caller's allocation
-    # takes it back, the graph refuses.
+    # A graph of a launch that splits eagerly replays after a larger call
+    # replaced the partial tiles' space, or found no room in the budget for
+    # more of it, and after a caller's allocation took the space back: no graph
+    # points into it.
     be = Gfx950Backend(0)
     be.set_buffer_budget(device=512 << 20)
     rows, k, T, big_rows, big_T = 200, 1024, 20, 2100, 100
@@ -126,8 +126,11 @@ def test_captured_partials_space_outlives_its_growth(full):
     now, limit = be.buffer_usage(DOMAIN_DEVICE)
     assert (now == used) if full else (now > used)
     rest = be.alloc((limit - now) // 4096 * 4096 + 8192)
-    with pytest.raises(BackendError):
+    assert be.buffer_usage(DOMAIN_DEVICE)[0] - rest.len < now  # the space went
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
         graph.launch()
+        check(be, y, T, Q6K, raw, rows, k, x_h, "replayed without the space")
     rest.close()
     if filler:
         filler.close()
@@ -149,6 +152,26 @@ def test_nan_and_infinity_stay_in_their_token(backend):
     assert np.array_equal(got[keep], ref[keep])
     assert np.isnan(got[3]).all() and not np.isfinite(got[18]).any()
 
+
+
+def test_captured_launch_splits_into_the_scratch():
+    # With room in the reserved scratch a captured launch splits as an eager
+    # one does: the same bits, whatever else uses the scratch in between.
+    be = Gfx950Backend(0)
+    rows, k, T = 300, 1024, 70
+    raw = synth.weight(Q6K, rows, k, 1, True)
+    w, x_h = be.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
+    x, y, e = be.f32_buf(x_h), out_buf(be, T * rows), out_buf(be, T * rows)
+    be.qmatmul(w, x, e)
+    be.reserve_scratch(64 << 20)
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        be.greedy(x)  # writes the scratch
+        graph.launch()
+        assert np.array_equal(be.download_f32(y), be.download_f32(e))
+    graph.close()
+    be.close()
 
 
 def test_refused_allocation_leaves_partials_and_graphs():
