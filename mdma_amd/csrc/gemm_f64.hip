@@ -41,6 +41,7 @@ constexpr uint32_t BK = 256;           // columns of a block
 constexpr uint32_t XP = BK + 4;        // LDS pitch of a token's block (floats): 16 tokens on distinct banks
 constexpr int RW = 2;                  // 16-row tiles per wave
 constexpr uint32_t TR = 4 * RW * 16;   // rows of a workgroup's tile (gated: half gate, half up)
+constexpr uint64_t F64_LOOP_TOKENS = 128;  // most tokens taken 8 at a time where there is no space for partials
 
 struct F64Args {
   const uint8_t *w[3];
@@ -329,15 +330,17 @@ __global__ __launch_bounds__(256) void gemm_f64_merge_kernel(F64Args a, uint32_t
   store_tile<TW, GLU>(a, p, acc, yg, threadIdx.x >> 6, threadIdx.x & 63);
 }
 
+// Workgroups over a.units (tile, block) pairs, and the bytes of their partials.
+uint32_t grid_of(mdma_ctx *ctx, int tw, uint32_t units) {
+  return std::min(units, (uint32_t)ctx->cu_count * (tw <= 2 ? 2 : 1));
+}
+uint64_t part_bytes(uint32_t G, int tw) { return (uint64_t)G * 2 * RW * tw * 4 * 256 * 8; }
+
 template <int DT, int TW, bool GLU>
 void launch(mdma_ctx *ctx, F64Args &a, uint32_t tiles, float *yg) {
-  const uint32_t units = tiles * a.nb;  // (checked to fit by the caller)
-  uint32_t G = (uint32_t)ctx->cu_count * (TW <= 2 ? 2 : 1);
-  if (G > units) G = units;
-  a.units = units;
-  a.part = tiles % G ? static_cast<double *>(split_parts(ctx, (uint64_t)G * 2 * RW * TW * 4 * 256 * 8)) : nullptr;
+  uint32_t G = grid_of(ctx, TW, a.units);
   if (a.part) {
-    a.per_q = units / G, a.per_r = units % G;
+    a.per_q = a.units / G, a.per_r = a.units % G;
   } else {  // runs of whole tiles
     const uint32_t n = (tiles + G - 1) / G;
     G = (tiles + n - 1) / n;
@@ -547,7 +550,25 @@ bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
   a.nt = (uint32_t)((t16 + 3) / 4);
   const int tw = (int)((t16 + a.nt - 1) / a.nt);
   if (row_tiles * a.nt * a.nb > 0x7fffffffull) return false;
-  const uint32_t tiles = (uint32_t)row_tiles * a.nt;
+  const uint32_t tiles = (uint32_t)row_tiles * a.nt, G = grid_of(ctx, tw, a.units = tiles * a.nb);
+  if (tiles % G) {
+    a.part = static_cast<double *>(split_parts(ctx, part_bytes(G, tw)));
+    // No space for partials and tiles for less than half the CUs: 8 tokens at
+    // a time, whose kernel needs none. us, 8-token launches / whole tiles:
+    // 4096x4096 Q6_K T = 9: 20.3 / 94, 64 (32 tiles): 104 / 288; 4096x14336 T =
+    // 16: 82 / 349; gate/up 2x14336x4096 Q4_K (224 tiles) T = 16: 119 / 90. From
+    // about 200 tokens the launches add up to a tile's time even over few rows.
+    if (!a.part && T <= F64_LOOP_TOKENS && 2 * (uint64_t)tiles < (uint64_t)ctx->cu_count) {
+      for (uint64_t t0 = 0; t0 < T; t0 += 8) {
+        const uint64_t tn = std::min<uint64_t>(8, T - t0);
+        GemvJob js[3];
+        for (int i = 0; i < n_jobs; i++) js[i] = jobs[i], js[i].y += js[i].y ? t0 * js[i].n_out : 0;
+        if (glu) launch_gemv_f32_gated(ctx, js[0], js[1], x + t0 * j0.n_in, tn, glu_y + t0 * j0.n_out);
+        else launch_gemv_f32(ctx, js, n_jobs, x + t0 * j0.n_in, tn);
+      }
+      return true;
+    }
+  }
 #define MDMA_F64_GO(DT)                                 \
   if (glu) launch_tw<DT, true>(ctx, a, tw, tiles, glu_y); \
   else launch_tw<DT, false>(ctx, a, tw, tiles, nullptr)

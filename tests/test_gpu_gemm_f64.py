@@ -62,11 +62,13 @@ def test_gate_up_at_tile_edges(backend, dtype, k, T):
     assert np.allclose(got[:T * rows], ref, rtol=6 * 2.0**-24, atol=0)
 
 
-def test_captured_launch_without_partials_space(backend):
-    # Under capture the partial tiles' space cannot be made: the launch runs
-    # unsplit, and its replays give the eager results.
+@pytest.mark.parametrize("rows,T", [(200, 70), (200, 9), (200, 128), (200, 129), (16700, 12)])
+def test_captured_launch_without_partials_space(rows, T):
+    # Under capture the partial tiles' space cannot be made: the launch takes 8
+    # tokens at a time (and a last one alone), or whole tiles where these are
+    # many or the tokens more than 128, and its replays give the eager results.
     be = Gfx950Backend(0)
-    rows, k, T = 200, 1024, 70
+    k = 1024
     raw = synth.weight(Q6K, rows, k, 1, True)
     w, x_h = be.upload_weight(raw, Q6K, (rows, k)), synth.normal_f32(T * k, 2)
     x, y = be.f32_buf(x_h), out_buf(be, T * rows)
@@ -76,6 +78,28 @@ def test_captured_launch_without_partials_space(backend):
         be.qmatmul(w, x, be.alloc(T * rows * 4))  # eager: makes the space; the graph does not hold it
         graph.launch()
         check(be, y, T, Q6K, raw, rows, k, x_h, "captured")
+    graph.close()
+    be.close()
+
+
+@pytest.mark.parametrize("T", [9, 23])
+def test_captured_gate_up_without_partials_space(T):
+    be = Gfx950Backend(0)
+    rows, k = 150, 1024
+    w = [be.upload_weight(synth.weight(Q4K, rows, k, s, True), Q4K, (rows, k)) for s in (5, 6)]
+    x = be.f32_buf(synth.normal_f32(T * k, T) * 0.1)
+    g, u, want = (be.alloc(T * rows * 4) for _ in range(3))
+    y = out_buf(be, T * rows)
+    graph = be.capture(lambda: be.ffn_gate_up(w[0], w[1], x, g, u, y))
+    be.ffn_gate_up(w[0], w[1], x, g, u, want)
+    ref = be.download_f32(want)
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        graph.launch()
+        got = be.download_f32(y)
+        assert np.all(got[T * rows:] == CANARY)
+        # Both are sums in f64 rounded once, then silu_mul's own roundings.
+        assert np.allclose(got[:T * rows], ref, rtol=6 * 2.0**-24, atol=0)
     graph.close()
     be.close()
 
