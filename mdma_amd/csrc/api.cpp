@@ -415,7 +415,7 @@ char *scratch(mdma_ctx *ctx, uint64_t bytes) {
 
 char *q8_buffer(mdma_ctx *ctx, uint64_t bytes) {
   if (bytes <= ctx->q8_cap) return ctx->q8;
-  const uint64_t cap = bytes < (1u << 20) ? (1u << 20) : bytes + bytes / 4;
+  const uint64_t cap = bytes < Q8_BUFFER_MIN ? Q8_BUFFER_MIN : bytes + bytes / 4;
   ctx->q8_valid = false;
   return regrow(ctx, ctx->q8, ctx->q8_cap, cap, 1, "int8 activation buffer growth");
 }

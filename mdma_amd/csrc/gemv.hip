@@ -802,9 +802,15 @@ uint64_t gemm_input_bytes(uint64_t n) {
   return (n + 255) / 256 * 256 + (n / 32 * 4 + 255) / 256 * 256 + (n / 16 * 4 + 255) / 256 * 256;
 }
 
+void q8_slots_at(char *s, uint64_t n, int8_t **qx, float **dx, int32_t **s16) {
+  const uint64_t qb = (n + 255) / 256 * 256, db = (n / 256 * 4 + 255) / 256 * 256;
+  *qx = reinterpret_cast<int8_t *>(s);
+  *dx = reinterpret_cast<float *>(s + qb);
+  *s16 = reinterpret_cast<int32_t *>(s + qb + db);
+}
+
 void q8_slots(mdma_ctx *ctx, uint64_t T, uint64_t n_in, int8_t **qx, float **dx, int32_t **s16) {
   const uint64_t n = T * n_in;
-  const uint64_t qb = (n + 255) / 256 * 256, db = (n / 256 * 4 + 255) / 256 * 256;
   char *s;
   if (ctx->fixed_scratch) {  // an allocation-free call: its fixed buffer
     if (q8_slot_bytes(n) > ctx->fixed_cap) fail(MDMA_ERR_BUFFER_BUDGET, "int8 activations exceed the fixed scratch");
@@ -812,9 +818,16 @@ void q8_slots(mdma_ctx *ctx, uint64_t T, uint64_t n_in, int8_t **qx, float **dx,
   } else {
     s = q8_buffer(ctx, q8_slot_bytes(n));
   }
-  *qx = reinterpret_cast<int8_t *>(s);
-  *dx = reinterpret_cast<float *>(s + qb);
-  *s16 = reinterpret_cast<int32_t *>(s + qb + db);
+  q8_slots_at(s, n, qx, dx, s16);
+}
+
+// Whether x's int8 form is in the activation buffer, or goes there without
+// growing it past what 16 tokens would.
+bool q8_fits(const mdma_ctx *ctx, const float *x, uint64_t T, uint64_t n_in) {
+  const uint64_t n = T * n_in;
+  if (ctx->q8_valid && ctx->q8_x == x && ctx->q8_n == n && ctx->q8_n_in == n_in) return true;
+  if (ctx->fixed_scratch) return q8_slot_bytes(n) <= ctx->fixed_cap;
+  return q8_slot_bytes(n) <= std::max<uint64_t>(ctx->q8_cap, ctx->q8 ? 0 : Q8_BUFFER_MIN);
 }
 
 void q8_mark(mdma_ctx *ctx, const float *x, uint64_t T, uint64_t n_in) {

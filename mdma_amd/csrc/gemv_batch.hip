@@ -1681,11 +1681,7 @@ void wide_launch(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, c
   uint32_t G = tiles;
   ws.items = tiles * ws.nch;
   ws.per_q = ws.nch, ws.per_r = 0;
-  if (tiles <= (uint32_t)ctx->cu_count) {
-    const uint32_t g2 = std::min(ws.items, 2 * (uint32_t)ctx->cu_count);
-    ws.part = static_cast<float *>(split_parts(ctx, (uint64_t)ws.items * NT * 4 * 256 * 4));
-    if (ws.part && g2 > tiles) G = g2, ws.per_q = ws.items / G, ws.per_r = ws.items % G;
-  }
+  if (ws.part) G = std::min(ws.items, 2 * (uint32_t)ctx->cu_count), ws.per_q = ws.items / G, ws.per_r = ws.items % G;
   if (ws.s.j[0].dots)
     gemv_wide<W, NT, GLU, true><<<dim3(G), dim3(256), 0, ctx->stream>>>(ws, qx, dx);
   else
@@ -1761,11 +1757,28 @@ bool launch_gemv_wide(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated
     j.tiles = (j.n_out + (gated ? 31 : 63)) / (gated ? 32 : 64);
     if (i < ws.s.n) tiles += j.tiles;
   }
+  // The chunk sums of split tiles, and x's int8 form where the activation
+  // buffer would have to grow for more than 16 tokens (which a full budget
+  // refuses and which ends graphs), in space that needs neither. Without it
+  // the 16-token launches: unsplit, few tiles walk all their chunks in turn
+  // (us, unsplit / 16-token launches: 4096x14336 Q6_K T = 17 82 / 32, 4096x4096
+  // T = 63 38.8 / 35.2).
+  const uint32_t nt = (uint32_t)tiles, cus = (uint32_t)ctx->cu_count;
+  const uint64_t pb = nt <= cus && std::min<uint64_t>(tiles * ws.nch, 2 * cus) > nt
+                          ? tiles * ws.nch * ((T + 15) / 16) * 4 * 256 * 4 : 0;
+  const uint64_t sb = q8_fits(ctx, x, T, n_in) ? 0 : (q8_slot_bytes(T * n_in) + 255) / 256 * 256;
+  char *sp = pb + sb ? static_cast<char *>(split_parts(ctx, sb + pb)) : nullptr;
+  if (pb + sb && !sp) return false;
   int8_t *qx;
   float *dx;
   int32_t *s16;
-  quantize_into_scratch(ctx, x, T, n_in, &qx, &dx, &s16);
-  const uint32_t nt = (uint32_t)tiles;
+  if (sb) {
+    q8_slots_at(sp, T * n_in, &qx, &dx, &s16);
+    launch_quantize_act(ctx, x, T * n_in, 256, qx, dx, s16);
+  } else {
+    quantize_into_scratch(ctx, x, T, n_in, &qx, &dx, &s16);
+  }
+  if (pb) ws.part = reinterpret_cast<float *>(sp + sb);
 #define MDMA_WIDE_GO(W)                                  \
   if (gated) wide_fmt<W, true>(ctx, ws, nt, qx, dx);     \
   else wide_fmt<W, false>(ctx, ws, nt, qx, dx)

@@ -202,7 +202,9 @@ uint64_t gemm_input_bytes(uint64_t n);
 // Scratch space of at least `bytes` on the context's device; growing it
 // synchronizes the stream (callers hold the context lock).
 char *scratch(mdma_ctx *ctx, uint64_t bytes);
-// The int8-activation buffer (grown like scratch; growth drops the cached x).
+// The int8-activation buffer (grown like scratch, from Q8_BUFFER_MIN bytes;
+// growth drops the cached x).
+constexpr uint64_t Q8_BUFFER_MIN = 1u << 20;
 char *q8_buffer(mdma_ctx *ctx, uint64_t bytes);
 // Device space for `chunks` partial results of the two-pass argmax (grown
 // like scratch).
@@ -329,6 +331,8 @@ bool launch_gemv_i8_normed(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const
 // Slots of the int8-activation buffer for x [T, n_in] (int8 values, per-256
 // scales, sums of 16), and marking them as holding x's quantization.
 void q8_slots(mdma_ctx *ctx, uint64_t T, uint64_t n_in, int8_t **qx, float **dx, int32_t **s16);
+void q8_slots_at(char *s, uint64_t n, int8_t **qx, float **dx, int32_t **s16);
+bool q8_fits(const mdma_ctx *ctx, const float *x, uint64_t T, uint64_t n_in);
 void q8_mark(mdma_ctx *ctx, const float *x, uint64_t T, uint64_t n_in);
 // The buffer holds the int8 form of the one row x of n values.
 bool q8_holds(mdma_ctx *ctx, const float *x, uint64_t n);

@@ -63,7 +63,7 @@ def test_gate_up_equal_staged(i8, dtype, rows, k, T):
 
 
 def test_captured_and_over_budget_run_unsplit():
-    # No space for the split tiles' chunk sums: the same bits.
+    # No space for the split tiles' chunk sums: 16 tokens a launch, the same bits.
     be = Gfx950Backend(0)
     be.set_act_mode(bm.ACT_I8)
     rows, k, T = 256, 2048, 40
@@ -88,5 +88,47 @@ def test_captured_and_over_budget_run_unsplit():
     be.qmatmul(w, x, y)
     assert np.array_equal(be.download_f32(y), ref)
     rest.close()
+    graph.close()
+    be.close()
+
+
+def test_int8_buffer_is_not_grown_past_16_tokens():
+    # 63 tokens of 14336 values do not fit the int8 buffer's first megabyte,
+    # 16 do: the call neither grows it (under a capture or a full budget it
+    # could not, and growth ends graphs) nor refuses.
+    be = Gfx950Backend(0)
+    be.set_act_mode(bm.ACT_I8)
+    be.set_buffer_budget(device=64 << 20)
+    rows, k, T = 100, 14336, 63
+    w = be.upload_weight(synth.weight(Q6K, rows, k, 1, True), Q6K, (rows, k))
+    x, y, want = be.f32_buf(synth.normal_f32(T * k, 2)), be.alloc(T * rows * 4), be.alloc(T * rows * 4)
+    be.reserve_scratch(1 << 19)
+    be.set_batch_kernel(bm.BATCH_STAGED)
+    be.qmatmul(w, x, want)
+    ref = be.download_f32(want)
+    be.set_batch_kernel(bm.BATCH_AUTO)
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+
+    def same(call):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        call()
+        assert np.array_equal(be.download_f32(y), ref)
+
+    used, limit = be.buffer_usage(bm.DOMAIN_DEVICE)
+    rest = be.alloc(limit - used)
+    for _ in range(2):
+        same(lambda: be.qmatmul(w, x, y))  # a full budget: 16 tokens a launch
+        same(graph.launch)
+    rest.close()
+    for _ in range(2):
+        same(lambda: be.qmatmul(w, x, y))  # one launch, its int8 form beside the chunk sums
+        same(graph.launch)
+    assert be.buffer_usage(bm.DOMAIN_DEVICE)[0] > used
+    be.reserve_scratch(8 << 20)
+    graph.close()
+    graph = be.capture(lambda: be.qmatmul(w, x, y))  # one launch, in the scratch
+    for _ in range(3):
+        same(graph.launch)
+        same(lambda: be.qmatmul(w, x, y))
     graph.close()
     be.close()
