@@ -126,7 +126,7 @@ struct Unit64<DT_Q6_K> {
 };
 
 // Q8_0: units (blocks) g and g + 4 of the 8 in a 256-column block; units
-// past the row's end count as zero weights.
+// past the row's end count as zero weights, and zero x (zero_tail).
 template <>
 struct Unit64<DT_Q8_0> {
   uint4 a[2], b[2];
@@ -201,6 +201,17 @@ __device__ __forceinline__ void store_tile(const F64Args &a, const Place<TW> &p,
     }
 }
 
+// x past the row's end of its last, partial block (Q8_0 only): zeroes over
+// what the DMA read there (the row's last columns again), which a zero weight
+// would turn into NaN where it is infinite.
+template <int DT, int N>
+__device__ __forceinline__ void zero_tail(float (*xb)[XP], uint32_t b, uint32_t n_in, uint32_t lane) {
+  if (DT != DT_Q8_0 || (b + 1) * BK <= n_in) return;
+  if (b * BK + 4 * lane < n_in) return;
+#pragma unroll
+  for (int r = 0; r < N; r++) *reinterpret_cast<v4f *>(&xb[r][4 * lane]) = v4f{0, 0, 0, 0};
+}
+
 __device__ __forceinline__ uint32_t run_start(const F64Args &a, uint32_t w) { return w * a.per_q + min(w, a.per_r); }
 
 template <int DT, int TW, bool GLU>
@@ -249,6 +260,7 @@ __global__ __launch_bounds__(256, TW <= 2 ? 2 : 1) void gemm_f64_kernel(F64Args 
         cur[i].coef(b, g, a.n_in);
       }
       lds_wait_dma();
+      zero_tail<DT, 4 * TW>(&xs[b & 1][wave * (4 * TW)], b, a.n_in, lane);
       lds_barrier();  // every wave's x of block b is in LDS; block b - 1's reads are done
       if (b + 1 < b1) {
         load_x(b + 1, (b + 1) & 1);
@@ -423,6 +435,7 @@ __global__ __launch_bounds__(64 * NW, TT <= 4 ? 4 : 2) void gemv_f64_kernel(F64A
       for (int t = 0; t < NT; t++) acc[i][t] = 0.0;
     for (uint32_t b = wave; b < a.nb; b += NW) {
       lds_wait_dma();
+      zero_tail<DT, TT>(xs[wave][buf], b, a.n_in, lane);
 #pragma unroll
       for (int i = 0; i < R; i++) {
         cur[i] = nxt[i];

@@ -241,3 +241,30 @@ def test_launches_after_an_allocation_the_device_refused(partials):
     be.qmatmul(w, x, y)
     check(be, y, T, Q6K, raw, rows, k, x_h, "after the refusal")
     be.close()
+
+
+@pytest.mark.parametrize("k", [288, 32, 512])
+@pytest.mark.parametrize("T", [2, 4, 8, 20])
+@pytest.mark.parametrize("fused", [False, True])
+def test_infinity_in_a_rows_last_columns(backend, k, T, fused):
+    # A row of blocks that do not fill the last 256 columns: what stands in the
+    # rest is no input. The sums are infinite (NaN for a zero weight), as the
+    # CPU's are.
+    rows = 97
+    raw = synth.weight(Q8, rows, k, 1, True)
+    x_h = synth.normal_f32(T * k, 2).reshape(T, k)
+    x_h[0, k - 1], x_h[T - 1, k - 4] = np.inf, -np.inf
+    w, x, y = backend.upload_weight(raw, Q8, (rows, k)), backend.f32_buf(x_h), out_buf(backend, T * rows)
+    want = ffi.qmatmul(Q8, raw, rows, k, x_h).reshape(T, rows)
+    if fused:
+        g, u = backend.alloc(T * rows * 4), backend.alloc(T * rows * 4)
+        backend.ffn_gate_up(w, w, x, g, u, y)
+        with np.errstate(all="ignore"):
+            want = want / (1 + np.exp(-want)) * want
+    else:
+        backend.qmatmul(w, x, y)
+    got = backend.download_f32(y)[:T * rows].reshape(T, rows)
+    bad = [0, T - 1]
+    assert np.isinf(want[bad]).sum() > rows // 2  # (few weights are zero; silu(-inf) is NaN)
+    assert np.array_equal(got[bad], want[bad], equal_nan=True)
+    assert np.allclose(got[1:T - 1], want[1:T - 1], rtol=1e-4, atol=1e-4)
