@@ -384,7 +384,7 @@ void launch_tw(mdma_ctx *ctx, F64Args &a, int tw, uint32_t tiles, float *yg) {
 // take the sum of their times), so the products and the weights' two VALU
 // operations bound the kernel together, about 33 cycles per 64 weights and 4
 // tokens. us, row teams / here: gate/up 2x14336x4096 Q4_K T = 2: 73 / 38.7,
-// 4: 135 / 45, 8: 267 / 62 (the 16-token tile: 83); 4096x14336 Q6_K 40 / 24.4,
+// 4: 135 / 41, 8: 267 / 62 (the 16-token tile: 83); 4096x14336 Q6_K 40 / 24.4,
 // 66 / 26.6, 134 / 41.5. Lane l supplies
 // row l % 16 of the tile and token l % 4, both for k group l / 16, as above,
 // and holds the sum of token l / 16, row l % 16.
@@ -393,13 +393,18 @@ void launch_tw(mdma_ctx *ctx, F64Args &a, int tw, uint32_t tiles, float *yg) {
 // rows of gate and the same of up) in turn, so that neighbouring waves read
 // neighbouring 64 bytes of a row, and add their sums in wave order through
 // LDS. x comes by DMA into the wave's own double buffer: no barrier but the
-// one per tile. The next block's loads are in flight behind the current one's
-// products, across tiles too.
+// one per tile (a second where the sums have one buffer: gated 3 and 4 tokens,
+// for which a second workgroup fits the CU's LDS then, gate/up 2x14336x4096 at 4
+// tokens 45.7 -> 41.2 us, 2x5632x2048 14.5 -> 12.1). The next block's loads
+// are in flight behind the current one's products, across tiles too.
+constexpr int f64_waves(int TT) { return TT <= 4 ? 16 : 8; }  // on a CU
 template <int DT, int TT, bool GLU, int NW>
-__global__ __launch_bounds__(64 * NW, TT <= 4 ? 4 : 2) void gemv_f64_kernel(F64Args a, float *yg) {
-  constexpr int R = GLU ? 2 : 1, NT = (TT + 3) / 4, RB = TT <= 4 ? 2 : 1;
+__global__ __launch_bounds__(64 * NW, f64_waves(TT) / 4) void gemv_f64_kernel(F64Args a, float *yg) {
+  constexpr int R = GLU ? 2 : 1, NT = (TT + 3) / 4, RB = TT <= 4 && !(GLU && TT == 4) ? 2 : 1;
   __shared__ __attribute__((aligned(16))) float xs[NW][2][TT][XP];
   __shared__ __attribute__((aligned(16))) double red[RB][NW][R * NT][64];
+  // As many workgroups on a CU as launch_small's grid counts on.
+  static_assert((sizeof(xs) + sizeof(red)) * (f64_waves(TT) / NW) <= 160 * 1024, "LDS");
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t g = lane / 16, l16 = lane % 16;
   const uint32_t tiles = a.units;
@@ -502,7 +507,7 @@ __global__ __launch_bounds__(64 * NW, TT <= 4 ? 4 : 2) void gemv_f64_kernel(F64A
 
 template <int DT, int TT, bool GLU, int NW>
 void launch_small(mdma_ctx *ctx, F64Args &a, float *yg) {
-  const uint32_t G = std::min(a.units, (uint32_t)ctx->cu_count * (TT <= 4 ? 16 : 8) / NW);
+  const uint32_t G = std::min(a.units, (uint32_t)ctx->cu_count * f64_waves(TT) / NW);
   gemv_f64_kernel<DT, TT, GLU, NW><<<dim3(G), dim3(64 * NW), 0, ctx->stream>>>(a, yg);
   hip_check(hipGetLastError(), "gemv_f64 launch");
 }
