@@ -520,6 +520,15 @@ __device__ __forceinline__ float quarter_sum(float v) {
   return __builtin_bit_cast(float, (uint32_t)c[0]) + __builtin_bit_cast(float, (uint32_t)c[1]);
 }
 
+// exp2(d (c_hi + c_lo)) for a finite d, the product's rounding put back: the
+// factors of whole sums, where the rounding of an exponent of 10 alone would
+// be 5 units of the last place.
+__device__ __forceinline__ float exp2_scaled(float d, float c_hi, float c_lo) {
+  const float t = d * c_hi, e = __builtin_fmaf(d, c_lo, __builtin_fmaf(d, c_hi, -t));
+  const float r = __builtin_amdgcn_exp2f(t);
+  return __builtin_fmaf(r, 0.693147181f * e, r);
+}
+
 template <int G, int HD>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restrict__ q, const uint16_t *__restrict__ K,
                                                            const uint16_t *__restrict__ V, float *__restrict__ o,
@@ -656,7 +665,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     mx = quarter_max(mx);
     if (__any(mx > m + slack)) {  // (also the first visible tile, m = -inf)
       const float mn = fmaxf(m, mx);
-      const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * c_hi);
+      const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : exp2_scaled(m - mn, c_hi, c_lo);
       l *= al;
 #pragma unroll
       for (int n = 0; n < ND; n++) O[n] *= al;
@@ -747,9 +756,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
           continue;
         }
         const float mn = fmaxf(M, mc[i]);  // finite: chunk 0's M is
-        const float da = M - mn, db = mc[i] - mn;
-        const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(da, c_hi, da * c_lo));
-        const float b = mc[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(__builtin_fmaf(db, c_hi, db * c_lo));
+        const float a = exp2_scaled(M - mn, c_hi, c_lo);
+        const float b = mc[i] == -INFINITY ? 0.f : exp2_scaled(mc[i] - mn, c_hi, c_lo);
         L = L * a + lc[i] * b;
 #pragma unroll
         for (int n = 0; n < ND; n++) OA[n] = OA[n] * a + Oc[i][n] * b;

@@ -273,3 +273,44 @@ def test_captured_few_queries_take_the_per_query_kernel(backend):
         np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-6)
         assert np.array_equal(got[:few], backend.download_f32(o7))
     graph.close()
+
+
+@pytest.mark.parametrize("hd,nq,nkv", [(128, 8, 2), (64, 8, 8)])
+def test_prompt_attention_rescales_without_bias(backend, hd, nq, nkv):
+    # 2^d keys of score 0 and value 0, then one of d octaves and a bit more and
+    # value 1: the old sums, rescaled by 2^-d, weigh as much as the last key.
+    # Each output's own roundings are a few u = 2^-24 either way (the score of
+    # 10 octaves alone up to 5, the exponentials, sums and division 1 each);
+    # over queries and heads of many different scores they cancel.
+    n_q, kv_len, d = 96, 1024, 9.5
+    q = np.zeros((n_q, nq, hd), np.float32)
+    want_s = d + np.linspace(0.0, 0.5, n_q * nq).reshape(n_q, nq)  # the last key's score in octaves
+    k = np.zeros((kv_len, nkv, hd), np.float32)
+    k[kv_len - n_q - 1, :, 0] = 1.0
+    q[:, :, 0] = (want_s * np.log(2.0) * np.sqrt(hd)).astype(np.float32)
+    v = np.zeros((kv_len, nkv, hd), np.float32)
+    v[kv_len - n_q - 1] = 1.0
+    kb, vb, o = backend.alloc(k.size * 2), backend.alloc(v.size * 2), backend.alloc(q.size * 4)
+    backend.upload(kb, 0, k.astype(np.float16))
+    backend.upload(vb, 0, v.astype(np.float16))
+    qb = backend.f32_buf(q)
+    w = np.exp(q[:, :, 0].astype(np.float64) / np.sqrt(hd))
+    seen = (kv_len - n_q + np.arange(n_q))[:, None]  # keys of score 0 that a query sees
+    want = w / (w + seen)
+
+    def check():
+        got = backend.download_f32(o).reshape(n_q, nq, hd)[:, :, 0].astype(np.float64)
+        err = (got - want) / want
+        assert np.abs(err).max() < 8 * 2.0**-24
+        assert abs(err.mean()) < 0.6 * 2.0**-24, err.mean() * 2.0**24
+
+    def call():
+        backend.attn(qb, KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
+
+    call()  # key chunks: the factor is the merge's
+    check()
+    graph = backend.capture(call)  # one chunk: the loop's
+    backend.upload(o, 0, np.zeros(q.size, np.float32))
+    graph.launch()
+    check()
+    graph.close()
