@@ -488,13 +488,17 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // 7 tiles 23.3).
 constexpr double ATT_MERGE_TILES = 0.25;
 // Queries from which it is the faster kernel: any prompt of 64, and from 8
-// where the per-query kernel's K/V reads add up (us, per query / here, 32
-// heads: 48 queries over 3900 keys 98 / 27.5, 16 over 1500 20.4 / 15.1, 8 over
-// 3900 25.6 / 20.9, 16 over 500 11.4 / 11.3, 16 over 100 6.9 / 8.1; 20 heads of
-// G = 1: 8 over 1000 11.9 / 14.9). Under a capture or in a fixed scratch, where
-// the key chunks are not made, few queries stay with the per-query kernel: one
-// workgroup a KV head would walk all the tiles in turn.
-constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_PREFILL_PAIRS = 16384;
+// where the rows (queries times query heads) fill workgroups and their keys
+// add up to more than the launch's chain of tiles and merge. us, per query /
+// here, 128 dims; 32 heads, 8 KV: 48 queries over 3900 keys 98 / 27.5, 12 over
+// 1400 18.5 / 15.9, 8 over 3300 25.5 / 20.6; 20 heads, G = 1: 20 over 1700 27.4 /
+// 18.7; 8 heads, G = 8 and 1: 32 over 2100 22.6 / 17.9 and 23.6 / 17.5; 64
+// dims, G = 1: 16 heads, 20 over 2300 26 / 12. Below the line 32 heads, 16 KV:
+// 8 over 2048 17.1 / 17.7; 8 heads: 16 over 3900 18.0 / 20.7, 8 over 2048 10.0 / 16.1.
+// Under a capture or in a fixed scratch, where the key chunks are not made,
+// few queries stay with the per-query kernel: one workgroup a KV head would
+// walk all the tiles in turn.
+constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_FEW_ROWS = 160, ATT_FEW_WORK = 9 << 16;
 
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
@@ -1475,6 +1479,61 @@ void launch_rope_kv_write(mdma_ctx *ctx, float *q, uint64_t q_heads, const float
 }
 
 namespace {
+// attn_prefill_kernel's launch: blocks of queries, and key chunks of ct tiles,
+// about two workgroups per CU (what stays resident) over the call's tile
+// work, at least two tiles each and long enough for the merge.
+struct PromptPlan {
+  uint64_t nqb, ct, n_ch, part_bytes;
+};
+PromptPlan prompt_plan(const mdma_ctx *ctx, uint64_t n_q, uint64_t kv_len, uint64_t hd, uint64_t n_kv_heads, uint64_t G) {
+  const uint64_t QT = 64 / G, nqb = (n_q + QT - 1) / QT, pre = kv_len - n_q;
+  uint64_t units = 0, max_t = 0;
+  for (uint64_t b = 0; b < nqb; b++) {
+    const uint64_t t = (pre + std::min((b + 1) * QT, n_q) - 1) / 64 + 1;
+    units += t;
+    max_t = std::max(max_t, t);
+  }
+  units *= n_kv_heads;
+  const uint64_t cus = ctx->cu_count ? ctx->cu_count : 256;
+  const uint64_t mrg = (uint64_t)std::ceil(std::sqrt(ATT_MERGE_TILES * (double)max_t));  // cheap enough to merge
+  const uint64_t ct = std::max({(uint64_t)2, (units + 2 * cus - 1) / (2 * cus), mrg}), n_ch = (max_t + ct - 1) / ct;
+  return {nqb, ct, n_ch, n_kv_heads * nqb * n_ch * (2 + 4 * (hd / 16)) * 256 * 4};
+}
+
+// Without part and cnt: no key chunks.
+void launch_prompt(mdma_ctx *ctx, const PromptPlan &p, const float *q, const uint16_t *k, const uint16_t *v, float *o,
+                   uint64_t n_q, uint64_t kv_len, uint64_t hd, uint64_t n_q_heads, uint64_t n_kv_heads, float *part,
+                   uint32_t *cnt) {
+  // scale * log2 e in two floats, both positive (a masked score's -inf
+  // times each of them is then -inf).
+  const double c = 1.4426950408889634 / std::sqrt((double)hd);
+  const float c_hi = std::nextafter((float)c, 0.f), c_lo = (float)(c - (double)c_hi);
+  const uint64_t GP = n_q_heads / n_kv_heads, KO = n_q_heads * hd;
+  // Asked for (a16_want_y == o): also the output projection's f16-path
+  // input, into the caller's buffer.
+  const bool want = ctx->a16_want_y == o && ctx->a16_want_bytes >= gemm_f16_input_bytes(n_q, KO);
+  const F16In fin = want ? gemm_f16_input_at(ctx->a16_want_buf, n_q, KO) : F16In{};
+  const dim3 grid((uint32_t)n_kv_heads, (uint32_t)p.nqb, (uint32_t)(part ? p.n_ch : 1));
+#define MDMA_ATTP(GG, HH)                                                                                          \
+  attn_prefill_kernel<GG, HH><<<grid, dim3(256), 0, ctx->stream>>>(                                                \
+      q, k, v, o, (uint32_t)n_q, (uint32_t)(kv_len - n_q), (uint32_t)n_q_heads, (uint32_t)n_kv_heads,              \
+      c_hi, c_lo, (uint32_t)(part ? p.ct : 0), part, cnt, fin)
+  if (hd == 128) {
+    if (GP == 1) MDMA_ATTP(1, 128);
+    else if (GP == 2) MDMA_ATTP(2, 128);
+    else if (GP == 4) MDMA_ATTP(4, 128);
+    else MDMA_ATTP(8, 128);
+  } else {
+    if (GP == 1) MDMA_ATTP(1, 64);
+    else if (GP == 2) MDMA_ATTP(2, 64);
+    else if (GP == 4) MDMA_ATTP(4, 64);
+    else MDMA_ATTP(8, 64);
+  }
+#undef MDMA_ATTP
+  hip_check(hipGetLastError(), "attn prefill launch");
+  if (want) a16_mark(ctx, o, n_q, KO, ctx->a16_want_buf, false);
+}
+
 // rope: RoPE and the new key's cache write folded in (decode only); the
 // cache is written only then. A rope with no k only carries pos_dev (a
 // captured decode step reading its position from device memory, kv_len the
@@ -1486,65 +1545,21 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
   uint16_t *k = const_cast<uint16_t *>(kc), *v = const_cast<uint16_t *>(vc);
   const uint32_t *pos_dev = rope_in ? rope_in->pos_dev : nullptr;
   const uint64_t GP = n_kv_heads ? n_q_heads / n_kv_heads : 0;
-  if (!rope_in && !q8 && !seq_stride && kv_len >= n_q &&
-      (n_q >= ATT_PREFILL_MIN || (n_q >= ATT_PREFILL_FEW && n_q * kv_len >= ATT_PREFILL_PAIRS && !ctx->capturing &&
-                                  !ctx->fixed_scratch)) && (hd == 64 || hd == 128) &&
-      n_kv_heads && GP * n_kv_heads == n_q_heads && (GP == 1 || GP == 2 || GP == 4 || GP == 8) &&
-      kv_len * n_kv_heads * hd < (1ull << 32) && n_kv_heads < 65536) {
-    // A prompt's causal attention on the matrix cores (attn_prefill_kernel).
-    const uint64_t QT = 64 / GP, nqb = (n_q + QT - 1) / QT;
-    // scale * log2 e in two floats, both positive (a masked score's -inf
-    // times each of them is then -inf).
-    const double c = 1.4426950408889634 / std::sqrt((double)hd);
-    const float c_hi = std::nextafter((float)c, 0.f), c_lo = (float)(c - (double)c_hi);
-    const uint32_t pre = (uint32_t)(kv_len - n_q);
-    // Key chunks of ct tiles: about two workgroups per CU (what stays
-    // resident) over the prompt's tile work, at least two tiles each and long
-    // enough for the merge; none when no block has more than ct tiles, under
-    // stream capture or in a fixed scratch.
-    uint64_t units = 0, max_t = 0;
-    for (uint64_t b = 0; b < nqb; b++) {
-      const uint64_t t = (pre + std::min((b + 1) * QT, n_q) - 1) / 64 + 1;
-      units += t;
-      max_t = std::max(max_t, t);
-    }
-    units *= n_kv_heads;
-    const uint64_t cus = ctx->cu_count ? ctx->cu_count : 256;
-    const uint64_t mrg = (uint64_t)std::ceil(std::sqrt(ATT_MERGE_TILES * (double)max_t));  // cheap enough to merge
-    uint64_t ct = std::max({(uint64_t)2, (units + 2 * cus - 1) / (2 * cus), mrg}), n_ch = (max_t + ct - 1) / ct;
-    const uint64_t NV = 2 + 4 * (hd / 16), pbytes = n_kv_heads * nqb * n_ch * NV * 256 * 4;
-    if (n_ch < 2 || ctx->capturing || ctx->fixed_scratch || pbytes > (256ull << 20)) ct = 0, n_ch = 1;
-    float *part = ct ? reinterpret_cast<float *>(scratch(ctx, pbytes)) : nullptr;
-    uint32_t *cnt = ct ? attn_counters(ctx, n_kv_heads * nqb) : nullptr;
-    // Asked for (a16_want_y == o): also the output projection's f16-path
-    // input, into the caller's buffer.
-    const uint64_t KO = n_q_heads * hd;
-    const bool want = ctx->a16_want_y == o && ctx->a16_want_bytes >= gemm_f16_input_bytes(n_q, KO);
-    const F16In fin = want ? gemm_f16_input_at(ctx->a16_want_buf, n_q, KO) : F16In{};
-    const dim3 grid((uint32_t)n_kv_heads, (uint32_t)nqb, (uint32_t)n_ch);
-#define MDMA_ATTP(GG, HH)                                                                                          \
-  attn_prefill_kernel<GG, HH><<<grid, dim3(256), 0, ctx->stream>>>(q, k, v, o, (uint32_t)n_q, pre, (uint32_t)n_q_heads, \
-                                                                   (uint32_t)n_kv_heads, c_hi, c_lo, (uint32_t)ct, part, cnt, \
-                                                                   fin)
-    if (hd == 128) {
-      if (GP == 1) MDMA_ATTP(1, 128);
-      else if (GP == 2) MDMA_ATTP(2, 128);
-      else if (GP == 4) MDMA_ATTP(4, 128);
-      else MDMA_ATTP(8, 128);
-    } else {
-      if (GP == 1) MDMA_ATTP(1, 64);
-      else if (GP == 2) MDMA_ATTP(2, 64);
-      else if (GP == 4) MDMA_ATTP(4, 64);
-      else MDMA_ATTP(8, 64);
-    }
-#undef MDMA_ATTP
-    hip_check(hipGetLastError(), "attn prefill launch");
-    if (want) a16_mark(ctx, o, n_q, KO, ctx->a16_want_buf, false);
+  const float scale = 1.0f / sqrtf((float)hd);
+  // A causal call of one sequence on the matrix cores (attn_prefill_kernel)?
+  const bool prompt = !rope_in && !q8 && !seq_stride && kv_len >= n_q && (hd == 64 || hd == 128) && n_kv_heads &&
+                      GP * n_kv_heads == n_q_heads && (GP == 1 || GP == 2 || GP == 4 || GP == 8) &&
+                      kv_len * n_kv_heads * hd < (1ull << 32) && n_kv_heads < 65536;
+  if (prompt && n_q >= ATT_PREFILL_MIN) {
+    const PromptPlan p = prompt_plan(ctx, n_q, kv_len, hd, n_kv_heads, GP);
+    const bool split = p.n_ch > 1 && !ctx->capturing && !ctx->fixed_scratch && p.part_bytes <= (256ull << 20);
+    float *part = split ? reinterpret_cast<float *>(scratch(ctx, p.part_bytes)) : nullptr;
+    uint32_t *cnt = split ? attn_counters(ctx, n_kv_heads * p.nqb) : nullptr;
+    launch_prompt(ctx, p, q, k, v, o, n_q, kv_len, hd, n_q_heads, n_kv_heads, part, cnt);
     return true;
   }
   const AttnRope *rope = rope_in && rope_in->k ? rope_in : nullptr;
   if (pos_dev && !(seq_stride || n_q == 1)) return false;
-  const float scale = 1.0f / sqrtf((float)hd);
   const uint32_t prefix = (uint32_t)(seq_stride ? kv_len - 1 : kv_len - n_q);
   const uint64_t GQ = n_kv_heads ? n_q_heads / n_kv_heads : 0, C = (hd + 127) / 128;
   // Runs of tiles per (query, KV head): enough workgroups to cover the chip
@@ -1581,6 +1596,24 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     // Counters for the most sub-groups any launch of this shape may take (a
     // captured step and the eager one may choose differently).
     uint32_t *cnt = part_bytes ? attn_counters(ctx, n_q * n_kv_heads * MDMA_ATT_SUB) : nullptr;
+    // A few queries on the matrix cores, where there is room for their key
+    // chunks' partials. The context's buffers are by now what this kernel needs
+    // (a capture of the same call finds them), and they grow no further: the
+    // counters come from the partials' space if there are too few.
+    if (prompt && n_q >= ATT_PREFILL_FEW && n_q * n_q_heads >= ATT_FEW_ROWS &&
+        n_q * n_q_heads * kv_len >= ATT_FEW_WORK && !ctx->capturing && !ctx->fixed_scratch) {
+      const PromptPlan p = prompt_plan(ctx, n_q, kv_len, hd, n_kv_heads, GP);
+      const uint64_t nc = n_kv_heads * p.nqb * CNT_STRIDE;
+      const uint64_t cb = nc <= ctx->attn_cnt_cap ? 0 : (nc * 4 + 255) / 256 * 256;
+      char *sp = p.n_ch > 1 && p.part_bytes <= (256ull << 20) ? static_cast<char *>(split_parts(ctx, cb + p.part_bytes))
+                                                             : nullptr;
+      if (sp) {
+        if (cb) hip_check(hipMemsetAsync(sp, 0, cb, ctx->stream), "attention counter clear");
+        launch_prompt(ctx, p, q, k, v, o, n_q, kv_len, hd, n_q_heads, n_kv_heads, reinterpret_cast<float *>(sp + cb),
+                      cb ? reinterpret_cast<uint32_t *>(sp) : ctx->attn_cnt);
+        return true;
+      }
+    }
     const AttnQ8 a8 = q8 ? *q8 : AttnQ8{nullptr, nullptr, nullptr};
     AttnRope ar = rope ? *rope : AttnRope{nullptr, nullptr, nullptr, 0, pos_dev, 0};
     ar.runs0 = (uint32_t)runs0;

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from mdma_amd import synth
-from mdma_amd.backend import AttnSpec, KvView, RopeSpec, ShapeMismatch
+from mdma_amd.backend import DOMAIN_DEVICE, AttnSpec, Gfx950Backend, KvView, RopeSpec, ShapeMismatch
 from oracle import ffi
 
 pytestmark = pytest.mark.gpu
@@ -230,10 +230,13 @@ def test_prompt_attention_with_growing_scores(backend, hd, nq, nkv, n_q, kv_len,
 
 
 @pytest.mark.parametrize("hd,nq,nkv,n_q,kv_len", [(128, 32, 8, 8, 2048), (128, 8, 2, 9, 1821), (64, 4, 4, 17, 1000),
-                                                  (128, 4, 4, 63, 300), (64, 16, 2, 20, 2500), (128, 8, 4, 12, 4000)])
+                                                  (128, 4, 4, 63, 300), (64, 16, 2, 20, 2500), (128, 8, 4, 12, 4000),
+                                                  (128, 32, 8, 8, 2304), (128, 20, 20, 9, 3300), (64, 8, 1, 20, 3700),
+                                                  (128, 16, 8, 63, 590)])
 def test_few_queries_over_long_prefixes(backend, hd, nq, nkv, n_q, kv_len):
-    # 8 to 63 queries on the matrix-core kernel: part-filled query blocks,
-    # many key chunks and their merge (four at a time, remainders of four).
+    # 8 to 63 queries on both sides of the line to the matrix-core kernel:
+    # part-filled query blocks, many key chunks and their merge (four at a
+    # time, remainders of four).
     q = synth.normal_f32(n_q * nq * hd, 1)
     k, v = f16r(synth.normal_f32(kv_len * nkv * hd, 2)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
     kb, vb = backend.alloc(k.size * 2), backend.alloc(v.size * 2)
@@ -252,7 +255,7 @@ def test_captured_few_queries_take_the_per_query_kernel(backend):
     # Under a capture the matrix-core kernel has no key chunks: 8 queries stay
     # with the per-query kernel, whose first 7 rows are a 7-query call's bits
     # (the same runs of tiles per query).
-    hd, nq, nkv, n_q, kv_len = 128, 32, 8, 8, 2048
+    hd, nq, nkv, n_q, kv_len = 128, 32, 8, 8, 2400
     q = synth.normal_f32(n_q * nq * hd, 1)
     k, v = f16r(synth.normal_f32(kv_len * nkv * hd, 2)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
     kb, vb = backend.alloc(k.size * 2), backend.alloc(v.size * 2)
@@ -314,3 +317,55 @@ def test_prompt_attention_rescales_without_bias(backend, hd, nq, nkv):
     graph.launch()
     check()
     graph.close()
+
+
+def kv_bufs(be, k, v):
+    bufs = [be.alloc(a.size * 2) for a in (k, v)]
+    for b, a in zip(bufs, (k, v)):
+        be.upload(b, 0, a.astype(np.float16))
+    return bufs
+
+
+@pytest.mark.parametrize("n_q,kv_len,nq,nkv", [(16, 2048, 32, 8), (63, 1100, 32, 32)])
+def test_few_queries_ask_for_no_more_than_the_per_query_kernel(n_q, kv_len, nq, nkv):
+    # The key chunks' space neither grows the context's buffers (which ends
+    # graphs) nor makes a full budget refuse the call, and the eager call
+    # leaves what a capture of it needs. (63 queries of 32 KV heads: the
+    # per-query kernel runs unsplit and asks for nothing.)
+    hd = 128
+    be = Gfx950Backend(0)
+    be.set_buffer_budget(device=256 << 20)
+    q = synth.normal_f32(n_q * nq * hd, 1)
+    k, v = f16r(synth.normal_f32(kv_len * nkv * hd, 2)), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
+    kb, vb = kv_bufs(be, k, v)
+    o, qb, spec, kv = be.alloc(q.size * 4), be.f32_buf(q), AttnSpec(hd, nq, nkv), KvView(kb, vb, kv_len)
+    want = ffi.attention(q, k, v, kv_len, hd, nq, nkv)
+
+    def same(call):
+        be.upload(o, 0, np.zeros(q.size, np.float32))
+        call()
+        np.testing.assert_allclose(be.download_f32(o), want, rtol=2e-5, atol=2e-6)
+
+    def call():
+        be.attn(qb, kv, spec, o)
+
+    same(call)
+    graph = be.capture(call)
+    add = be.capture(lambda: be.add(qb, qb, o))
+    for _ in range(2):
+        same(graph.launch)
+        same(call)
+    used, limit = be.buffer_usage(DOMAIN_DEVICE)
+    rest = be.alloc(limit - used + 4096)  # takes the key chunks' space
+    rest2 = be.alloc(be.buffer_usage(DOMAIN_DEVICE)[1] - be.buffer_usage(DOMAIN_DEVICE)[0])
+    for _ in range(2):
+        same(call)
+        same(graph.launch)
+        add.launch()
+    for r in (rest, rest2):
+        r.close()
+    same(call)
+    add.launch()
+    for g in (graph, add):
+        g.close()
+    be.close()
