@@ -453,9 +453,10 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // times the G query heads of one KV head; wave w owns rows 16w..16w+15.
 // Per tile of 64 keys:
 //   S = Q K^T on v_mfma_f32_16x16x32_f16. The f16 keys are exact operands;
-//     q is split exactly into three f16 parts (hi = f16(q), mid = f16(q -
-//     hi), lo = q - hi - mid: 11 + 11 + 2 of its 24 bits), three MFMAs of
-//     exact products added in f32, as the f32 kernels' dot products are;
+//     q, its row scaled by a power of two, is split into three f16 parts (hi =
+//     f16(q), mid = f16(q - hi), lo = q - hi - mid: 11 + 11 + 2 of its 24
+//     bits), three MFMAs of exact products added in f32, as the f32 kernels'
+//     dot products are;
 //   the MFMAs form S^T (keys x queries), so a lane holds 16 scores of one
 //     query: the online softmax is in registers, its maximum two lane
 //     swaps, and the exponentials are already the B operand of
@@ -537,9 +538,9 @@ template <int G, int HD>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restrict__ q, const uint16_t *__restrict__ K,
                                                            const uint16_t *__restrict__ V, float *__restrict__ o,
                                                            uint32_t n_q, uint32_t prefix, uint32_t n_q_heads,
-                                                           uint32_t n_kv_heads, float c_hi, float c_lo, uint32_t ct,
-                                                           float *__restrict__ part, uint32_t *__restrict__ cnt,
-                                                           F16In in) {
+                                                           uint32_t n_kv_heads, float scale, float c_hi, float c_lo,
+                                                           uint32_t ct, float *__restrict__ part,
+                                                           uint32_t *__restrict__ cnt, F16In in) {
   constexpr int QT = 64 / G;             // queries per workgroup
   constexpr int NC = HD / 32;            // 32-dim K steps of S
   constexpr int ND = HD / 16;            // 16-dim blocks of O
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   constexpr int VP = 64 + 8;             // padded row of the transposed V tile (f16)
   __shared__ __attribute__((aligned(16))) uint16_t ks[64 * HD];        // keys x dims, chunks swizzled
   __shared__ __attribute__((aligned(16))) uint16_t vt[HD * VP];        // dims x keys
-  sgpr_ready(q, K, V, o, n_q, prefix, n_q_heads, n_kv_heads, c_hi, c_lo);
+  sgpr_ready(q, K, V, o, n_q, prefix, n_q_heads, n_kv_heads, scale, c_hi, c_lo);
   const uint32_t kvh = blockIdx.x, q0 = blockIdx.y * QT;
   const uint32_t tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lq = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -581,23 +582,38 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   const uint32_t n_ch = ct ? (n_tiles + ct - 1) / ct : 1, ch = blockIdx.z;
   if (ch >= n_ch) return;  // (uniform: this block has fewer chunks)
   const uint32_t t_begin = ct ? ch * ct : 0, t_end = ct ? min(t_begin + ct, n_tiles) : n_tiles;
-  gload(t_begin);
 
   // This lane's Q operand row (16 wave + l16) as f16 hi + mid + lo, dims
-  // 32c + 8lq (each remainder is exact in f32).
+  // 32c + 8lq (each remainder is exact in f32), times the power of two that
+  // brings the row's largest value to [2^14, 2^15): values down to 2^-15 of
+  // it keep all 24 bits, smaller ones 2^-40 of it. The scores' factor takes
+  // the power back.
   v8h_t qhi[NC], qmid[NC], qlo[NC];
   const uint32_t row = 16 * wave + l16, qi = q0 + row / G, head = kvh * G + row % G;
   {
     const float *qr = q + ((size_t)min(qi, n_q - 1) * n_q_heads + head) * HD + 8 * lq;
+    v4f_u xv[2 * NC];
+    float qm = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2 * NC; i++) xv[i] = *reinterpret_cast<const v4f_u *>(qr + 32 * (i >> 1) + 4 * (i & 1));
+    __builtin_amdgcn_sched_barrier(0);
+    gload(t_begin);  // (behind q's loads: in flight over q's split)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * NC; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) qm = fmaxf(qm, fabsf(xv[i][e]));
+    const int sh = min(141 - (int)(__builtin_bit_cast(uint32_t, quarter_max(qm)) >> 23), 96);
+    const float up = __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23), down = __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
+    c_hi *= down;
+    c_lo *= down;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      const float4 a = *reinterpret_cast<const float4 *>(qr + 32 * c);
-      const float4 b = *reinterpret_cast<const float4 *>(qr + 32 * c + 4);
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        const _Float16 hi = (_Float16)x[e];
-        const float r1 = x[e] - (float)hi;
+        const float x = xv[2 * c + (e >> 2)][e & 3] * up;
+        const _Float16 hi = (_Float16)x;
+        const float r1 = x - (float)hi;
         const _Float16 mid = (_Float16)r1;
         qhi[c][e] = hi;
         qmid[c][e] = mid;
@@ -777,6 +793,52 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   const uint32_t KO = n_q_heads * HD;
 #pragma unroll
   for (int n = 0; n < ND; n++) O[n] = O[n] / l;
+  // A row that came out not finite: from an infinity or a NaN, perhaps one of
+  // a key the query does not see (0 times it in the MFMA) or an infinite value
+  // whose weight's low part is 0 or negative. Such rows again in f32, key by
+  // key, over the keys they see.
+  v4f_t z = {0.f, 0.f, 0.f, 0.f};  // NaN from any that is not finite
+#pragma unroll
+  for (int n = 0; n < ND; n++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) z[j] = fmaf(O[n][j], 0.f, z[j]);
+  const float zs = (z[0] + z[1]) + (z[2] + z[3]);
+  for (uint64_t todo = __ballot(zs != 0.f && qi < n_q); todo;) {
+    const uint32_t r = __builtin_ctzll(todo) & 15;
+    todo &= ~(0x0001000100010001ull << r);
+    const uint32_t rqi = q0 + (16 * wave + r) / G, n_vis = prefix + rqi + 1;
+    const float *qr = q + ((size_t)rqi * n_q_heads + kvh * G + (16 * wave + r) % G) * HD;
+    auto score = [&](uint32_t key) {
+      const uint16_t *kr = Kh + (size_t)key * kv_row;
+      float s = 0.f;
+      for (int d = 0; d < HD; d++) s = fmaf(qr[d], h2f(kr[d]), s);
+      return s * scale;
+    };
+    float rm = -INFINITY, rl = 0.f, acc[HD / 64] = {};
+    for (uint32_t k0 = 0; k0 < n_vis; k0 += 64) rm = fmaxf(rm, score(min(k0 + lane, n_vis - 1)));
+#pragma unroll
+    for (int i = 32; i >= 1; i >>= 1) rm = fmaxf(rm, __shfl_xor(rm, i, 64));
+    for (uint32_t k0 = 0; k0 < n_vis; k0 += 64) {
+      const uint32_t n = min(64u, n_vis - k0);
+      const float p = expf(score(min(k0 + lane, n_vis - 1)) - rm);
+      rl += lane < n ? p : 0.f;
+      for (uint32_t k = 0; k < n; k++) {
+        const float pk = __shfl(p, (int)k, 64);
+#pragma unroll
+        for (int i = 0; i < HD / 64; i++)
+          acc[i] = fmaf(pk, h2f(Vh[(size_t)(k0 + k) * kv_row + 64 * i + lane]), acc[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 32; i >= 1; i >>= 1) rl += __shfl_xor(rl, i, 64);
+#pragma unroll
+    for (int n = 0; n < ND; n++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const float v = __shfl(acc[n / 4], 16 * (n % 4) + 4 * (int)lq + j, 64) / rl;
+        if (l16 == r) O[n][j] = v;
+      }
+  }
   if (qo) {
     // The output projection's f16-path input (gemm_act_kernel's arithmetic):
     // dims 32 b + [0, 32) of row (qi, head) are one quantization block, dims
@@ -1517,7 +1579,7 @@ void launch_prompt(mdma_ctx *ctx, const PromptPlan &p, const float *q, const uin
 #define MDMA_ATTP(GG, HH)                                                                                          \
   attn_prefill_kernel<GG, HH><<<grid, dim3(256), 0, ctx->stream>>>(                                                \
       q, k, v, o, (uint32_t)n_q, (uint32_t)(kv_len - n_q), (uint32_t)n_q_heads, (uint32_t)n_kv_heads,              \
-      c_hi, c_lo, (uint32_t)(part ? p.ct : 0), part, cnt, fin)
+      1.0f / sqrtf((float)hd), c_hi, c_lo, (uint32_t)(part ? p.ct : 0), part, cnt, fin)
   if (hd == 128) {
     if (GP == 1) MDMA_ATTP(1, 128);
     else if (GP == 2) MDMA_ATTP(2, 128);

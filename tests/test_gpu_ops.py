@@ -326,6 +326,74 @@ def kv_bufs(be, k, v):
     return bufs
 
 
+# hd, query heads, KV heads, queries, keys: few queries and prompts on the
+# matrix-core kernel, part-filled blocks, one key chunk and several.
+PROMPTS = [(128, 32, 8, 8, 2400), (64, 16, 16, 17, 2200), (128, 20, 20, 63, 500), (64, 8, 8, 64, 100), (128, 8, 1, 70, 700),
+           (128, 8, 4, 130, 130)]
+
+
+@pytest.mark.parametrize("hd,nq,nkv,n_q,kv_len", PROMPTS)
+@pytest.mark.parametrize("what", ["large", "small", "mixed"])
+def test_prompt_attention_over_the_range_of_q(backend, hd, nq, nkv, n_q, kv_len, what):
+    # Query values past f16's range and far below it, keys the other way, so
+    # that the scores stay ordinary: q keeps its f32 precision. Bounds as in
+    # test_few_queries_over_long_prefixes.
+    q = synth.normal_f32(n_q * nq * hd, 1).reshape(n_q, nq, hd)
+    k, v = synth.normal_f32(kv_len * nkv * hd, 2).reshape(kv_len, nkv, hd), f16r(synth.normal_f32(kv_len * nkv * hd, 3))
+    if what == "large":
+        q[:, :, 3], k[:, :, 3] = q[:, :, 3] * 1e6, k[:, :, 3] * 1e-6  # (f16 subnormals)
+    elif what == "small":
+        q, k = q * 1e-4, k * 1e4
+    else:  # rows of every size, one of zeros
+        size = 10.0 ** np.linspace(-38, 2, n_q * nq).reshape(n_q, nq, 1)
+        q = (q * size).astype(np.float32)
+        q[n_q // 2] = 0
+        k = k * 0.1
+    q, k = q.astype(np.float32).reshape(-1), f16r(k.astype(np.float32).reshape(-1))
+    kb, vb = kv_bufs(backend, k, v)
+    o = backend.alloc(q.size * 4)
+    backend.attn(backend.f32_buf(q), KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
+    want = ffi.attention(q, k, v, kv_len, hd, nq, nkv)
+    # "mixed": the largest rows' sums of |q| |k| are up to 130 * 0.64 * 100 * 0.1 * 0.64 =
+    # 530, / sqrt(hd) 47 to 66; an f32 sum in any order of 128 such terms, here and in
+    # the CPU's, is off by up to a few 2^-24 of that, 2e-5 together, and the
+    # outputs (values below 5) by that factor.
+    np.testing.assert_allclose(backend.download_f32(o), want, rtol=2e-5, atol=1e-4 if what == "mixed" else 4e-6)
+
+
+@pytest.mark.parametrize("hd,nq,nkv,n_q,kv_len", PROMPTS)
+@pytest.mark.parametrize("captured", [False, True])
+def test_prompt_attention_with_values_that_are_not_finite(backend, hd, nq, nkv, n_q, kv_len, captured):
+    # A key that a query does not see may hold anything; one it sees makes
+    # the output what the CPU's is. Infinite values at a key in the middle and
+    # the last few keys, NaN keys and values at the last, one infinite query.
+    q = synth.normal_f32(n_q * nq * hd, 1).reshape(n_q, nq, hd)
+    k = f16r(synth.normal_f32(kv_len * nkv * hd, 2)).reshape(kv_len, nkv, hd)
+    v = f16r(synth.normal_f32(kv_len * nkv * hd, 3)).reshape(kv_len, nkv, hd)
+    v[kv_len - 3, :, 5], v[kv_len - 2, 0, 7], v[kv_len - n_q // 2 - 1, nkv - 1, 0] = np.inf, -np.inf, np.inf
+    v[kv_len - 1], k[kv_len - 1, nkv - 1] = np.nan, np.nan
+    q[n_q // 3, nq - 1, 9] = np.inf
+    kb, vb = kv_bufs(backend, k.reshape(-1), v.reshape(-1))
+    o, qb = backend.alloc(q.size * 4), backend.f32_buf(q.reshape(-1))
+
+    def call():
+        backend.attn(qb, KvView(kb, vb, kv_len), AttnSpec(hd, nq, nkv), o)
+
+    call()
+    if captured:
+        graph = backend.capture(call)
+        backend.upload(o, 0, np.zeros(q.size, np.float32))
+        graph.launch()
+    with np.errstate(all="ignore"):
+        want = ffi.attention(q.reshape(-1), k.reshape(-1), v.reshape(-1), kv_len, hd, nq, nkv)
+    got = backend.download_f32(o)
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).sum() > want.size // 2
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    np.testing.assert_allclose(got[ok], want[ok], rtol=2e-5, atol=4e-6)
+
+
 @pytest.mark.parametrize("n_q,kv_len,nq,nkv", [(16, 2048, 32, 8), (63, 1100, 32, 32)])
 def test_few_queries_ask_for_no_more_than_the_per_query_kernel(n_q, kv_len, nq, nkv):
     # The key chunks' space neither grows the context's buffers (which ends
