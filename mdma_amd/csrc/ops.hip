@@ -467,9 +467,13 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // product is rounded once; m is the largest score seen to within 2^8 (the
 // sums are rescaled only when a tile passes it by more: p <= 256), l the
 // sum, the output O / l. Only tiles past a wave's first query mask.
+// The low parts, of q and of P, add up in accumulators of their own: there
+// they take no roundings at the size of the whole sums (the error against 64
+// bits of 1500 queries over 2500 keys 4.1e-7 -> 3.1e-7, of 8 over 2400 2.45e-7 ->
+// 2.09e-7, the per-query kernel's 2.16e-7; 2% of the time).
 // What bounds it is issue: 80 MFMAs a tile and wave (16 cycles each) beside
-// about 250 VALU instructions, two waves per SIMD. 1500 queries over 2500
-// keys, 32 heads of 128: 142 us; with P through LDS, expf and a mask per score
+// about 270 VALU instructions, two waves per SIMD. 1500 queries over 2500
+// keys, 32 heads of 128: 151 us; with P through LDS, expf and a mask per score
 // (600 VALU instructions) it was 252.
 // Key chunks (ct > 0): a query block's tiles are split into chunks of ct
 // tiles, one workgroup each (blockIdx.z), so the long blocks at the end of
@@ -625,9 +629,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   const uint32_t vis = prefix + qi, vis0 = prefix + q0 + 16 * wave / G;
   const float slack = 8.0f / c_hi;  // in scores: a factor 2^8 of p
   float m = -INFINITY, l = 0.f;     // l: this lane's keys only
-  v4f_t O[ND];
+  v4f_t O[ND], Ol[ND];               // Ol: of the probabilities' low parts
 #pragma unroll
-  for (int n = 0; n < ND; n++) O[n] = v4f_t{0.f, 0.f, 0.f, 0.f};
+  for (int n = 0; n < ND; n++) O[n] = Ol[n] = v4f_t{0.f, 0.f, 0.f, 0.f};
 
   for (uint32_t t = t_begin; t < t_end; t++) {
     lds_barrier();  // the previous tile's reads of ks and vt are done
@@ -652,9 +656,11 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     if (t + 1 < t_end) gload(t + 1);  // in flight over this tile's arithmetic
 
     // ---- S^T = K Q^T: 64 keys x 16 queries per wave ----
-    v4f_t S[4];
+    // (q's low parts in sums of their own: added to the high part's they would
+    // take a rounding at its size at every step.)
+    v4f_t S[4], Sl[4];
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) S[kb] = v4f_t{0.f, 0.f, 0.f, 0.f};
+    for (int kb = 0; kb < 4; kb++) S[kb] = Sl[kb] = v4f_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < NC; c++) {
       v8h_t A[4];
@@ -664,12 +670,14 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
         A[kb] = *reinterpret_cast<const v8h_t *>(&ks[key * HD + 8 * ((4 * c + lq) ^ (key & (KCH - 1)))]);
       }
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qlo[c], S[kb], 0, 0, 0);
+      for (int kb = 0; kb < 4; kb++) Sl[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qlo[c], Sl[kb], 0, 0, 0);
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qmid[c], S[kb], 0, 0, 0);
+      for (int kb = 0; kb < 4; kb++) Sl[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qmid[c], Sl[kb], 0, 0, 0);
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qhi[c], S[kb], 0, 0, 0);
     }
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) S[kb] += Sl[kb];
     // ---- online softmax: S[kb][r] is key 64 t + 16 kb + 4 lq + r ----
     if (64 * t + 63 > vis0) {  // (uniform) a key some query of the wave does not see
       const uint32_t k0 = 64 * t + 4 * lq;
@@ -688,7 +696,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
       const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : exp2_scaled(m - mn, c_hi, c_lo);
       l *= al;
 #pragma unroll
-      for (int n = 0; n < ND; n++) O[n] *= al;
+      for (int n = 0; n < ND; n++) O[n] *= al, Ol[n] *= al;
       m = mn;
     }
     const float mr = m == -INFINITY ? 0.f : m;  // a later chunk's query may see no key yet
@@ -719,9 +727,11 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 #pragma unroll
       for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[n], Ph[c], O[n], 0, 0, 0);
 #pragma unroll
-      for (int n = 0; n < ND; n++) O[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[n], Pl[c], O[n], 0, 0, 0);
+      for (int n = 0; n < ND; n++) Ol[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[n], Pl[c], Ol[n], 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int n = 0; n < ND; n++) O[n] += Ol[n];
   if (n_ch > 1) {
     // Leave this chunk's (m, l, O), then the last chunk to arrive merges.
     constexpr int NV = 2 + 4 * ND;
