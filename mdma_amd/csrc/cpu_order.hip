@@ -258,7 +258,8 @@ __device__ __forceinline__ float chain_add(float s, uint32_t n4, Read &&rd) {
   return s;
 }
 
-// ---- up to 4 tokens over prepared rows: dequantization and chains apart ----
+// ---- few tiles over prepared rows: dequantization and chains apart ----
+// (4 tokens and 16 rows a workgroup, the groups of tokens in the grid)
 // With one lane doing everything for its row, the chain's next addition waits
 // for the column's whole dequantization (about 11 VALU instructions a
 // column), on one wave per SIMD. Here NP producer waves dequantize, multiply
@@ -381,6 +382,10 @@ template <int DT, int R, int NP, int TT>
 __global__ __launch_bounds__(64 * (NP + (R * TT + 63) / 64)) void gemv_seq_pipe_kernel(
     SeqSet js, uint32_t n_in, uint64_t row_bytes, const float *__restrict__ x, uint32_t T) {
 #pragma clang fp contract(off)
+  // Tokens TT blockIdx.y and up; T: those left.
+  x += (size_t)TT * blockIdx.y * n_in;
+  const uint32_t t0 = TT * blockIdx.y;
+  T -= t0;
   using Unit = SeqUnit<DT>;
   constexpr int UC = Unit::UC, NC = (R * TT + 63) / 64, UPW = 64 / R, UPS = NP * UPW;
   constexpr int SC = UPS * UC;          // columns of a stage
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(64 * (NP + (R * TT + 63) / 64)) void gemv_seq_pipe_
       s = chain_add(s, q4, [&](uint32_t k) { return pb[k][c]; });
     }
     const uint32_t row = tile * R + c % R, t = c / R;
-    if (wave * 64 + lane < LANES && row < n_out && t < T) y[(size_t)t * n_out + row] = s;
+    if (wave * 64 + lane < LANES && row < n_out && t < T) y[(size_t)(t0 + t) * n_out + row] = s;
     return;
   }
   const uint32_t p = wave - NC, ptid = p * 64 + lane, r = lane % R, uu = p * UPW + lane / R;
@@ -648,11 +653,19 @@ namespace {
 // 20.5 us in 16-row ones (64-row ones would use 64 of the 256 CUs).
 constexpr uint64_t SEQ_WIDE_ROWS = 16384;
 // Tiles of 16 rows and 4 tokens up to which the split kernel is the faster
-// one: past them the launch is bound by its products' VALU work, which the
-// 8-token kernel spends less of per token. us, split / one-lane kernel:
-// 4096x4096 Q6_K T = 1: 20.5 / 96.2, 2: 30.8 / 391, 8 (512 tiles): 86.2 / 395;
-// 2x14336x4096 Q4_K T = 4 (1792 tiles): 262 / 520, 8 (3584): 518 / 542.
-constexpr uint64_t SEQ_PIPE_TILES = 3584;
+// one, per job: past them the launch is bound by its products' VALU work
+// (0.145, 0.159, 0.088 us a tile of 4096 columns for Q4_K, Q6_K, Q8_0, and a
+// part that does not fall with the columns), which the 8-token kernel, whose
+// time is its chain's, spends less of per token; several jobs are as many of its
+// launches. us, split / 8-token kernel, 4096 columns: Q6_K 4096 rows T = 40
+// (2560 tiles) 408 / 421, 44 (2816) 447 / 421; Q4_K 28672 rows T = 4 (1792) 260 /
+// 275, 4096 rows T = 36 (2304) 330 / 272; Q8_0 4096 rows T = 40 223 / 251, 56
+// (3584) 307 / 265; Q4_K 512 rows of 2048, T = 200 (1600) 137 / 133; Q8_0 768
+// rows of 288, T = 200 (2400) 29.3 / 24.6, 288 rows (900) 15.2 / 22.2.
+uint64_t seq_pipe_tiles(int32_t dt, uint64_t n_in) {
+  const uint64_t top = dt == DT_Q4_K ? 2170 : dt == DT_Q6_K ? 2700 : 2850, fill = dt == DT_Q4_K ? 850 : 200;
+  return top * n_in / (n_in + fill);
+}
 
 template <int DT, int R, int NP, int TT>
 void seq_pipe(mdma_ctx *ctx, const GemvJob *jobs, int n, uint64_t row_bytes, const float *x, uint64_t T) {
@@ -663,7 +676,8 @@ void seq_pipe(mdma_ctx *ctx, const GemvJob *jobs, int n, uint64_t row_bytes, con
                     : SeqJob{nullptr, nullptr, 0, 0};
     tiles += js.j[i].tiles;
   }
-  gemv_seq_pipe_kernel<DT, R, NP, TT><<<dim3((uint32_t)tiles), dim3(64 * (NP + (R * TT + 63) / 64)), 0, ctx->stream>>>(
+  const dim3 grid((uint32_t)tiles, (uint32_t)((T + TT - 1) / TT));
+  gemv_seq_pipe_kernel<DT, R, NP, TT><<<grid, dim3(64 * (NP + (R * TT + 63) / 64)), 0, ctx->stream>>>(
       js, (uint32_t)jobs[0].n_in, row_bytes, x, (uint32_t)T);
   hip_check(hipGetLastError(), "gemv_seq_pipe launch");
 }
@@ -680,11 +694,7 @@ void seq_pipe_t(mdma_ctx *ctx, const GemvJob *jobs, int n, uint64_t row_bytes, c
   else if (T == 2)
     seq_pipe<DT, 16, 1, 2>(ctx, jobs, n, row_bytes, x, T);
   else
-    for (uint64_t t0 = 0; t0 < T; t0 += 4) {
-      GemvJob js[3];
-      for (int i = 0; i < n; i++) js[i] = jobs[i], js[i].y += t0 * jobs[i].n_out;
-      seq_pipe<DT, 16, 1, 4>(ctx, js, n, row_bytes, x + t0 * jobs[0].n_in, T - t0 < 4 ? T - t0 : 4);
-    }
+    seq_pipe<DT, 16, 1, 4>(ctx, jobs, n, row_bytes, x, T);
 }
 }  // namespace
 
@@ -697,7 +707,9 @@ void launch_gemv_seq(mdma_ctx *ctx, const GemvJob *jobs, int n, const float *x, 
     one = one && jobs[i].layout == j.layout && jobs[i].dtype == j.dtype && jobs[i].n_in == j.n_in && jobs[i].n_out > 0;
     tiles += (jobs[i].n_out + 15) / 16;
   }
-  if (!one || (T + 3) / 4 * tiles > (T == 1 ? 0x7ffffffull : SEQ_PIPE_TILES)) {
+  // (One token has no such limit; two take half a tile's products.)
+  if (!one || tiles > 0x7ffffffull ||
+      (T > 1 && (T == 2 ? tiles / 2 : (T + 3) / 4 * tiles) > n * seq_pipe_tiles(j.dtype, j.n_in))) {
     for (int i = 0; i < n; i++) launch_gemv_seq(ctx, jobs[i], x, T);
     return;
   }

@@ -124,6 +124,24 @@ def test_fused_projections_at_tile_edges(cpu_mode, dtype, k, T):
         assert np.array_equal(bits(got[:T * r].reshape(T, r)), bits(ffi.qmatmul(dtype, raw, r, k, x))), r
 
 
+@pytest.mark.parametrize("dtype,k,rows,T", [(Q8, 288, 288, 200), (Q8, 288, 33, 9), (Q4K, 512, 40, 70), (Q6K, 256, 17, 131),
+                                            (Q4K, 256, 1700, 18), (Q8, 64, 800, 75)])
+def test_groups_of_four_tokens_in_one_launch(cpu_mode, dtype, k, rows, T):
+    # Whole and part-filled groups of 4 tokens, a last group of one, on both
+    # sides of the line to the 8-token kernel; one job and three.
+    be = cpu_mode
+    raw = synth.weight(dtype, rows, k, rows + k, True)
+    w, x = weight(be, dtype, raw, rows, k, "prepared"), synth.normal_f32(T * k, T + k)
+    want = bits(ffi.qmatmul(dtype, raw, rows, k, x))
+    assert np.array_equal(bits(gpu_qmatmul(be, w, rows, x, T)), want)
+    outs = [be.f32_buf(np.full(T * rows + 8, CANARY, np.float32)) for _ in range(3)]
+    be.qmatmul_qkv(w, w, w, be.f32_buf(x), *outs)
+    for o in outs:
+        got = be.download_f32(o)
+        assert np.all(got[T * rows:] == CANARY), "wrote past the output"
+        assert np.array_equal(bits(got[:T * rows].reshape(T, rows)), want)
+
+
 @pytest.mark.parametrize("dtype,k", [(Q4K, 256), (Q4K, 768), (Q6K, 512), (Q8, 160)])
 def test_wide_workgroups_at_tile_edges(cpu_mode, dtype, k):
     # One token over more rows than the 16-row tiles take: 64-row workgroups.
