@@ -617,6 +617,8 @@ int mdma_gfx950_set_buffer_budget(mdma_ctx *ctx, uint64_t device_bytes, uint64_t
     need(ctx, "set_buffer_budget");
     std::lock_guard<std::recursive_mutex> g(ctx->lock);
     // BufferBudget::replace (src/memory/buffers.rs:61-70): only an unused ledger.
+    // (The split partials' space is no use of the caller's.)
+    if (ctx->budget[MDMA_DOMAIN_DEVICE].used == mdma::split_parts_held(ctx)) mdma::drop_split_parts(ctx);
     if (ctx->budget[MDMA_DOMAIN_DEVICE].used || ctx->budget[MDMA_DOMAIN_HOST].used)
       fail(MDMA_ERR_BACKEND, "buffer budget must be installed before allocations or sharing");
     ctx->budget[MDMA_DOMAIN_DEVICE].limit = device_bytes;

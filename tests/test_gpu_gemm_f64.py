@@ -268,3 +268,20 @@ def test_infinity_in_a_rows_last_columns(backend, k, T, fused):
     assert np.isinf(want[bad]).sum() > rows // 2  # (few weights are zero; silu(-inf) is NaN)
     assert np.array_equal(got[bad], want[bad], equal_nan=True)
     assert np.allclose(got[1:T - 1], want[1:T - 1], rtol=1e-4, atol=1e-4)
+
+
+def test_partials_space_is_no_use_of_the_budget():
+    # With every buffer of the caller's freed the ledger counts as unused (the
+    # f32 mode's calls leave nothing else): a budget can be installed.
+    be = Gfx950Backend(0)
+    rows, k, T = 200, 1024, 70
+    w = be.upload_weight(synth.weight(Q4K, rows, k, 1, True), Q4K, (rows, k))
+    x, y = be.f32_buf(synth.normal_f32(T * k, 2)), out_buf(be, T * rows)
+    be.qmatmul(w, x, y)
+    with pytest.raises(BackendError):
+        be.set_buffer_budget(device=1 << 20)
+    for b in (w.buf, x, y):
+        b.close()
+    be.set_buffer_budget(device=1 << 20)
+    assert be.buffer_usage(DOMAIN_DEVICE) == (0, 1 << 20)
+    be.close()
