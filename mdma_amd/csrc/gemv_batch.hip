@@ -1224,8 +1224,9 @@ __global__ __launch_bounds__(256) void tile_repack_q6_kernel(const uint8_t *__re
 // ---------------------------------------------------------------------------
 // 17 to 63 tokens: one launch instead of one ring launch per 16 tokens, so
 // the weights are read and unpacked once. The same products, scalings and
-// summation order as above (the results are the same bits as 16-token
-// launches).
+// summation order as above (the same bits as its 16-token launches; a last
+// one or two tokens of a loop of those go to the row teams, whose f32 sums
+// round differently).
 //
 // A workgroup is 4 waves of 16 rows each (gated: two of gate, two of the
 // same rows of up) over NT tiles of 16 tokens. The weights go from HBM to
@@ -1239,7 +1240,7 @@ __global__ __launch_bounds__(256) void tile_repack_q6_kernel(const uint8_t *__re
 //
 // Launches of no more tiles than CUs split the fixed column chunks over
 // workgroups: each leaves its chunks' sums, and a second kernel adds them in
-// chunk order. What bounds it is instruction issue at two waves per SIMD (one
+// chunk order (without space for the sums: 16-token launches). What bounds it is instruction issue at two waves per SIMD (one
 // integer multiply-add per result and scale group, and the unpacking). us at
 // 43 tokens, 16-token launches / here: gate/up 2x14336x4096 Q4_K 56.9 / 35.6,
 // 4096x14336 Q6_K 55.1 / 32.2, 4096x4096 Q6_K 28.0 / 17.6; at 17: 34.4 / 27.9,
@@ -1695,8 +1696,8 @@ void wide_launch(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, c
 
 template <class W, bool GLU>
 void wide_fmt(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, const float *dx) {
-  if (ws.T <= 16) wide_launch<W, 1, GLU>(ctx, ws, tiles, qx, dx);
-  else if (ws.T <= 32) wide_launch<W, 2, GLU>(ctx, ws, tiles, qx, dx);
+  static_assert(WIDE_MIN_TOKENS > 16, "two token tiles at least");
+  if (ws.T <= 32) wide_launch<W, 2, GLU>(ctx, ws, tiles, qx, dx);
   else if (ws.T <= 48) wide_launch<W, 3, GLU>(ctx, ws, tiles, qx, dx);
   else wide_launch<W, 4, GLU>(ctx, ws, tiles, qx, dx);
 }

@@ -281,8 +281,9 @@ void launch_gemv_batch(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gate
                        float *ygated);
 // Tokens from which int8-mode GEMVs of prepared rows go to the batch kernel.
 constexpr uint64_t BATCH_MIN_TOKENS = 3;
-// 17 to 63 tokens in one launch (gemv_batch.hip), the same bits as 16-token
-// launches; false, launching nothing, where it does not cover the call.
+// 17 to 63 tokens in one launch (gemv_batch.hip), the same bits as the batch
+// kernel's 16-token launches; false, launching nothing, where it does not
+// cover the call or has no space for its partial sums.
 constexpr uint64_t WIDE_MIN_TOKENS = 17;
 bool launch_gemv_wide(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated, const float *x, uint64_t T,
                       float *ygated);
