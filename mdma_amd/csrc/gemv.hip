@@ -851,7 +851,7 @@ void quantize_into_scratch(mdma_ctx *ctx, const float *x, uint64_t T, uint64_t n
 }
 
 
-// BATCH_MIN_TOKENS: below it int8-mode GEMVs of prepared rows run the
+// BATCH_MIN_TOKENS: in calls of fewer int8-mode GEMVs of prepared rows run the
 // row-team kernels, which keep each token's activations in registers. At
 // Llama-3-8B shapes the batch kernel's ring is faster from 3 tokens on every
 // weight (gate/up 16.2 us against 28.9 us at 3 tokens); at 2 the row teams
@@ -1002,15 +1002,13 @@ void launch_gemv_i8(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float 
   }
   if (launch_gemv_wide(ctx, jobs, n_jobs, false, x, T, nullptr)) return;
   if (T >= BATCH_MIN_TOKENS && gemv_batch_ok(jobs, n_jobs, 16)) {
-    // Up to 16 tokens per matrix-core launch (a short remainder: row teams).
+    // Up to 16 tokens per matrix-core launch, a remainder of one or two too: the
+    // bits of gemv_wide, which takes such calls where it has the space.
     for (uint64_t t0 = 0; t0 < T; t0 += 16) {
       const uint64_t tn = T - t0 < 16 ? T - t0 : 16;
       GemvJob js[3];
       for (int i = 0; i < n_jobs; i++) js[i] = offset_job(jobs[i], t0);
-      if (tn < BATCH_MIN_TOKENS)
-        launch_gemv_team(ctx, MDMA_ACT_I8, js, n_jobs, false, x + t0 * jobs[0].n_in, tn, nullptr);
-      else
-        launch_gemv_batch(ctx, js, n_jobs, false, x + t0 * jobs[0].n_in, tn, nullptr);
+      launch_gemv_batch(ctx, js, n_jobs, false, x + t0 * jobs[0].n_in, tn, nullptr);
     }
     return;
   }
@@ -1052,12 +1050,7 @@ void launch_gemv_i8_gated(mdma_ctx *ctx, const GemvJob &gate, const GemvJob &up,
     for (uint64_t t0 = 0; t0 < T; t0 += 16) {
       const uint64_t tn = T - t0 < 16 ? T - t0 : 16;
       const GemvJob js[2] = {offset_job(gate, t0), offset_job(up, t0)};
-      const float *xt = x + t0 * gate.n_in;
-      float *yt = y + t0 * gate.n_out;
-      if (tn < BATCH_MIN_TOKENS)
-        launch_gemv_team(ctx, MDMA_ACT_I8, js, 2, true, xt, tn, yt);
-      else
-        launch_gemv_batch(ctx, js, 2, true, xt, tn, yt);
+      launch_gemv_batch(ctx, js, 2, true, x + t0 * gate.n_in, tn, y + t0 * gate.n_out);
     }
     return;
   }

@@ -1224,9 +1224,8 @@ __global__ __launch_bounds__(256) void tile_repack_q6_kernel(const uint8_t *__re
 // ---------------------------------------------------------------------------
 // 17 to 63 tokens: one launch instead of one ring launch per 16 tokens, so
 // the weights are read and unpacked once. The same products, scalings and
-// summation order as above (the same bits as its 16-token launches; a last
-// one or two tokens of a loop of those go to the row teams, whose f32 sums
-// round differently).
+// summation order as above: the same bits as its 16-token launches, which take
+// a loop's last one or two tokens too.
 //
 // A workgroup is 4 waves of 16 rows each (gated: two of gate, two of the
 // same rows of up) over NT tiles of 16 tokens. The weights go from HBM to

@@ -3,9 +3,7 @@ register-staged kernel's 16-token launches, at the edges of its tiles (rows of
 64, gated 32; token tiles of 16), of its column chunks (one block, fewer than
 eight, an odd number, not a multiple of eight), with its tiles whole and with
 their chunks split over workgroups, fused and gated. The oracle side is
-test_i8_mode_batched (17 and 35 tokens) and the block-dot routes (40). (A
-16-token loop leaves a remainder of one or two tokens to the row teams, whose
-f32 sums round differently: the counts here leave none.)"""
+test_i8_mode_batched (17 and 35 tokens) and the block-dot routes (40)."""
 import numpy as np
 import pytest
 
@@ -43,7 +41,7 @@ def both(be, sizes, call):
 @pytest.mark.parametrize("dtype", [Q4K, Q6K, Q8])
 @pytest.mark.parametrize("rows,k", [((1, 64, 65), 256), ((129, 16, 63), 1280), ((96, 32, 32), 4096), ((70, 1, 1), 14336),
                                     ((16500, 40, 8), 768)])
-@pytest.mark.parametrize("T", [19, 35, 48, 63])
+@pytest.mark.parametrize("T", [17, 19, 34, 35, 48, 63])
 def test_projections_equal_staged(i8, dtype, rows, k, T):
     ws = [i8.upload_weight(synth.weight(dtype, r, k, 7 + r, True), dtype, (r, k)) for r in rows]
     x = i8.f32_buf(synth.normal_f32(T * k, T + k))
@@ -53,13 +51,33 @@ def test_projections_equal_staged(i8, dtype, rows, k, T):
 
 @pytest.mark.parametrize("dtype", [Q4K, Q6K, Q8])
 @pytest.mark.parametrize("rows,k", [(33, 768), (200, 4096), (8300, 512)])
-@pytest.mark.parametrize("T", [19, 32, 51])
+@pytest.mark.parametrize("T", [18, 19, 32, 49, 51])
 def test_gate_up_equal_staged(i8, dtype, rows, k, T):
     ws = [i8.upload_weight(synth.weight(dtype, rows, k, s, True), dtype, (rows, k)) for s in (1, 2)]
     x = i8.f32_buf(synth.normal_f32(T * k, T) * 0.1)
     gs, us = i8.alloc(T * rows * 4), i8.alloc(T * rows * 4)
     a, b = both(i8, [T * rows], lambda o: i8.ffn_gate_up(ws[0], ws[1], x, gs, us, o[0]))
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("T", [17, 18, 40, 50])
+def test_captured_call_gives_the_eager_bits(T):
+    # A capture has no space for the chunk sums: 16 tokens a launch, the last
+    # one or two included.
+    be = Gfx950Backend(0)
+    be.set_act_mode(bm.ACT_I8)
+    rows, k = 200, 2048
+    w = be.upload_weight(synth.weight(Q6K, rows, k, 1, True), Q6K, (rows, k))
+    x, y = be.f32_buf(synth.normal_f32(T * k, 2)), be.alloc(T * rows * 4)
+    be.qmatmul(w, x, y)
+    ref = be.download_f32(y)
+    graph = be.capture(lambda: be.qmatmul(w, x, y))
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        graph.launch()
+        assert np.array_equal(be.download_f32(y).view(np.uint32), ref.view(np.uint32))
+    graph.close()
+    be.close()
 
 
 def test_captured_and_over_budget_run_unsplit():
