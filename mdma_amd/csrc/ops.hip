@@ -453,18 +453,17 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // times the G query heads of one KV head; wave w owns rows 16w..16w+15.
 // Per tile of 64 keys:
 //   S = Q K^T on v_mfma_f32_16x16x32_f16. The f16 keys are exact operands;
-//     q, its row scaled by a power of two, is split into three f16 parts (hi =
-//     f16(q), mid = f16(q - hi), lo = q - hi - mid: 11 + 11 + 2 of its 24
-//     bits), three MFMAs of exact products added in f32, as the f32 kernels'
-//     dot products are;
+//     q times scale * log2 e, its row scaled by a power of two, is split into
+//     three f16 parts (11 bits each), three MFMAs of exact products added in
+//     f32, as the f32 kernels' dot products are;
 //   the MFMAs form S^T (keys x queries), so a lane holds 16 scores of one
 //     query: the online softmax is in registers, its maximum two lane
 //     swaps, and the exponentials are already the B operand of
 //   O^T += V^T P^T on the same MFMA (the k order is any order of the keys,
 //     taken as S^T left them), P split into f16 hi and lo in place; V goes
 //     to LDS transposed (dims x keys).
-// p = exp2((s - m) * scale * log2 e), the constant in two parts so that the
-// product is rounded once; m is the largest score seen to within 2^8 (the
+// p = exp2(s - m), the factor being in q's parts (to 2^-33: in the exponent it
+// would take a rounding); m is the largest score seen to within 2^8 (the
 // sums are rescaled only when a tile passes it by more: p <= 256), l the
 // sum, the output O / l. Only tiles past a wave's first query mask.
 // The low parts, of q and of P, add up in accumulators of their own: there
@@ -472,8 +471,8 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 // bits of 1500 queries over 2500 keys 4.1e-7 -> 3.1e-7, of 8 over 2400 2.45e-7 ->
 // 2.09e-7, the per-query kernel's 2.16e-7; 2% of the time).
 // What bounds it is issue: 80 MFMAs a tile and wave (16 cycles each) beside
-// about 270 VALU instructions, two waves per SIMD. 1500 queries over 2500
-// keys, 32 heads of 128: 151 us; with P through LDS, expf and a mask per score
+// about 250 VALU instructions, two waves per SIMD. 1500 queries over 2500
+// keys, 32 heads of 128: 149 us; with P through LDS, expf and a mask per score
 // (600 VALU instructions) it was 252.
 // Key chunks (ct > 0): a query block's tiles are split into chunks of ct
 // tiles, one workgroup each (blockIdx.z), so the long blocks at the end of
@@ -529,15 +528,6 @@ __device__ __forceinline__ float quarter_sum(float v) {
   return __builtin_bit_cast(float, (uint32_t)c[0]) + __builtin_bit_cast(float, (uint32_t)c[1]);
 }
 
-// exp2(d (c_hi + c_lo)) for a finite d, the product's rounding put back: the
-// factors of whole sums, where the rounding of an exponent of 10 alone would
-// be 5 units of the last place.
-__device__ __forceinline__ float exp2_scaled(float d, float c_hi, float c_lo) {
-  const float t = d * c_hi, e = __builtin_fmaf(d, c_lo, __builtin_fmaf(d, c_hi, -t));
-  const float r = __builtin_amdgcn_exp2f(t);
-  return __builtin_fmaf(r, 0.693147181f * e, r);
-}
-
 template <int G, int HD>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restrict__ q, const uint16_t *__restrict__ K,
                                                            const uint16_t *__restrict__ V, float *__restrict__ o,
@@ -587,13 +577,15 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   if (ch >= n_ch) return;  // (uniform: this block has fewer chunks)
   const uint32_t t_begin = ct ? ch * ct : 0, t_end = ct ? min(t_begin + ct, n_tiles) : n_tiles;
 
-  // This lane's Q operand row (16 wave + l16) as f16 hi + mid + lo, dims
-  // 32c + 8lq (each remainder is exact in f32), times the power of two that
-  // brings the row's largest value to [2^14, 2^15): values down to 2^-15 of
-  // it keep all 24 bits, smaller ones 2^-40 of it. The scores' factor takes
-  // the power back.
+  // This lane's Q operand row (16 wave + l16) times scale * log2 e = c_hi +
+  // c_lo (0.13 or 0.18) as f16 hi + mid + lo, dims 32c + 8lq (the product's
+  // rounding put back into the remainder). The row is first scaled by the
+  // power of two that brings its largest value to [2^17, 2^18), its largest
+  // part to 2^14 and more and below f16's 65504: values down to 2^-15 of it
+  // keep 24 bits, smaller ones 2^-40 of it. down takes the power back.
   v8h_t qhi[NC], qmid[NC], qlo[NC];
   const uint32_t row = 16 * wave + l16, qi = q0 + row / G, head = kvh * G + row % G;
+  float up, down;
   {
     const float *qr = q + ((size_t)min(qi, n_q - 1) * n_q_heads + head) * HD + 8 * lq;
     v4f_u xv[2 * NC];
@@ -607,17 +599,18 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     for (int i = 0; i < 2 * NC; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) qm = fmaxf(qm, fabsf(xv[i][e]));
-    const int sh = min(141 - (int)(__builtin_bit_cast(uint32_t, quarter_max(qm)) >> 23), 96);
-    const float up = __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23), down = __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
-    c_hi *= down;
-    c_lo *= down;
+    const int sh = min(144 - (int)(__builtin_bit_cast(uint32_t, quarter_max(qm)) >> 23), 96);
+    up = __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23);
+    down = __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
 #pragma unroll
     for (int c = 0; c < NC; c++) {
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         const float x = xv[2 * c + (e >> 2)][e & 3] * up;
-        const _Float16 hi = (_Float16)x;
-        const float r1 = x - (float)hi;
+        float y = x * c_hi;
+        asm("" : "+v"(y));  // (one value for hi and the remainder: no fused forms of it)
+        const _Float16 hi = (_Float16)y;
+        const float r1 = y - (float)hi + fmaf(x, c_lo, fmaf(x, c_hi, -y));
         const _Float16 mid = (_Float16)r1;
         qhi[c][e] = hi;
         qmid[c][e] = mid;
@@ -627,7 +620,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
   }
   // The last key this lane's query sees, and the wave's first query.
   const uint32_t vis = prefix + qi, vis0 = prefix + q0 + 16 * wave / G;
-  const float slack = 8.0f / c_hi;  // in scores: a factor 2^8 of p
+  const float slack = 8.0f * up;    // a factor 2^8 of p
   float m = -INFINITY, l = 0.f;     // l: this lane's keys only
   v4f_t O[ND], Ol[ND];               // Ol: of the probabilities' low parts
 #pragma unroll
@@ -676,9 +669,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
 #pragma unroll
       for (int kb = 0; kb < 4; kb++) S[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kb], qhi[c], S[kb], 0, 0, 0);
     }
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++) S[kb] += Sl[kb];
-    // ---- online softmax: S[kb][r] is key 64 t + 16 kb + 4 lq + r ----
+    // ---- online softmax: S[kb][r] (+ Sl, 2^-11 of it: not in the
+    // maximum, which is only a reference point) is key 64 t + 16 kb + 4 lq + r ----
     if (64 * t + 63 > vis0) {  // (uniform) a key some query of the wave does not see
       const uint32_t k0 = 64 * t + 4 * lq;
 #pragma unroll
@@ -693,21 +685,21 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
     mx = quarter_max(mx);
     if (__any(mx > m + slack)) {  // (also the first visible tile, m = -inf)
       const float mn = fmaxf(m, mx);
-      const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : exp2_scaled(m - mn, c_hi, c_lo);
+      const float al = mn == m ? 1.f : m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * down);
       l *= al;
 #pragma unroll
       for (int n = 0; n < ND; n++) O[n] *= al, Ol[n] *= al;
       m = mn;
     }
-    const float mr = m == -INFINITY ? 0.f : m;  // a later chunk's query may see no key yet
+    const float md = m == -INFINITY ? 0.f : m * down;  // a later chunk's query may see no key yet
     v8h_t Ph[2], Pl[2];
     float ps[4] = {};  // (summed apart: l takes one rounding a tile at its own size)
 #pragma unroll
     for (int kb = 0; kb < 4; kb++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const float d = S[kb][r] - mr;
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(d, c_hi, d * c_lo));  // 0 for masked keys
+        // (0 for masked keys)
+        const float pv = __builtin_amdgcn_exp2f(fmaf(Sl[kb][r], down, fmaf(S[kb][r], down, -md)));
         ps[r] += pv;
         const _Float16 hi = (_Float16)pv;
         Ph[kb >> 1][4 * (kb & 1) + r] = hi;
@@ -786,8 +778,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const float *__restri
           continue;
         }
         const float mn = fmaxf(M, mc[i]);  // finite: chunk 0's M is
-        const float a = exp2_scaled(M - mn, c_hi, c_lo);
-        const float b = mc[i] == -INFINITY ? 0.f : exp2_scaled(mc[i] - mn, c_hi, c_lo);
+        const float a = __builtin_amdgcn_exp2f((M - mn) * down);
+        const float b = mc[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mc[i] - mn) * down);
         L = L * a + lc[i] * b;
 #pragma unroll
         for (int n = 0; n < ND; n++) OA[n] = OA[n] * a + Oc[i][n] * b;
@@ -1576,10 +1568,9 @@ PromptPlan prompt_plan(const mdma_ctx *ctx, uint64_t n_q, uint64_t kv_len, uint6
 void launch_prompt(mdma_ctx *ctx, const PromptPlan &p, const float *q, const uint16_t *k, const uint16_t *v, float *o,
                    uint64_t n_q, uint64_t kv_len, uint64_t hd, uint64_t n_q_heads, uint64_t n_kv_heads, float *part,
                    uint32_t *cnt) {
-  // scale * log2 e in two floats, both positive (a masked score's -inf
-  // times each of them is then -inf).
+  // scale * log2 e in two floats.
   const double c = 1.4426950408889634 / std::sqrt((double)hd);
-  const float c_hi = std::nextafter((float)c, 0.f), c_lo = (float)(c - (double)c_hi);
+  const float c_hi = (float)c, c_lo = (float)(c - (double)c_hi);
   const uint64_t GP = n_q_heads / n_kv_heads, KO = n_q_heads * hd;
   // Asked for (a16_want_y == o): also the output projection's f16-path
   // input, into the caller's buffer.
