@@ -166,11 +166,13 @@ int mdma_gfx950_set_norm_fusion(mdma_ctx *ctx, int on);
 typedef enum { MDMA_PREFILL_AUTO = 0, MDMA_PREFILL_I8 = 1 } mdma_prefill_kernel;
 int mdma_gfx950_set_prefill_kernel(mdma_ctx *ctx, int kind);
 /* Extra: the int8 mode's batched decode GEMV kernel (calls of 3 tokens or
- * more on prepared-layout weights that the prefill GEMM does not take (3 to
- * 63 tokens), up to 16 tokens per launch). AUTO (default) streams each block of
- * the weight tile, activations and scales through a per-wave LDS ring by
- * DMA; STAGED loads them into registers and stages the weights in LDS (for
- * A/B measurement and the equality test: both give the same bits). */
+ * more on prepared-layout weights that the prefill GEMM does not take: 3 to
+ * 63 tokens). AUTO (default) takes 17 tokens and more in one launch where there
+ * is device space for its partial sums, and otherwise up to 16 per launch,
+ * streaming each block of the weight tile, activations and scales through a
+ * per-wave LDS ring by DMA; STAGED, up to 16 per launch, loads them into
+ * registers and stages the weights in LDS (for A/B measurement and the
+ * equality test: both give the same bits). */
 typedef enum { MDMA_BATCH_AUTO = 0, MDMA_BATCH_STAGED = 1 } mdma_batch_kernel;
 int mdma_gfx950_set_batch_kernel(mdma_ctx *ctx, int kind);
 /* Extra (no counterpart in the reference): with on != 0, the AUTO batch
@@ -324,7 +326,11 @@ int mdma_gfx950_qmatmul_i8_noalloc(mdma_ctx *ctx, const mdma_qweight *w, const m
  * replaced any buffer of its own since the capture (scratch growth, the
  * repack of a weight from the trait-shaped upload_weight); reserve_scratch
  * before capturing and capture again after. Buffers the caller frees must
- * outlive the graphs that use them. */
+ * outlive the graphs that use them. The space in which several-token launches
+ * leave partial sums is never in a graph: a captured launch splits its work
+ * only where the reserved scratch holds them (f32 mode, 9 tokens and more: up to
+ * 34 MB; int8 mode, 17 to 63: 4 KB per 16 tokens, 64 rows
+ * and eighth of the columns), and otherwise takes 8 or 16 tokens at a time. */
 typedef struct mdma_graph mdma_graph;
 int mdma_gfx950_graph_begin(mdma_ctx *ctx);
 int mdma_gfx950_graph_end(mdma_ctx *ctx, mdma_graph **out);

@@ -278,8 +278,9 @@ class Gfx950Backend:
         _check(lib().mdma_gfx950_set_prefill_kernel(self.ctx, int(kind)))
 
     def set_batch_kernel(self, kind: int):
-        """BATCH_AUTO: batched int8 GEMVs (3 to 63 tokens) stream through the
-        DMA ring kernel; BATCH_STAGED: the register-staged kernel (same bits)."""
+        """BATCH_AUTO: batched int8 GEMVs (3 to 63 tokens) in one launch from 17
+        tokens, through the DMA ring kernel below; BATCH_STAGED: the
+        register-staged kernel, 16 tokens a launch (same bits)."""
         _check(lib().mdma_gfx950_set_batch_kernel(self.ctx, int(kind)))
 
     def set_batch_layout(self, on: bool):
