@@ -1767,11 +1767,14 @@ bool launch_gemv_wide(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, bool gated
   const uint64_t pb = nt <= cus && std::min<uint64_t>(tiles * ws.nch, 2 * cus) > nt
                           ? tiles * ws.nch * ((T + 15) / 16) * 4 * 256 * 4 : 0;
   const uint64_t sb = q8_fits(ctx, x, T, n_in) ? 0 : (q8_slot_bytes(T * n_in) + 255) / 256 * 256;
-  char *sp = pb + sb ? static_cast<char *>(split_parts(ctx, sb + pb)) : nullptr;
-  if (pb + sb && !sp) return false;
   int8_t *qx;
   float *dx;
   int32_t *s16;
+  // The activation buffer's first megabyte before the space: on a full budget
+  // its growth takes the space back.
+  if (!sb) q8_slots(ctx, T, n_in, &qx, &dx, &s16);
+  char *sp = pb + sb ? static_cast<char *>(split_parts(ctx, sb + pb)) : nullptr;
+  if (pb + sb && !sp) return false;
   if (sb) {
     q8_slots_at(sp, T * n_in, &qx, &dx, &s16);
     launch_quantize_act(ctx, x, T * n_in, 256, qx, dx, s16);

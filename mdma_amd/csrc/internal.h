@@ -400,12 +400,13 @@ void launch_gemm_f16(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float
 constexpr uint64_t F64_MIN_TOKENS = 2;
 bool launch_gemm_f64(mdma_ctx *ctx, const GemvJob *jobs, int n_jobs, const float *x, uint64_t T,
                      float *glu_y = nullptr);
-// Device space for the partial sums of a launch that splits K (until the next
-// launch that asks): the context's scratch where it is large enough, else
-// space of its own, which a caller's allocation may take back; null where
-// that may not grow now (an allocation-free call, a full budget or device).
-// A captured launch gets the scratch or nothing: the growth of the scratch
-// ends a graph in any case (buf_epoch), giving the other space back must not.
+// Device space for the partial sums of a launch that splits K, until the next
+// launch that asks or the next growth of a context buffer (so it is asked for
+// last): the context's scratch where it is large enough, else space of its
+// own, which a caller's allocation may take back; null where that may not grow
+// now (an allocation-free call, a full budget or device). A captured launch
+// gets the scratch or nothing: the growth of the scratch ends a graph in any
+// case (buf_epoch), giving the other space back must not.
 void *split_parts(mdma_ctx *ctx, uint64_t bytes);
 void launch_quantize_act(mdma_ctx *ctx, const float *x, uint64_t n, uint64_t group, int8_t *q,
                          float *d, int32_t *sum16);

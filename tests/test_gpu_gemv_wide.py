@@ -150,3 +150,30 @@ def test_int8_buffer_is_not_grown_past_16_tokens():
         same(lambda: be.qmatmul(w, x, y))
     graph.close()
     be.close()
+
+
+@pytest.mark.parametrize("room", [100, 300])
+def test_int8_buffer_and_chunk_sums_on_a_budget(room):
+    # A first call with room for the int8 buffer's megabyte and little more: the
+    # chunk sums' 192 KB fit beside it or not, and neither takes the other's.
+    be = Gfx950Backend(0)
+    be.set_act_mode(bm.ACT_I8)
+    rows, k, T = 100, 2048, 40
+    raw = synth.weight(Q4K, rows, k, 1, True)
+    be.set_buffer_budget(device=64 << 20)
+    w = be.upload_weight(raw, Q4K, (rows, k))
+    x, y = be.f32_buf(synth.normal_f32(T * k, 2)), be.alloc(T * rows * 4)
+    used, limit = be.buffer_usage(bm.DOMAIN_DEVICE)
+    rest = be.alloc(limit - used - (1 << 20) - (room << 10))
+    got = []
+    for _ in range(3):
+        be.upload(y, 0, np.zeros(T * rows, np.float32))
+        be.qmatmul(w, x, y)
+        got.append(be.download_f32(y).view(np.uint32))
+    free = limit - be.buffer_usage(bm.DOMAIN_DEVICE)[0]
+    assert (free == room << 10) if room < 192 else (free < room << 10)
+    rest.close()
+    be.set_batch_kernel(bm.BATCH_STAGED)
+    be.qmatmul(w, x, y)
+    assert all(np.array_equal(g, be.download_f32(y).view(np.uint32)) for g in got)
+    be.close()
