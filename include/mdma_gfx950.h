@@ -357,7 +357,8 @@ int mdma_gfx950_set_replay_params(mdma_ctx *ctx, const mdma_buf *params, uint64_
 /* Extra (no counterpart in the reference; for benchmarks and profiling):
  * the next GEMV kernel this context launches on prepared weights is
  * dispatched with these hipEvent_t handles (either may be NULL), which its
- * dispatch packet timestamps at kernel start and end (hipExtLaunchKernel).
+ * dispatch packet timestamps at kernel start and end (hipExtLaunchKernel; where
+ * a launch splits its work, the end of the kernel that adds the parts).
  * Applies to one launch; not allowed during graph capture. */
 int mdma_gfx950_time_next_gemv(mdma_ctx *ctx, void *start_event, void *stop_event);
 

@@ -358,10 +358,12 @@ void launch(mdma_ctx *ctx, F64Args &a, uint32_t tiles, float *yg) {
     G = (tiles + n - 1) / n;
     a.per_q = n * a.nb, a.per_r = 0;
   }
-  gemm_f64_kernel<DT, TW, GLU><<<dim3(G), dim3(256), 0, ctx->stream>>>(a, yg);
+  const TimeEvents ev(ctx);
+  launch_timed(gemm_f64_kernel<DT, TW, GLU>, dim3(G), dim3(256), ctx->stream, ev.start, a.part ? nullptr : ev.stop, a,
+               yg);
   hip_check(hipGetLastError(), "gemm_f64 launch");
   if (a.part) {
-    gemm_f64_merge_kernel<TW, GLU><<<dim3(tiles), dim3(256), 0, ctx->stream>>>(a, G, yg);
+    launch_timed(gemm_f64_merge_kernel<TW, GLU>, dim3(tiles), dim3(256), ctx->stream, nullptr, ev.stop, a, G, yg);
     hip_check(hipGetLastError(), "gemm_f64 merge launch");
   }
 }
@@ -508,7 +510,8 @@ __global__ __launch_bounds__(64 * NW, f64_waves(TT) / 4) void gemv_f64_kernel(F6
 template <int DT, int TT, bool GLU, int NW>
 void launch_small(mdma_ctx *ctx, F64Args &a, float *yg) {
   const uint32_t G = std::min(a.units, (uint32_t)ctx->cu_count * f64_waves(TT) / NW);
-  gemv_f64_kernel<DT, TT, GLU, NW><<<dim3(G), dim3(64 * NW), 0, ctx->stream>>>(a, yg);
+  const TimeEvents ev(ctx);
+  launch_timed(gemv_f64_kernel<DT, TT, GLU, NW>, dim3(G), dim3(64 * NW), ctx->stream, ev.start, ev.stop, a, yg);
   hip_check(hipGetLastError(), "gemv_f64 launch");
 }
 template <int DT, bool GLU>

@@ -1682,13 +1682,15 @@ void wide_launch(mdma_ctx *ctx, WideSet &ws, uint32_t tiles, const int8_t *qx, c
   ws.items = tiles * ws.nch;
   ws.per_q = ws.nch, ws.per_r = 0;
   if (ws.part) G = std::min(ws.items, 2 * (uint32_t)ctx->cu_count), ws.per_q = ws.items / G, ws.per_r = ws.items % G;
+  const TimeEvents ev(ctx);
+  const hipEvent_t stop = G > tiles ? nullptr : ev.stop;
   if (ws.s.j[0].dots)
-    gemv_wide<W, NT, GLU, true><<<dim3(G), dim3(256), 0, ctx->stream>>>(ws, qx, dx);
+    launch_timed(gemv_wide<W, NT, GLU, true>, dim3(G), dim3(256), ctx->stream, ev.start, stop, ws, qx, dx);
   else
-    gemv_wide<W, NT, GLU, false><<<dim3(G), dim3(256), 0, ctx->stream>>>(ws, qx, dx);
+    launch_timed(gemv_wide<W, NT, GLU, false>, dim3(G), dim3(256), ctx->stream, ev.start, stop, ws, qx, dx);
   hip_check(hipGetLastError(), "gemv wide launch");
   if (G > tiles) {
-    gemv_wide_merge<NT, GLU><<<dim3(tiles, NT * 4), dim3(256), 0, ctx->stream>>>(ws);
+    launch_timed(gemv_wide_merge<NT, GLU>, dim3(tiles, NT * 4), dim3(256), ctx->stream, nullptr, ev.stop, ws);
     hip_check(hipGetLastError(), "gemv wide merge launch");
   }
 }

@@ -1,10 +1,27 @@
 // Device helpers shared by the gfx950 GEMV kernels: f16 conversion, 16-byte
 // streaming loads, DPP wave reductions and the Q4_K block pieces.
 #pragma once
+#include <hip/hip_ext.h>
 
 #include "internal.h"
 
 namespace mdma {
+
+// The events of mdma_gfx950_time_next_gemv, taken by the launch that they time.
+struct TimeEvents {
+  hipEvent_t start, stop;
+  explicit TimeEvents(mdma_ctx *ctx) : start(ctx->time_start), stop(ctx->time_stop) {
+    ctx->time_start = ctx->time_stop = nullptr;
+  }
+};
+// A launch whose dispatch timestamps the events given (either may be null).
+template <class... P, class... A>
+void launch_timed(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t stream, hipEvent_t start, hipEvent_t stop,
+                  A &&...args) {
+  if (start || stop) hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, start, stop, 0, args...);
+  else kernel<<<grid, block, 0, stream>>>(args...);
+}
+
 namespace {
 
 // Values made ready in SGPRs at this point (kernel arguments: their scalar

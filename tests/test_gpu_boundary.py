@@ -289,3 +289,59 @@ def test_graph_of_raw_weight_refuses_after_repack(backend):
     with pytest.raises(bm.Backend):
         graph.launch()
     graph.close()
+
+
+@pytest.mark.parametrize("mode,dtype,rows,k,T", [("f32", 12, 300, 1024, 1), ("f32", 12, 300, 1024, 4), ("f32", 14, 300, 1024, 20),
+                                                ("f32", 8, 40000, 288, 20), ("int8", 14, 300, 1024, 8), ("int8", 14, 300, 1024, 40),
+                                                ("int8", 12, 20000, 256, 40), ("int8", 8, 300, 1024, 100)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_time_next_gemv_times_the_next_call_and_no_other(mode, dtype, rows, k, T, gated):
+    # Every kernel over prepared rows, split and whole, takes the events: they
+    # are recorded when the call ends, and a later call leaves them alone.
+    import bench
+    from mdma_amd.backend import ACT_F32, ACT_I8, Gfx950Backend
+
+    be = Gfx950Backend(0)
+    be.set_act_mode({"f32": ACT_F32, "int8": ACT_I8}[mode])
+    w = be.upload_weight(synth.weight(dtype, rows, k, 1, True), dtype, (rows, k))
+    x, y, g, u = be.f32_buf(synth.normal_f32(T * k, 2)), *(be.alloc(T * rows * 4) for _ in range(3))
+
+    def call():
+        if gated:
+            be.ffn_gate_up(w, w, x, g, u, y)
+        else:
+            be.qmatmul(w, x, y)
+
+    ev = bench.HipEvents()
+    a, b = ev.event(), ev.event()
+    call()
+    be.join_execution()
+    be.time_next_gemv(a.value, b.value)
+    call()
+    be.join_execution()
+    ms = ev.elapsed_ms(a, b)  # (fails for events that were not recorded)
+    assert 0 < ms < 1000
+    call()
+    be.join_execution()
+    assert ev.elapsed_ms(a, b) == ms
+    be.close()
+    ev.destroy(a)
+    ev.destroy(b)
+
+
+@pytest.mark.parametrize("mode,T", [("f32", 3), ("f32", 20), ("int8", 20), ("cpu", 3)])
+def test_several_tokens_refuse_an_unaligned_x(mode, T):
+    # The kernels read x 16 bytes at a time, some by DMA: a view at another
+    # offset is refused.
+    from mdma_amd.backend import ACT_F32, ACT_F32_CPU, ACT_I8, Gfx950Backend, ShapeMismatch
+
+    be = Gfx950Backend(0)
+    be.set_act_mode({"f32": ACT_F32, "int8": ACT_I8, "cpu": ACT_F32_CPU}[mode])
+    rows, k = 64, 512
+    w = be.upload_weight(synth.weight(12, rows, k, 1, True), 12, (rows, k))
+    x, y = be.f32_buf(synth.normal_f32(T * k + 4, 2)), be.alloc(T * rows * 4)
+    for off in (4, 8, 12):
+        with pytest.raises(ShapeMismatch):
+            be.qmatmul(w, be.view(x, off, T * k * 4), y)
+    be.qmatmul(w, be.view(x, 16, T * k * 4), y)
+    be.close()
