@@ -449,8 +449,9 @@ __global__ __launch_bounds__(256) void attn_kernel(const float *__restrict__ q, 
 
 // Causal GQA attention for a prompt (one sequence, seq_stride 0: query i
 // sees keys [0, prefix + i]; ATT_PREFILL_MIN queries or more, or a few over a
-// long prefix) on the matrix cores, flash-attention style. A workgroup takes 64 rows, 64/G queries
-// times the G query heads of one KV head; wave w owns rows 16w..16w+15.
+// long prefix) on the matrix cores, flash-attention style. A workgroup takes
+// 64 rows, 64/G queries times the G query heads of one KV head; wave w owns
+// rows 16w..16w+15.
 // Per tile of 64 keys:
 //   S = Q K^T on v_mfma_f32_16x16x32_f16. The f16 keys are exact operands;
 //     q times scale * log2 e, its row scaled by a power of two, is split into
@@ -495,14 +496,14 @@ constexpr double ATT_MERGE_TILES = 0.25;
 // where the rows (queries times query heads) fill workgroups and their keys
 // add up to more than the launch's chain of tiles and merge. us, per query /
 // here, 128 dims; 32 heads, 8 KV: 48 queries over 3900 keys 98 / 27.5, 12 over
-// 1400 18.5 / 15.9, 8 over 3300 25.5 / 20.6; 20 heads, G = 1: 20 over 1700 27.4 /
-// 18.7; 8 heads, G = 8 and 1: 32 over 2100 22.6 / 17.9 and 23.6 / 17.5; 64
-// dims, G = 1: 16 heads, 20 over 2300 26 / 12. Below the line 32 heads, 16 KV:
-// 8 over 2048 17.1 / 17.7; 8 heads: 16 over 3900 18.0 / 20.7, 8 over 2048 10.0 / 16.1.
-// Under a capture or in a fixed scratch, where the key chunks are not made,
-// few queries stay with the per-query kernel: one workgroup a KV head would
-// walk all the tiles in turn.
-constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_FEW_ROWS = 160, ATT_FEW_WORK = 9 << 16;
+// 1400 18.5 / 15.9, 8 over 3300 25.5 / 20.6; 20 heads, G = 1: 13 over 2100 23.4 /
+// 19.3; 8 heads, G = 8 and 1: 32 over 2100 22.6 / 17.9 and 23.6 / 17.5; 64
+// dims, G = 1, 16 heads: 20 over 3300 33.1 / 13.7. On the line 32 heads, 8 and 16
+// KV: 8 over 2048 17.5 / 17.5 and 17.1 / 17.7; below it 8 heads: 16 over 3900 18.0 /
+// 20.7, 8 over 2048 10.0 / 16.1. Under a capture or in a fixed scratch, where the
+// key chunks are not made, few queries stay with the per-query kernel: one
+// workgroup a KV head would walk all the tiles in turn.
+constexpr uint64_t ATT_PREFILL_MIN = 64, ATT_PREFILL_FEW = 8, ATT_FEW_ROWS = 160, ATT_FEW_WORK = 1 << 19;
 
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
@@ -1664,7 +1665,7 @@ bool attn_impl(mdma_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t
     // (a capture of the same call finds them), and they grow no further: the
     // counters come from the partials' space if there are too few.
     if (prompt && n_q >= ATT_PREFILL_FEW && n_q * n_q_heads >= ATT_FEW_ROWS &&
-        n_q * n_q_heads * kv_len >= ATT_FEW_WORK && !ctx->capturing && !ctx->fixed_scratch) {
+        n_q * n_q_heads * kv_len > ATT_FEW_WORK && !ctx->capturing && !ctx->fixed_scratch) {
       const PromptPlan p = prompt_plan(ctx, n_q, kv_len, hd, n_kv_heads, GP);
       const uint64_t nc = n_kv_heads * p.nqb * CNT_STRIDE;
       const uint64_t cb = nc <= ctx->attn_cnt_cap ? 0 : (nc * 4 + 255) / 256 * 256;
